@@ -73,7 +73,7 @@ _ref = None
 def build(ref=True):
     """Compile the oracle (and the reference when its tree is present) with oracle/Makefile."""
     targets = ["oracle"]
-    if ref and REF_TREE.is_dir():
+    if ref and (REF_TREE / "src" / "sampler.cpp").is_file():  # an empty mount point is no tree
         targets.append("ref")
     subprocess.run(["make", "-s", "-C", str(HERE), f"-j{min(8, os.cpu_count() or 1)}"] + targets, check=True)
 

@@ -29,6 +29,8 @@ from pathlib import Path
 HERE = Path(__file__).resolve().parent
 ROOT = HERE.parents[1]
 REF = Path(os.environ.get("VSMP_REF_TREE", "/root/reference"))
+if not (REF / "CMakeLists.txt").is_file():  # an empty mount point counts as an absent tree
+    REF = REF / "absent"
 OUT = HERE / "_build"
 TARGETS = ["verbo", "verbo_shared", "verbo_cli", "verbo_tests"]
 
