@@ -767,3 +767,65 @@ def test_general_path_all_rows_marked(ctx):
     run.report()
     assert (run.info["flags"] & V.FLAG_SEQ_CUTS).all(), run.info["flags"]
     assert (run.info["keep"] == run.o_info["keep"]).all() and (run.ids == run.o_ids).all()
+
+
+@pytest.mark.parametrize("parts", [1, 3, 64])
+@pytest.mark.parametrize("Vv", [1030, 20003, 70001])
+def test_general_split_parts(monkeypatch, parts, Vv):
+    """General rows cut into parts (per-row parameters, so every plan in one batch): parts of several
+    register chunks, a last part of a few elements, empty parts, top-k lists of 257 to 1,024 elements
+    and beyond, a bucket of 4,000 to 5,000 equal values (whose count the raw sums cannot give), min-p
+    prefixes, draws without a cut, rows that are flat, cold, tied in steps, all -inf but one, and
+    the reference's draw stream advanced once per row."""
+    import torch
+
+    monkeypatch.setenv("VSMP_MODE", "split")
+    monkeypatch.setenv("VSMP_SPLIT_P", str(parts))
+    ctx = V.Context(0)
+    rng = np.random.default_rng(parts * 100003 + Vv)
+    kinds = ["normal", "flat", "steps", "equal", "cold", "neginf", "spiky"]
+    opts = [dict(top_p=0.95), dict(top_p=1.0), dict(top_p=0.9, min_p=0.02), dict(top_p=1.0, min_p=1e-4), dict(top_k=257, top_p=0.9),
+            dict(top_k=1000, min_p=0.01), dict(top_k=1024, top_p=0.5), dict(top_k=Vv - 1, top_p=0.8), dict(top_p=0.01)]
+    B = len(kinds) * len(opts)
+    lg = rng.normal(0, 1.0, (B, Vv)).astype(np.float32)
+    p = np.zeros(B, V.SAMPLING_DTYPE)
+    p["temp"] = rng.choice([0.4, 1.0, 1.3], B)
+    p["repeat"] = rng.choice([1.0, 1.3, 0.8], B)
+    p["seed"] = rng.integers(1, 1 << 62, B)
+    for r in range(B):
+        for f, v in opts[r // len(kinds)].items():
+            p[r][f] = v
+        kind = kinds[r % len(kinds)]
+        if kind == "flat":
+            lg[r] = 1.5
+        elif kind == "steps":
+            lg[r] = np.round(lg[r] * 16) / 16
+        elif kind == "equal":
+            n = min(Vv - 5, int(rng.integers(4000, 5000)))
+            lg[r, rng.permutation(Vv)[:n]] = 0.25
+        elif kind == "cold":
+            p[r]["temp"] = 0.01
+        elif kind == "neginf":
+            lg[r] = -np.inf
+            lg[r, rng.integers(0, Vv)] = 2.0
+        elif kind == "spiky":
+            lg[r, rng.integers(0, Vv, 12)] += 7.0
+    hists = [rng.integers(-2, Vv + 2, int(rng.integers(0, 400))) for _ in range(B)]
+    h, off = csr(hists)
+    log("general split parts", parts, Vv, B)
+    run = Run(ctx, lg, p, h, off)
+    assert (run.info["path"] == V.PATH_GENERAL).sum() >= B // 2
+    assert run.report()[1] == 0
+    # the draw stream: three calls without diagnostics advance it once each, as one workgroup per row does
+    states, ids = [], []
+    for mode in ("split", "rows"):
+        c = ctx if mode == "split" else mode_ctx("rows")
+        st = torch.arange(7, 7 + 2 * B, dtype=torch.int64, device="cuda")
+        pr = V.to_device_params(p)
+        x = torch.zeros(B, (Vv + 3) // 4 * 4, device="cuda")
+        x[:, :Vv] = torch.from_numpy(lg).cuda()
+        dh, do = torch.from_numpy(h).cuda(), torch.from_numpy(off).cuda()
+        out = [c.pick_batch(x[:, :Vv], pr, dh, do, V.U_XORSHIFT, rng_state=st).cpu() for _ in range(3)]
+        states.append(st.cpu())
+        ids.append(torch.stack(out))
+    assert torch.equal(states[0], states[1]) and torch.equal(ids[0], ids[1])

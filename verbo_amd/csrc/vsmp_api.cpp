@@ -7,6 +7,7 @@
 #include <algorithm>
 #include <chrono>
 #include <climits>
+#include <cmath>
 #include <cstdint>
 #include <cstdlib>
 #include <cstring>
@@ -122,6 +123,9 @@ struct vsmp_ctx {
   size_t n_tick = 0;
   unsigned int* g_npen = nullptr;
   size_t n_gnpen = 0;
+  // split general rows: one allocation (split_scratch); every call fills what it reads
+  unsigned char* p_scr = nullptr;
+  size_t n_pscr = 0;
   // LM-head path (vsmp_head_pick): probe logits, row bounds and modes, candidate lists, and the
   // logits of rows that are written whole (general rows) when the caller keeps none
   float* h_probe = nullptr;
@@ -155,6 +159,13 @@ struct vsmp_ctx {
 namespace vsmp {
 namespace {
 
+// How a small batch's general rows are cut (general_parts).
+struct GenParts {
+  int P;         // 0: no split
+  size_t rows;   // what the scratch is sized for: the rows and parts of this batch or of any smaller one
+  size_t slots;  // at this vocabulary, so that a context warmed up at a batch can serve smaller ones
+};
+
 struct Plan {
   bool rows;   // row mode: one workgroup per row (k_rows), else slices (k_stage1 + k_finish)
   bool split;  // a small greedy or top-k batch: each row cut into P parts in one launch
@@ -164,6 +175,9 @@ struct Plan {
   bool any_general, any_smallk, any_finish;
   bool no_rows_kernel;  // row mode with every row general: k_general alone takes the batch
   bool side_general;    // row mode with per-row parameters: k_general next to k_rows, on a side stream
+  GenParts gen;         // row mode: parts per general row at this shape; its scratch is sized whatever
+                        // the parameters, as the exact redo's is
+  bool gen_split;       // ... taken by this call's general rows
 };
 
 // VSMP_MODE=rows|slices|split pins the decomposition (testing and tuning); default: split parts
@@ -212,6 +226,54 @@ int topk_parts(int B, int V, int cus, int k, bool forced, long long forced_p) {
   if (!forced && (B > 24 || P < 8)) return 0;
   if (static_cast<long long>(B) * P > INT32_MAX) return 0;
   return static_cast<int>(std::max<long long>(P, 1));
+}
+
+// Parts per general row of a small batch. 0: one workgroup per row. A part costs the histogram's
+// global atomics (up to 4,096 whatever its elements) and its own elements, so the best number falls as
+// the square root of the batch: measured (top-k off, top-p .95) 48, 24, 10, 8 and 6 parts at 1, 4, 16,
+// 32 and 64 rows of 151,936, 28, 16, 6 and 5 at 1, 4, 16 and 32 of 49,152, which sqrt(V / (64 B))
+// meets. Against one workgroup per row, whose time hardly grows with the batch: 151,936 logits 1 row
+// 30.2 against 69.4 us, 16 rows 42.6 / 74.1, 64 rows 66.3 / 79.8, 128 rows 89.4 / 83.0; 49,152 logits
+// 1 row 27.9 / 38.5, 32 rows 36.8 / 40.7, 64 rows 43.3 / 40.8. The line between lies near B = V / 1600;
+// the split is taken to V / 2000.
+GenParts general_parts(int B, int V, bool forced, long long forced_p) {
+  const long long V4 = (static_cast<long long>(V) + 3) / 4;
+  const long long most = static_cast<long long>(kGenPartChunk) * kGenPartChunks;
+  const long long pmin = (V4 + most - 1) / most;
+  const long long pmax = std::max(pmin, std::min<long long>(kGenMaxParts, V4 / 256));
+  if (pmin > kGenMaxParts || static_cast<long long>(B) * kGenMaxParts > INT32_MAX / kGenPartList) return {};
+  const long long want = forced_p > 0 ? forced_p : std::llround(std::sqrt(V / (64.0 * B)));
+  const long long P = std::min(std::max(want, pmin), pmax);
+  if (forced) return {static_cast<int>(P), static_cast<size_t>(B), static_cast<size_t>(B * P)};
+  const long long rows = std::min<long long>(B, V / 2000);
+  if (rows < 1 || pmax < 2) return {};
+  const long long slots = std::max({rows * pmin, rows * P, static_cast<long long>(std::sqrt(rows * (V / 64.0)) + 0.5 * rows) + 1});
+  return {rows == B && P >= 2 ? static_cast<int>(P) : 0, static_cast<size_t>(rows), static_cast<size_t>(slots)};
+}
+
+// Where the split general rows' scratch lies in its allocation, 16-byte aligned.
+struct SplitScratch {
+  size_t list, hfix, max, mass, cnt, min, bits, tick, bytes;
+};
+SplitScratch split_scratch(const GenParts& gp, int words) {
+  const size_t rows = gp.rows, slots = gp.slots;
+  SplitScratch s{};
+  size_t at = 0;
+  auto take = [&at](size_t bytes) {
+    const size_t o = at;
+    at += (bytes + 15) & ~size_t{15};
+    return o;
+  };
+  s.list = take(slots * kGenPartList * sizeof(uint64_t));
+  s.hfix = take(rows * kGenBuckets * sizeof(uint64_t));
+  s.max = take(slots * sizeof(uint64_t));
+  s.mass = take(slots * 2 * sizeof(double));
+  s.cnt = take(slots * kGenPartCnt * sizeof(int));
+  s.min = take(slots * sizeof(unsigned));
+  s.bits = take(rows * static_cast<size_t>(words) * sizeof(unsigned));
+  s.tick = take(rows * sizeof(unsigned));
+  s.bytes = at;
+  return s;
 }
 
 // Slice shape: enough workgroups to fill the chip (>= 2048), slices of 256*EPT elements, and no
@@ -263,6 +325,12 @@ Plan plan(const vsmp_ctx* ctx, int B, int V, const vsmp_params* hostp) {
     // leaves those rows alone), on a stream forked from the caller's: the few long general rows
     // then overlap the row kernel instead of following it.
     pl.side_general = !hostp;
+    // k <= kGenCap or top-k off: k_general's split takes the row (with per-row parameters it leaves
+    // other rows to one of their workgroups)
+    if (pl.any_general && fm != 1) {
+      pl.gen = general_parts(B, V, fm == 2, ctx->split_p);
+      pl.gen_split = pl.gen.P > 0 && (!hostp || hostp->top_k <= kGenCap || hostp->top_k >= V);
+    }
     pl.any_smallk = false;
     pl.any_finish = false;
     return pl;
@@ -375,10 +443,10 @@ int launch_batch(vsmp_ctx* ctx, const float* logits, int B, int V, long long ld,
   const size_t slots = static_cast<size_t>(B) * static_cast<size_t>(pl.S);
   if (slots > static_cast<size_t>(INT32_MAX) / kKmax) return set_error("vsmp: batch too large");
   const int words = a.words;
-  if (!grow(ctx->s_cnt, ctx->n_cnt, slots, false, "scratch", st) ||
-      !grow(ctx->s_npen, ctx->n_npen, slots, false, "scratch", st) ||
-      !grow(ctx->s_max, ctx->n_max, slots, false, "scratch", st) ||
-      !grow(ctx->s_min, ctx->n_min, slots, false, "scratch", st))
+  if (!pl.rows && (!grow(ctx->s_cnt, ctx->n_cnt, slots, false, "scratch", st) ||  // row mode uses none of these
+                   !grow(ctx->s_npen, ctx->n_npen, slots, false, "scratch", st) ||
+                   !grow(ctx->s_max, ctx->n_max, slots, false, "scratch", st) ||
+                   !grow(ctx->s_min, ctx->n_min, slots, false, "scratch", st)))
     return -1;
   if (pl.any_smallk && !grow(ctx->s_cand, ctx->n_cand, slots * kKmax, false, "scratch", st)) return -1;
   // General rows marked near a top-p tie are redone exactly (rows up to kExactMaxVocab). The scratch
@@ -393,6 +461,11 @@ int launch_batch(vsmp_ctx* ctx, const float* logits, int B, int V, long long ld,
     return -1;
   if (pl.any_general && !pl.rows && !grow(ctx->s_bits, ctx->n_bits, static_cast<size_t>(B) * words, false, "scratch", st))
     return -1;
+  SplitScratch ss{};
+  if (pl.gen.rows > 0) {
+    ss = split_scratch(pl.gen, words);
+    if (!grow(ctx->p_scr, ctx->n_pscr, ss.bytes, false, "scratch", st)) return -1;
+  }
   if (a.pen_bits) {  // diagnostics: the kernels store or OR each row's penalised ids into zeroed bitmaps
     launch_zero_u32(a.pen_bits, static_cast<long long>(B) * words, st);
     if (!hip_ok(hipGetLastError(), "zero-fill launch")) return -1;
@@ -407,6 +480,17 @@ int launch_batch(vsmp_ctx* ctx, const float* logits, int B, int V, long long ld,
   a.s_max = ctx->s_max;
   a.s_min = ctx->s_min;
   a.s_bits = ctx->s_bits;
+  if (pl.gen_split) {
+    a.P = pl.gen.P;
+    a.p_list = reinterpret_cast<unsigned long long*>(ctx->p_scr + ss.list);
+    a.p_hfix = reinterpret_cast<unsigned long long*>(ctx->p_scr + ss.hfix);
+    a.s_max = reinterpret_cast<unsigned long long*>(ctx->p_scr + ss.max);
+    a.p_mass = reinterpret_cast<double*>(ctx->p_scr + ss.mass);
+    a.p_cnt = reinterpret_cast<int*>(ctx->p_scr + ss.cnt);
+    a.s_min = reinterpret_cast<unsigned*>(ctx->p_scr + ss.min);
+    a.s_bits = reinterpret_cast<unsigned*>(ctx->p_scr + ss.bits);
+    a.g_tick = reinterpret_cast<unsigned*>(ctx->p_scr + ss.tick);
+  }
   a.gen_fused = pl.rows ? 1 : 0;
   a.x_flag = exact ? ctx->x_flag : nullptr;
   a.x_u = ctx->x_u;
@@ -430,7 +514,10 @@ int launch_batch(vsmp_ctx* ctx, const float* logits, int B, int V, long long ld,
     if (!hip_ok(hipEventRecord(ctx->fork_ev, st), "hipEventRecord") ||
         !hip_ok(hipStreamWaitEvent(ctx->side, ctx->fork_ev, 0), "hipStreamWaitEvent"))
       return -1;
-    launch_general(a, ctx->cus, ctx->side);
+    if (pl.gen_split)
+      launch_general_split(a, ctx->side);
+    else
+      launch_general(a, ctx->cus, ctx->side);
     bool ok = hip_ok(hipGetLastError(), "general-path launch");
     if (ok && exact) {
       launch_general_exact(a, exact_slots(a.x_n, B), ctx->side);
@@ -459,7 +546,10 @@ int launch_batch(vsmp_ctx* ctx, const float* logits, int B, int V, long long ld,
     if (!hip_ok(hipGetLastError(), "finish launch")) return -1;
   }
   if (pl.any_general) {
-    launch_general(a, ctx->cus, st);
+    if (pl.gen_split)
+      launch_general_split(a, st);
+    else
+      launch_general(a, ctx->cus, st);
     if (!hip_ok(hipGetLastError(), "general-path launch")) return -1;
     if (exact) {
       launch_general_exact(a, exact_slots(a.x_n, B), st);
@@ -766,7 +856,7 @@ void vsmp_ctx_free(vsmp_ctx* c) {
   (void)hipDeviceSynchronize();
   void* bufs[] = {c->x_flag, c->x_u,    c->x_buf,    c->s_cand, c->s_cnt,   c->s_npen,   c->s_max,
                   c->s_min,  c->s_bits, c->g_slot,   c->g_tick, c->g_npen,  c->h_probe,  c->h_full,
-                  c->h_tk,   c->h_rmode, c->h_rcand, c->h_rcnt};
+                  c->h_tk,   c->h_rmode, c->h_rcand, c->h_rcnt, c->p_scr};
   for (void* p : bufs)
     if (p) (void)hipFree(p);
   for (unsigned char* h : c->hs_host)

@@ -17,6 +17,12 @@ constexpr int kMaxMergeSlices = 64;  // slices a small-k row may be cut into
 constexpr int kGenThreads = 1024;  // threads per general-path workgroup (one row each)
 constexpr int kGenBuckets = 4096;  // level-0 mass buckets of the general path
 constexpr int kGenCap = 1024;      // elements the general path sorts in LDS at once (power of two)
+constexpr int kGenPartList = 2048; // entries a part of a split general row may hand over
+constexpr int kGenMaxParts = 64;   // parts a general row may be cut into (one lane each reads their results)
+constexpr int kGenPartChunk = 4096;  // 16-byte groups of a part held in registers at once
+constexpr int kGenPartChunks = 4;    // chunks per part at most
+constexpr int kGenPartCnt = 8;       // counts per part: min-p prefix, its listed elements, overflow bucket,
+constexpr int kGenPartListA = 4;     // and from here the select's lists A and B
 constexpr int kMaxVocab = 1 << 20;  // larger rows are rejected: every accepted row can be redone exactly
 constexpr int kRowMaxVocab = 1 << 19;                    // row mode keeps the row's bitmap in LDS
 constexpr size_t kRowMaxDynLds = (kRowMaxVocab / 32) * 4;
@@ -74,6 +80,12 @@ struct KArgs {
   unsigned long long* g_slot;
   unsigned int* g_tick;
   unsigned int* g_npen;
+  // split general rows: P parts per row, the tickets above, per row the level-0 histogram's raw sums,
+  // per part its min-p prefix's mass and its overflow bucket's, kGenPartCnt counts and a list
+  unsigned long long* p_hfix;  // [B][kGenBuckets]
+  double* p_mass;              // [B*P][2]
+  int* p_cnt;                  // [B*P][kGenPartCnt]
+  unsigned long long* p_list;  // [B*P][kGenPartList]
 };
 
 constexpr int kSplitMaxPartGroups = 4096;  // 16-byte groups one split part loads (all in flight)
@@ -83,6 +95,8 @@ void launch_finish(const KArgs& a, hipStream_t st);
 void launch_rows(const KArgs& a, hipStream_t st);
 // cus: the device's CUs (0: unknown), which sets the workgroup size for large general batches.
 void launch_general(const KArgs& a, int cus, hipStream_t st);
+// General rows cut into a.P parts each: k_gen_max, k_gen_hist and k_general<512, true>.
+void launch_general_split(const KArgs& a, hipStream_t st);
 void launch_general_exact(const KArgs& a, int slots, hipStream_t st);
 void launch_numer_probe(const float* d, double* y, long long n, float temp, float qs, bool fixed_point, hipStream_t st);
 // Workgroups (and scratch slots of 2 * x_n entries) of k_general_exact for a batch of B rows: one

@@ -25,6 +25,8 @@
 //            the numerators (fixed-point sums per bucket), then count and mass selects over the
 //            row, with histograms in LDS. In row mode it takes the row's maximum pass and penalty
 //            bitmap itself.
+//  k_gen_max, k_gen_hist, k_general<512, true>  the same for a batch of few general rows: each row cut
+//            into parts over several CUs, one launch per pass.
 //  k_general_exact  after k_general: the rows it marked (a top-p cut at rounding distance of
 //            top_p) redone in the reference's order and sequential sums.
 //  k_read_probe  a plain streaming read, for the attainable-bandwidth measurement.
@@ -1442,6 +1444,25 @@ __device__ __forceinline__ int q_of_d(const GenCtx& g, float d) {
 }
 __device__ __forceinline__ int q_of(const GenCtx& g, float v) { return q_of_d(g, v - g.mx); }
 
+// The row's maximum, temperature and bucket scale, from its largest composite and smallest key.
+// capped: the buckets stop short of the row minimum (the overflow bucket may hold most of the row).
+__device__ __forceinline__ void gen_scale(GenCtx& g, float temp, uint64_t mxc, uint32_t mnk, bool& capped) {
+  g.mx = comp_val(mxc);
+  g.temp = temp;
+  g.inv_temp = 1.0 / static_cast<double>(temp);
+  float range = g.mx - key_val(mnk);
+  const float cap = 64.0f * temp;
+  capped = !(range <= cap);
+  if (capped) range = cap;
+  g.qs = range > 0.0f ? static_cast<float>(kGenBuckets) / range : 0.0f;
+}
+// A floor under d = v - mx (the float the numerators take) for every element whose numerator can
+// reach the min-p threshold thr, d / temp >= log(thr) (exp within 1e-15): the exact numerator is
+// taken only above it.
+__device__ __forceinline__ float minp_floor(float temp, double thr) {
+  return static_cast<float>(static_cast<double>(temp) * log(thr) * 1.001) - 1e-3f;
+}
+
 // The main pass's numerator exp(double(d) / temp) by a table over bucket pairs: buckets 2j and
 // 2j + 1 share the point c_j = -(2j + 1) w, w = 1 / (qs temp) (one bucket's width in exponent
 // units; the buckets reach at most 64 temp below the maximum, so w <= 1/64), etab[j] = exp(c_j).
@@ -1747,19 +1768,361 @@ __device__ __forceinline__ Sel refine_select(const GenCtx& g, GenShared<NT>& sh,
   return scan_sorted<MASS>(g, sh, sh.list, sh.lpr, m, rank_above, above, target);
 }
 
-// NT threads per workgroup: 1024, or 512 (two workgroups per CU, each holding its row's passes
-// while the other's wait on memory) for batches with more general rows than CUs.
+// ---- split general rows: a small batch's general rows, each cut into parts over several CUs -------
+//
+// With fewer general rows than CUs, k_general's one workgroup per row leaves most of the chip idle
+// and its three passes follow one another on one CU. Here row r is cut into P parts (whole words of
+// the penalty bitmap), one 512-thread workgroup each, and each pass is a launch of its own over all
+// parts of all rows:
+//  k_gen_max   the part's penalty bitmap (kept in global memory for the next two), first maximum and
+//              minimum; part 0 takes the row's draw; the row's histogram is cleared;
+//  k_gen_hist  the main pass: the part's fixed-point mass histogram in LDS, its non-empty buckets added
+//              to the row's in global memory (integer sums: the same totals in any order), and the
+//              part's share of the min-p prefix;
+//  k_general<512, true>  every part takes the prefixes of the row's histogram and the same plan from
+//              them, lists its elements of the selected buckets, and the part that takes the row's last
+//              ticket merges the lists and ends the row as k_general does.
+// A launch's results reach the next one at the kernel boundary; within the last launch lists and
+// counts travel in device-scope stores that complete before the part's ticket (as in k_topk_split).
+// Nothing waits on another workgroup.
+//
+// The histogram holds one 64-bit word per bucket, the sum of the terms' raw bits (numer_fix): with
+// the words' atomics at about 10 ns per thousand over the chip, a count beside each would double what
+// bounds k_gen_hist. A bucket of n < 4,032 elements sums to n kFixRawE + f, f below 2^52 (each term
+// within e^(+-1/64) of 2^40), so the top 12 bits are n kFixRawE's, an odd multiple of n mod 4096, and
+// give n back (gen_raw_count). A larger bucket decodes to something else; a decoded count above
+// kRawCountMax is taken as 0, so a bucket that is not decoded exactly is decoded too low, and the
+// counts of a row add up to its elements only when all are exact. Otherwise (rows of very many
+// equal values) one workgroup takes the row by itself, counting as k_general does.
+constexpr int kGsNT = 512;
+constexpr int kGsU = 8;
+constexpr int kGsChunk = kGsNT * kGsU;  // 16-byte groups a part holds in registers at once
+static_assert(kGenPartChunk == kGsChunk, "the planner sizes parts by kGenPartChunk");
+constexpr uint32_t kRawCountMax = 4000;
+constexpr uint32_t kRawInv = 0x7A3;  // (kFixRawE >> 52) kRawInv = 1 mod 4096
+static_assert(((kFixRawE >> 52) * kRawInv) % 4096 == 1 && (kFixRawE << 12) == 0, "the raw bits' count");
+__device__ __forceinline__ uint32_t gen_raw_count(uint64_t raw) {
+  const uint32_t n = (static_cast<uint32_t>(raw >> 52) * kRawInv) & 4095u;
+  return n <= kRawCountMax ? n : 0u;
+}
+
+struct GenPart {
+  int row, part;
+  int g0, g1;  // its 16-byte groups
+  int lo, hi;  // its elements
+};
+__device__ __forceinline__ GenPart gen_part(const KArgs& a) {
+  GenPart t;
+  t.row = static_cast<int>(blockIdx.x) / a.P;
+  t.part = static_cast<int>(blockIdx.x) - t.row * a.P;
+  const int V4 = (a.V + 3) >> 2;
+  const int G = ((V4 + a.P - 1) / a.P + 7) & ~7;  // whole 32-bit words of the bitmap
+  t.g0 = min(V4, t.part * G);
+  t.g1 = min(V4, t.g0 + G);
+  t.lo = 4 * t.g0;
+  t.hi = min(a.V, 4 * t.g1);
+  return t;
+}
+// The 16-byte groups of the part's chunk that starts at group c0, all loads in flight at once (past
+// the part: its last group, or the row's).
+__device__ __forceinline__ void gen_part_load(const float* rp, int V, const GenPart& t, int c0, float4 (&v)[kGsU]) {
+  const float4* rp4 = reinterpret_cast<const float4*>(rp);
+  const int glast = (t.g1 > t.g0 ? t.g1 : (V + 3) >> 2) - 1;
+#pragma unroll
+  for (int u = 0; u < kGsU; ++u) v[u] = rp4[min(c0 + u * kGsNT + static_cast<int>(threadIdx.x), glast)];
+}
+// The penalty bits of the thread's groups of that chunk, four bits each. bits: the bitmap from the
+// row's start, in global memory, or (base > 0 possible) from group `base` on.
+__device__ __forceinline__ uint32_t gen_part_nibs(const uint32_t* bits, const GenPart& t, int c0, int base = 0) {
+  uint32_t w[kGsU], nibs = 0u;
+  const int glast = max(t.g1 - 1, t.g0);
+#pragma unroll
+  for (int u = 0; u < kGsU; ++u) w[u] = bits[(min(c0 + u * kGsNT + static_cast<int>(threadIdx.x), glast) - base) >> 3];
+#pragma unroll
+  for (int u = 0; u < kGsU; ++u) {
+    const int f = c0 + u * kGsNT + static_cast<int>(threadIdx.x);
+    nibs |= ((w[u] >> (4 * (f & 7))) & 0xFu) << (4 * u);
+  }
+  return nibs;
+}
+__device__ __forceinline__ void gen_part_penalise(const GenRow& R, uint32_t nib, float (&x)[4]) {
+  if (!R.pen || !nib) return;
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+    if (nib & (1u << c)) x[c] = penalise(x[c], R.rep);
+}
+// The row's maximum (first index) and minimum from its parts', by each wave.
+__device__ __forceinline__ void gen_part_range(const KArgs& a, int row, uint64_t& mxc, uint32_t& mnk) {
+  const int lane = threadIdx.x & 63;
+  uint64_t m = lane < a.P ? a.s_max[static_cast<size_t>(row) * a.P + lane] : 0ull;
+  uint32_t n = lane < a.P ? a.s_min[static_cast<size_t>(row) * a.P + lane] : 0xFFFFFFFFu;
+  for (int o = 32; o > 0; o >>= 1) {
+    m = max64(m, __shfl_xor(m, o));
+    n = min(n, static_cast<uint32_t>(__shfl_xor(static_cast<int>(n), o)));
+  }
+  mxc = sgpr_u64(m);
+  mnk = sgpr_u32(n);
+}
+// A row whose k-th element the split selects: top-k off, or a top-k whose elements fit one list.
+__device__ __forceinline__ bool gen_split_row(int k, int V) { return k == V || k <= kGenCap; }
+
+__global__ __launch_bounds__(kGsNT) void k_gen_max(KArgs a) {
+  __shared__ uint32_t bits[kGenPartChunks * kGsChunk / 8];
+  __shared__ uint64_t red[kGsNT / 64];
+  const GenPart t = gen_part(a);
+  const int tid = threadIdx.x, V = a.V, row = t.row;
+  const vsmp_params P = sgpr_params(row_params(a, row));
+  if (path_of(P, V, a.smallk_ok) != kPathGeneral) return;
+  int h0, h1;
+  row_hist(a, row, h0, h1);
+  GenRow R;
+  R.pen = (P.repeat != 1.0f) && (h1 - h0) > 0;
+  R.rep = P.repeat;
+  const int H = h1 - h0;
+  const int hfrom = h0 + ((P.repeat_last > 0 && H > P.repeat_last) ? H - P.repeat_last : 0);
+  constexpr int HQ = 4;  // history ids first: the vector memory counter retires in order
+  int hid[HQ];
+  if (R.pen) {
+#pragma unroll
+    for (int q = 0; q < HQ; ++q) hid[q] = a.hist[min(hfrom + q * kGsNT + tid, h1 - 1)];
+  }
+  float4 v[kGsU];
+  const float* rp = a.logits + static_cast<size_t>(row) * static_cast<size_t>(a.ld);
+  gen_part_load(rp, V, t, t.g0, v);
+  for (int b = t.part * kGenBuckets / a.P + tid; b < (t.part + 1) * kGenBuckets / a.P; b += kGsNT)
+    a.p_hfix[static_cast<size_t>(row) * kGenBuckets + b] = 0ull;
+  if (t.part == 0 && tid == 0) {
+    a.x_u[row] = draw_u(a, row, P);
+    a.g_tick[row] = 0u;
+  }
+  if (R.pen) {  // src/sampler.cpp:53-65
+    const int words = (t.hi - t.lo + 31) >> 5;
+    for (int i = tid; i < words; i += kGsNT) bits[i] = 0u;
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < HQ; ++q) {
+      const int id = hid[q];
+      if (hfrom + q * kGsNT + tid < h1 && id >= t.lo && id < t.hi)
+        atomicOr(&bits[(id - t.lo) >> 5], 1u << ((id - t.lo) & 31));
+    }
+    for (int i = hfrom + HQ * kGsNT + tid; i < h1; i += kGsNT) {
+      const int id = a.hist[i];
+      if (id >= t.lo && id < t.hi) atomicOr(&bits[(id - t.lo) >> 5], 1u << ((id - t.lo) & 31));
+    }
+    __syncthreads();
+    uint32_t* gb = a.s_bits + static_cast<size_t>(row) * a.words + (t.lo >> 5);
+    for (int i = tid; i < words; i += kGsNT) gb[i] = bits[i];
+    if (a.pen_bits) store_pen_words<kGsNT>(a, row, t.lo >> 5, bits, words);
+  }
+  // the first maximum (a thread's elements come in increasing order) and the minimum, by float
+  // comparison as in k_general: -0 with +0, NaN never chosen
+  float rmx = -INFINITY, rmn = INFINITY;
+  int first = t.lo;
+  for (int c0 = t.g0; c0 < t.g1; c0 += kGsChunk) {
+    if (c0 != t.g0) gen_part_load(rp, V, t, c0, v);
+    const uint32_t nibs = R.pen ? gen_part_nibs(bits, t, c0, t.g0) : 0u;
+#pragma unroll
+    for (int u = 0; u < kGsU; ++u) {
+      const int f = c0 + u * kGsNT + tid;
+      if (f >= t.g1) continue;
+      float x[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
+      gen_part_penalise(R, (nibs >> (4 * u)) & 0xFu, x);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        if (4 * f + c >= V) continue;
+        if (x[c] > rmx) {
+          rmx = x[c];
+          first = 4 * f + c;
+        }
+        rmn = fminf(rmn, x[c]);
+      }
+    }
+  }
+  const bool any = t.hi > t.lo;
+  const uint64_t mxc = block_max64<kGsNT>(any ? comp(ord_key(rmx), static_cast<uint32_t>(first)) : 0ull, red);
+  const uint64_t mnk = block_min64<kGsNT>(any ? ord_key(rmn) : 0xFFFFFFFFu, red);
+  if (tid == 0) {
+    const size_t slot = static_cast<size_t>(row) * a.P + t.part;
+    a.s_max[slot] = mxc;
+    a.s_min[slot] = static_cast<uint32_t>(mnk);
+  }
+}
+
+__global__ __launch_bounds__(kGsNT) void k_gen_hist(KArgs a) {
+  __shared__ unsigned long long fix0[kGenBuckets];
+  __shared__ uint64_t list[kGenCap];
+  __shared__ uint64_t red[kGsNT / 64];
+  __shared__ int nlist;
+  const GenPart t = gen_part(a);
+  const int tid = threadIdx.x, V = a.V, row = t.row;
+  const vsmp_params P = sgpr_params(row_params(a, row));
+  if (path_of(P, V, a.smallk_ok) != kPathGeneral || !gen_split_row(top_k_of(P, V), V)) return;
+  int h0, h1;
+  row_hist(a, row, h0, h1);
+  GenCtx g;
+  g.R.rp = a.logits + static_cast<size_t>(row) * static_cast<size_t>(a.ld);
+  g.R.pen = (P.repeat != 1.0f) && (h1 - h0) > 0;
+  g.R.rep = P.repeat;
+  const uint32_t* gbits = a.s_bits + static_cast<size_t>(row) * a.words;
+  float4 v[kGsU];
+  gen_part_load(g.R.rp, V, t, t.g0, v);
+  uint32_t nibs = g.R.pen && t.hi > t.lo ? gen_part_nibs(gbits, t, t.g0) : 0u;
+  uint64_t mxc;
+  uint32_t mnk;
+  gen_part_range(a, row, mxc, mnk);
+  for (int i = tid; i < kGenBuckets; i += kGsNT) fix0[i] = 0ull;
+  if (tid == 0) nlist = 0;
+  exp_tab_fill();
+  __syncthreads();
+  bool capped;
+  gen_scale(g, P.temp, mxc, mnk, capped);
+  // a flat row (k_general): nothing is added, so its counts do not add up and one workgroup takes it
+  if (comp_key(mxc) == mnk && isfinite(g.mx)) return;
+  const FixCoef fc = fix_coef(table_width(g.qs, P.temp), P.temp, g.inv_temp);
+  const bool minp = P.min_p > 0.0f;
+  const double thr = static_cast<double>(P.min_p);
+  const float dmin = minp ? minp_floor(P.temp, thr) : INFINITY;
+  const bool ovf_exact = capped && minp && thr < 1e-26;
+  uint32_t t_cntm = 0u, t_ocnt = 0u;
+  double t_totm = 0.0, t_omass = 0.0;
+  for (int c0 = t.g0; c0 < t.g1; c0 += kGsChunk) {
+    if (c0 != t.g0) {
+      gen_part_load(g.R.rp, V, t, c0, v);
+      nibs = g.R.pen ? gen_part_nibs(gbits, t, c0) : 0u;
+    }
+#pragma unroll
+    for (int u = 0; u < kGsU; ++u) {
+      const int f = c0 + u * kGsNT + tid;
+      if (f >= t.g1) continue;
+      float x[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
+      gen_part_penalise(g.R, (nibs >> (4 * u)) & 0xFu, x);
+      float d[4];
+      int q[4];
+      uint64_t m[4];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        d[c] = x[c] - g.mx;
+        q[c] = q_of_d(g, d[c]);
+        m[c] = numer_fix(fc, d[c], q[c]);
+      }
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        if (4 * f + c >= V) continue;
+        if (capped && q[c] == kGenBuckets - 1) {  // the overflow bucket, as in k_general
+          ++t_ocnt;
+          if (ovf_exact) {
+            const double p = numer_g(g, x[c]);
+            t_omass += p;
+            if (p >= thr) {
+              ++t_cntm;
+              t_totm += p;
+            }
+          }
+          continue;
+        }
+        atomicAdd(&fix0[q[c]], static_cast<unsigned long long>(m[c]));
+        if (d[c] >= dmin) {
+          const double p = numer_g(g, x[c]);
+          if (p >= thr) {
+            ++t_cntm;
+            t_totm += p;
+            const int pos = atomicAdd(&nlist, 1);
+            if (pos < kGenCap) list[pos] = comp(ord_key(x[c]), static_cast<uint32_t>(4 * f + c));
+          }
+        }
+      }
+    }
+  }
+  __syncthreads();
+  // the row's histogram: each part starts on buckets of its own, so that the parts do not meet
+  unsigned long long* hf = a.p_hfix + static_cast<size_t>(row) * kGenBuckets;
+  const int b0 = (t.part * (kGenBuckets / a.P)) & ~63;
+#pragma unroll
+  for (int i = 0; i < kGenBuckets / kGsNT; ++i) {
+    const int b = (b0 + i * kGsNT + tid) & (kGenBuckets - 1);
+    const unsigned long long f = fix0[b];
+    if (f) __hip_atomic_fetch_add(&hf[b], f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  if (!minp && !capped) return;
+  const size_t slot = static_cast<size_t>(row) * a.P + t.part;
+  const int nl = nlist;
+  for (int i = tid; i < min(nl, kGenCap); i += kGsNT) a.p_list[slot * kGenPartList + i] = list[i];
+  const uint32_t cm = block_sum_u32<kGsNT>(t_cntm, reinterpret_cast<uint32_t*>(red));
+  const uint32_t oc = block_sum_u32<kGsNT>(t_ocnt, reinterpret_cast<uint32_t*>(red));
+  const double tm = block_sum_f64<kGsNT>(t_totm, reinterpret_cast<double*>(red));
+  const double om = block_sum_f64<kGsNT>(t_omass, reinterpret_cast<double*>(red));
+  if (tid == 0) {
+    int* pc = a.p_cnt + kGenPartCnt * slot;
+    pc[0] = static_cast<int>(cm);
+    pc[1] = nl;
+    pc[2] = static_cast<int>(oc);
+    a.p_mass[2 * slot] = tm;
+    a.p_mass[2 * slot + 1] = om;
+  }
+}
+
+// Entry i of the parts' lists of a row laid end to end (off: where each part's starts).
+__device__ __forceinline__ uint64_t gen_entry(const KArgs& a, int row, int at, const int* off, int i) {
+  int p = 0;  // the last part whose entries start at or before i
+#pragma unroll
+  for (int s = 32; s > 0; s >>= 1)
+    if (off[p + s] <= i) p += s;
+  return __hip_atomic_load(&a.p_list[(static_cast<size_t>(row) * a.P + p) * kGenPartList + at + (i - off[p])],
+                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// off[0, 64] from the parts' counts number `which`, by one wave.
+__device__ __forceinline__ void gen_offsets(const KArgs& a, int row, int which, int* off) {
+  const int lane = threadIdx.x & 63;
+  const int n = lane < a.P ? __hip_atomic_load(&a.p_cnt[kGenPartCnt * (static_cast<size_t>(row) * a.P + lane) + which],
+                                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                           : 0;
+  off[lane + 1] = static_cast<int>(wave_incl_scan(static_cast<uint32_t>(n)));
+  if (lane == 0) off[0] = 0;
+}
+// The lists that the parts of a row handed over (count `which` of each part, entries from `at` of
+// its list), one after the other into dst (at most cap). Returns the number of entries.
 template <int NT>
+__device__ __forceinline__ int gen_gather(const KArgs& a, int row, int which, int at, uint64_t* dst, int cap, int* off) {
+  const int tid = threadIdx.x;
+  if (tid < 64) gen_offsets(a, row, which, off);
+  __syncthreads();
+  const int m = min(sgpr_i32(off[64]), cap);
+  for (int i = tid; i < m; i += NT) dst[i] = gen_entry(a, row, at, off, i);
+  __syncthreads();
+  return m;
+}
+// This part's lists and counts are stored (device-scope): takes the row's ticket (k_gen_max cleared
+// it) and returns true, the other parts' stores visible, in the part that takes the last one.
+__device__ __forceinline__ bool gen_last_part(const KArgs& a, int row, int* flag) {
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this thread's stores have completed
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const unsigned n = __hip_atomic_fetch_add(&a.g_tick[row], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const bool last = n == static_cast<unsigned>(a.P - 1);
+    if (last) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");  // as in k_topk_split
+    *flag = last;
+  }
+  __syncthreads();
+  return *flag != 0;
+}
+
+// NT threads per workgroup: 1024, or 512 (two workgroups per CU, each holding its row's passes
+// while the other's wait on memory) for batches with more general rows than CUs. SPLIT: a workgroup
+// per part of a row, after k_gen_max and k_gen_hist.
+template <int NT, bool SPLIT = false>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_general(KArgs a) {
   constexpr int kGenThreads = NT;
   __shared__ GenShared<NT> sh;
+  __shared__ int part_off[2][SPLIT ? kGenMaxParts + 1 : 1];
   const int V = a.V;
   const int tid = threadIdx.x;
   // Workgroup b takes the b-th general row. With per-row parameters the general rows are then the
   // first workgroups, which the dispatcher deals out evenly over the XCDs (one per CU at a time);
   // by row index they could crowd one XCD into a second round.
-  int row = blockIdx.x;
-  if (a.params) {
+  int row = SPLIT ? static_cast<int>(blockIdx.x) / a.P : static_cast<int>(blockIdx.x);
+  if (!SPLIT && a.params) {
     if (tid == 0) sh.ints[0] = -1;
     int base = 0;
     for (int r0 = 0; r0 < a.B; r0 += kGenThreads) {
@@ -1796,7 +2159,31 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
   g.R.bits = a.s_bits + static_cast<size_t>(row) * a.words;
   g.R.lds_bits = false;
   uint64_t mxc = 0ull, mnk = ~0ull;
-  if (a.gen_fused) {
+  GenPart part = {};  // SPLIT: this workgroup's part of the row
+  ulonglong2 hraw[SPLIT ? kGenBuckets / NT / 2 : 1];
+  int4 pcnt = {};
+  double2 pmass = {};
+  if constexpr (SPLIT) {
+    static_assert(NT == kGsNT, "a part's elements are held by its threads");
+    part = gen_part(a);
+    // what does not depend on the row's range, asked for first: the histogram (this thread's
+    // buckets) and what k_gen_hist counted per part
+    const ulonglong2* hf = reinterpret_cast<const ulonglong2*>(a.p_hfix + static_cast<size_t>(row) * kGenBuckets +
+                                                               kGenBuckets / kGenThreads * tid);
+#pragma unroll
+    for (int i = 0; i < kGenBuckets / kGenThreads / 2; ++i) hraw[i] = hf[i];
+    {
+      const size_t slot = static_cast<size_t>(row) * a.P + min(tid & 63, a.P - 1);
+      pcnt = *reinterpret_cast<const int4*>(&a.p_cnt[kGenPartCnt * slot]);
+      pmass = *reinterpret_cast<const double2*>(&a.p_mass[2 * slot]);
+    }
+    if (tid < 8) sh.ints[tid] = tid == 0 ? kGenBuckets : 0;
+    if (tid < 4) sh.fb[tid] = kGenBuckets;
+    uint32_t mn;
+    gen_part_range(a, row, mxc, mn);
+    mnk = mn;
+    __syncthreads();  // exp_tab_fill
+  } else if (a.gen_fused) {
     // Row mode: the penalty bitmap (src/sampler.cpp:53-65) straight into LDS (it fits: V <= 2^19),
     // then one pass for the row maximum and minimum. The row's later passes follow soon enough to
     // find much of it still in the Infinity Cache.
@@ -1865,30 +2252,147 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
     mxc = block_max64<kGenThreads>(mxc, sh.r64);
     mnk = block_min64<kGenThreads>(mnk, sh.r64);
   }
-  g.mx = comp_val(mxc);
-  g.temp = P.temp;
-  g.inv_temp = 1.0 / static_cast<double>(P.temp);
-  bool capped;  // the buckets stop short of the row minimum: the overflow bucket may hold most of it
-  {
-    float range = g.mx - key_val(static_cast<uint32_t>(mnk));
-    const float cap = 64.0f * P.temp;
-    capped = !(range <= cap);
-    if (capped) range = cap;
-    g.qs = range > 0.0f ? static_cast<float>(kGenBuckets) / range : 0.0f;
-  }
+  bool capped;
+  gen_scale(g, P.temp, mxc, static_cast<uint32_t>(mnk), capped);
   const int k = top_k_of(P, V);
   int flags = 0;
 
   // penalised-id count for the diagnostics
   uint32_t np = 0;
-  if (g.R.pen) {
-    for (int i = tid; i < a.words; i += kGenThreads) np += __popc(g.R.bits[i]);
-  }
-  np = block_sum_u32<kGenThreads>(np, sh.r32);
+  auto count_pen = [&]() {
+    if (g.R.pen) {
+      for (int i = tid; i < a.words; i += kGenThreads) np += __popc(g.R.bits[i]);
+    }
+    np = block_sum_u32<kGenThreads>(np, sh.r32);
+  };
+  if constexpr (!SPLIT) count_pen();
 
   // top-k prefix when 256 < k < V: the k-th element by count
   g.ckk = 0ull;
-  if (k < V) {
+  // SPLIT: alone = the rest of the row is taken by this workgroup by itself (part 0; the others have
+  // returned), pass by pass as without the split. Every part decides it from the same values.
+  bool alone = !SPLIT || !gen_split_row(k, V);
+  if constexpr (SPLIT)
+    if (alone && part.part != 0) return;
+  constexpr int BP = kGenBuckets / kGenThreads;
+  static_assert(BP % 4 == 0, "a thread's buckets are read as 16-byte vectors");
+  const int b0 = BP * tid;
+  int qk = 0;  // SPLIT, k < V: the bucket of the k-th element
+  double rm[SPLIT ? BP : 1], ms_before = 0.0;  // SPLIT: the inclusive masses of this thread's buckets
+  uint32_t rc[SPLIT ? BP : 1];
+  if constexpr (SPLIT) {
+    if (!alone) {
+      // the row's histogram, as k_gen_hist left it: this thread's buckets, then their prefixes
+      const int lane = tid & 63, w = tid >> 6;
+      double om = 0.0;
+      int oc = 0;
+      if (capped) {  // the overflow bucket, counted per part
+        om = lane < a.P ? pmass.y : 0.0;
+        oc = lane < a.P ? pcnt.z : 0;
+        for (int o = 32; o > 0; o >>= 1) {
+          om += __shfl_xor(om, o);
+          oc += __shfl_xor(oc, o);
+        }
+      }
+      const double wq = table_width(g.qs, P.temp);
+      double ms = 0.0;
+      uint32_t cs = 0;
+#pragma unroll
+      for (int i = 0; i < BP; ++i) {
+        const int b = b0 + i;
+        const uint64_t raw = (i & 1) ? hraw[i >> 1].y : hraw[i >> 1].x;
+        rc[i] = gen_raw_count(raw);
+        const double e = exp_tab(-static_cast<double>(b | 1) * wq);  // the main pass's table point
+        rm[i] = e * (static_cast<double>(raw - rc[i] * kFixRawE) * kFixUnit);
+        if (capped && b == kGenBuckets - 1) {
+          rc[i] = static_cast<uint32_t>(oc);
+          rm[i] = om;
+        }
+        ms += rm[i];
+        cs += rc[i];
+      }
+      const double im = wave_incl_scan_f64(ms);
+      const uint32_t ic = wave_incl_scan(cs);
+      if (lane == 63) {
+        sh.wm[w] = im;
+        sh.wc[w] = ic;
+      }
+      __syncthreads();
+      double em = 0.0;
+      uint32_t ec = 0u, total = 0u;
+#pragma unroll
+      for (int i = 0; i < GenShared<NT>::kGenNW; ++i) {
+        if (i == w) {
+          em = ms_before;
+          ec = total;
+        }
+        ms_before += sh.wm[i];
+        total += sh.wc[i];
+      }
+      em += im - ms;
+      ec += ic - cs;
+      int first = kGenBuckets;
+#pragma unroll
+      for (int i = 0; i < BP; ++i) {
+        em += rm[i];
+        const uint32_t n = rc[i];
+        ec += n;
+        rm[i] = n ? em : -1.0;  // no target is found in an empty bucket
+        sh.mass0[b0 + i] = em;
+        sh.cnt0[b0 + i] = ec;
+        if (first == kGenBuckets && ec >= static_cast<uint32_t>(k)) first = b0 + i;
+      }
+      if (k < V) wave_claim_min(&sh.ints[0], first < kGenBuckets, first);
+      __syncthreads();
+      if (sgpr_u32(total) != static_cast<uint32_t>(V)) {  // a bucket's count was not decoded
+        alone = true;
+        if (part.part != 0) return;
+        __syncthreads();
+      }
+    }
+    if (!alone) {
+      if (k < V) {  // the elements through the k-th's bucket have to fit one list
+        qk = sgpr_i32(sh.ints[0]);
+        alone = qk >= kGenBuckets || (capped && qk == kGenBuckets - 1) || sgpr_u32(sh.cnt0[min(qk, kGenBuckets - 1)]) > kGenPartList;
+        if (alone && part.part != 0) return;
+        __syncthreads();
+      }
+    }
+  }
+  // f(bucket, composite) for each of this part's elements; pv, pnibs: the part's first chunk.
+  auto part_each = [&](float4 (&pv)[kGsU], uint32_t pnibs, auto&& f) {
+    for (int c0 = part.g0; c0 < part.g1; c0 += kGsChunk) {
+      if (c0 != part.g0) {
+        gen_part_load(g.R.rp, V, part, c0, pv);
+        pnibs = g.R.pen ? gen_part_nibs(g.R.bits, part, c0) : 0u;
+      }
+#pragma unroll
+      for (int u = 0; u < kGsU; ++u) {
+        const int e = 4 * (c0 + u * kGenThreads + tid);
+        if (e >= part.hi) continue;
+        float x[4] = {pv[u].x, pv[u].y, pv[u].z, pv[u].w};
+        gen_part_penalise(g.R, (pnibs >> (4 * u)) & 0xFu, x);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (e + i < V) f(q_of(g, x[i]), comp(ord_key(x[i]), static_cast<uint32_t>(e + i)));
+      }
+    }
+  };
+  // hands this part's two lists over; false: another part ends the row
+  unsigned long long* plist = nullptr;
+  auto hand_over = [&]() -> bool {
+    __syncthreads();
+    if (tid < 2)
+      __hip_atomic_store(&a.p_cnt[kGenPartCnt * (static_cast<size_t>(row) * a.P + part.part) + kGenPartListA + tid], sh.ints[tid == 0 ? 4 : 7],
+                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return gen_last_part(a, row, &sh.ints[6]);
+  };
+  auto append = [&](int* n, int at, int cap, uint64_t ck) {
+    const int p = atomicAdd(n, 1);
+    if (p < cap) __hip_atomic_store(&plist[at + p], static_cast<unsigned long long>(ck), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  };
+  if constexpr (SPLIT) plist = a.p_list + (static_cast<size_t>(row) * a.P + part.part) * kGenPartList;
+  if (alone && k < V) {
     auto all_v = [](float) { return true; };
     auto all_c = [](uint64_t) { return true; };
     const Sel s = refine_select<false>(g, sh, all_v, all_c, static_cast<uint64_t>(static_cast<uint32_t>(mnk)) << 32, mxc, V, 0,
@@ -1900,6 +2404,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
   // relative to the table points, numer_fix, in the mass array's 8-byte slots until the prefix
   // below turns them into fp64 masses)
   uint64_t* fix0 = reinterpret_cast<uint64_t*>(sh.mass0);
+  if (alone)
   for (int i = tid; i < kGenBuckets; i += kGenThreads) {
     sh.cnt0[i] = 0u;
     fix0[i] = 0ull;
@@ -1908,17 +2413,18 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
   // prefix below has used it
   double* etab = sh.rmass;
   const double wq = table_width(g.qs, P.temp);
+  if (alone)
   for (int j = tid; j < kGenBuckets / 2; j += kGenThreads) etab[j] = exp_tab(-static_cast<double>(2 * j + 1) * wq);
   const FixCoef fc = fix_coef(wq, P.temp, g.inv_temp);
   // The main pass also collects the min-p prefix (its elements' exact numerators are taken there)
   // into the list, which aliases the refinement counts, idle until the pass ends.
-  if (tid == 0) sh.ints[4] = 0;
-  __syncthreads();
+  if (alone) {
+    if (tid == 0) sh.ints[4] = 0;
+    __syncthreads();
+  }
   const bool minp = P.min_p > 0.0f;
   const double thr = static_cast<double>(P.min_p);  // pr of the maximum is exactly 1
-  // A floor under d = v - mx (the float the numerators take) for every element whose numerator can
-  // reach thr, d / temp >= log(thr) (exp within 1e-15): the exact numerator is taken only above it.
-  const float dmin = minp ? static_cast<float>(static_cast<double>(P.temp) * log(thr) * 1.001) - 1e-3f : INFINITY;
+  const float dmin = minp ? minp_floor(P.temp, thr) : INFINITY;
   double t_totm = 0.0, t_omass = 0.0;
   uint64_t t_ofix = 0ull;
   uint32_t t_cntm = 0, t_ocnt = 0;
@@ -1994,7 +2500,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
   const bool flat = comp_key(mxc) == static_cast<uint32_t>(mnk) && isfinite(g.mx);
   // one instance per combination without a top-k restriction (the common case: no per-element
   // branches beyond the ones asked for); rows with one share an instance
-  if (flat) {
+  if (!alone) {  // SPLIT: k_gen_hist took the pass
+  } else if (flat) {
     const int n_in = cut_k ? k : V;
     if (tid == 0) {
       sh.cnt0[0] = static_cast<uint32_t>(n_in);
@@ -2019,7 +2526,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
     main_pass(std::false_type{}, std::true_type{}, std::false_type{});
   else
     main_pass(std::false_type{}, std::false_type{}, std::false_type{});
-  {
+  if (alone) {
     const uint32_t oc = block_sum_u32<kGenThreads>(t_ocnt, sh.r32);
     const double om = block_sum_f64<kGenThreads>(t_omass, sh.rd);
     for (int o = 32; o > 0; o >>= 1) t_ofix += __shfl_xor(t_ofix, o);
@@ -2032,7 +2539,20 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
   }
   double totm = 0.0;
   uint32_t cntm = 0;
-  if (minp) {
+  int nlist = 0;  // SPLIT: the min-p prefix's listed elements
+  if (minp && !alone) {
+    totm = (tid & 63) < a.P ? pmass.x : 0.0;
+    int n = (tid & 63) < a.P ? pcnt.x : 0;
+    nlist = (tid & 63) < a.P ? pcnt.y : 0;
+    for (int o = 32; o > 0; o >>= 1) {
+      totm += __shfl_xor(totm, o);
+      n += __shfl_xor(n, o);
+      nlist += __shfl_xor(nlist, o);
+    }
+    totm = sgpr_f64(totm);
+    cntm = static_cast<uint32_t>(sgpr_i32(n));
+    nlist = sgpr_i32(nlist);
+  } else if (minp) {
     totm = block_sum_f64<kGenThreads>(t_totm, sh.rd);
     cntm = block_sum_u32<kGenThreads>(t_cntm, sh.r32);
   }
@@ -2050,10 +2570,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
     return block_min64<kGenThreads>(t, sh.r64);
   };
   // level-0 inclusive prefixes (BP consecutive buckets per thread, bucket 0 = closest to the maximum)
-  constexpr int BP = kGenBuckets / kGenThreads;
-  static_assert(BP % 4 == 0, "a thread's buckets are read as 16-byte vectors");
-  const int b0 = BP * tid;
-  {
+  if (alone) {
     double m[BP];
     uint32_t c[BP];
     double ms = 0.0;
@@ -2083,7 +2600,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
     __syncthreads();
   }
   // the sum over the top-k prefix (src/sampler.cpp:84): the histogram's total
-  const double sum = sgpr_f64(sh.mass0[kGenBuckets - 1]);
+  double sum = sgpr_f64(sh.mass0[kGenBuckets - 1]);
 
   // src/sampler.cpp:86-91 (min-p), with the count of a prefix
   int keep = k;
@@ -2102,7 +2619,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
       last_from = 2;
     }
   }
-  const int keep_minp = keep;
+  int keep_minp = keep;
 
   // The first non-empty level-0 bucket whose inclusive mass reaches target (kGenBuckets: none), each
   // thread looking in its own BP consecutive buckets (read as 16-byte vectors). The k-th search
@@ -2191,9 +2708,9 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
 
   // src/sampler.cpp:101-108 draws u * tot over the kept prefix; u is taken first because, in the
   // usual case below, the top-p cut and the draw share one pass over the row.
-  if (tid == 0) sh.dbls[1] = draw_u(a, row, P);
-  __syncthreads();
-  const double u = sgpr_f64(sh.dbls[1]);
+  if (!SPLIT && tid == 0) sh.dbls[1] = draw_u(a, row, P);
+  if (!SPLIT) __syncthreads();
+  const double u = SPLIT ? a.x_u[row] : sgpr_f64(sh.dbls[1]);  // SPLIT: k_gen_max drew it
   const bool topp = P.top_p > 0.0f && P.top_p < 1.0f;
   const double tp = static_cast<double>(P.top_p);
   const double near_tp = near_topp(k);
@@ -2218,7 +2735,217 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
   // Small min-p prefix: its elements (numerator >= thr, all of them close to the maximum) are
   // collected whole, by the main pass as a rule; the top-p cut and the draw are then taken on the
   // sorted prefix sums.
-  if (minp && cntm >= 1u && cntm <= static_cast<uint32_t>(kGenCap)) {
+  if constexpr (SPLIT) {
+    if (!alone && k < V) {
+      // A top-k of at most kGenCap elements: every element through the k-th's bucket, listed by the
+      // parts and put in order by the last one (each bucket's entries at its count prefix, then
+      // ranked within the bucket), in the histogram's mass array, read no more. The sum, the cuts and
+      // the draw are taken on the sorted list.
+      float4 pv[kGsU];
+      gen_part_load(g.R.rp, V, part, part.g0, pv);
+      part_each(pv, g.R.pen ? gen_part_nibs(g.R.bits, part, part.g0) : 0u, [&](int q, uint64_t ck) {
+        if (q <= qk) append(&sh.ints[4], 0, kGenPartList, ck);
+      });
+      if (!hand_over()) return;
+      alone = true;
+      uint64_t* big = reinterpret_cast<uint64_t*>(sh.mass0);            // kGenPartList entries
+      uint32_t* fill = reinterpret_cast<uint32_t*>(big + kGenPartList);  // per bucket
+      static_assert(kGenPartList * 8 + kGenBuckets * 4 <= kGenBuckets * 8, "both fit the mass array");
+      for (int i = tid; i < kGenBuckets; i += kGenThreads) fill[i] = 0u;
+      // gathered through the refinement area (the lists' own place), half a list at a time at most
+      int* off = part_off[0];
+      const int m = gen_gather<NT>(a, row, kGenPartListA, 0, sh.list, 2 * kGenCap, off);
+      static_assert(sizeof(sh.list) + sizeof(sh.lpr) >= kGenPartList * 8, "the gathered list");
+      for (int i = tid; i < m; i += kGenThreads) {
+        const uint64_t x = sh.list[i];
+        const int q = q_of(g, comp_val(x));
+        big[(q > 0 ? sh.cnt0[q - 1] : 0u) + atomicAdd(&fill[q], 1u)] = x;
+      }
+      __syncthreads();
+      for (int i = tid; i < m; i += kGenThreads) {
+        const uint64_t x = big[i];
+        const int q = q_of(g, comp_val(x));
+        const int s0 = q > 0 ? static_cast<int>(sh.cnt0[q - 1]) : 0, s1 = static_cast<int>(sh.cnt0[q]);
+        int r = s0;
+        for (int j = s0; j < s1; ++j) r += big[j] > x;
+        if (r < k) sh.list[r] = x;
+      }
+      __syncthreads();
+      scan_sorted<true>(g, sh, sh.list, sh.lpr, k, 0, 0.0, INFINITY);
+      g.ckk = sgpr_u64(sh.list[k - 1]);
+      sum = sgpr_f64(sh.lpr[k - 1]);
+      if (minp) {
+        cntm = 0u;
+        for (int i = tid; i < k; i += kGenThreads) cntm += numer_g(g, comp_val(sh.list[i])) >= thr;
+        cntm = block_sum_u32<kGenThreads>(cntm, sh.r32);
+        keep = max(1, static_cast<int>(cntm));
+      }
+      keep_minp = keep;
+      tot = sgpr_f64(sh.lpr[keep - 1]);
+      last = sgpr_u64(sh.list[keep - 1]);
+      last_from = 2;
+      if (topp) apply_topp(find_in_prefix(sh, sh.list, sh.lpr, keep, 0, 0.0, tp * sum));
+      target = u * tot;
+      d = find_in_prefix(sh, sh.list, sh.lpr, keep, 0, 0.0, target);
+      shared = drawn = true;
+    }
+  }
+  if constexpr (SPLIT) {
+    if (!alone) {
+      // Top-k off: the shared pass below over the parts, or (no cut to find) the draw's bucket alone.
+      // List A: the cut's bucket; list B: the buckets the draw may fall in.
+      constexpr int LC = kGenCap / 2;
+      static_assert(LC == NT, "one entry of each list per thread");
+      const int lane = tid & 63, w = tid >> 6;
+      float4 pv[kGsU];
+      gen_part_load(g.R.rp, V, part, part.g0, pv);
+      const uint32_t pnibs = g.R.pen && part.hi > part.lo ? gen_part_nibs(g.R.bits, part, part.g0) : 0u;
+      auto first_bucket = [&](double t) {
+        int f = kGenBuckets;
+#pragma unroll
+        for (int i = BP - 1; i >= 0; --i)
+          if (rm[i] >= t) f = b0 + i;
+        return f;
+      };
+      const bool listed = minp && cntm >= 1u && cntm <= static_cast<uint32_t>(kGenCap);
+      const bool cut = topp && !(tot < tp * sum * (1.0 - near_tp));
+      const double tgt = tp * sum;
+      int qp = kGenBuckets, d_lo = kGenBuckets, d_hi = kGenBuckets, ra_p = 0;
+      double above_p = 0.0;
+      bool plan = false;
+      if (!listed && cut && tgt > 0.0 && u > 0.0) {
+        int f = first_bucket(tgt);
+        wave_claim_min(&sh.fb[0], f < kGenBuckets, f);
+        __syncthreads();
+        qp = sgpr_i32(sh.fb[0]);
+        if (qp < kGenBuckets) {
+          ra_p = qp > 0 ? sgpr_i32(static_cast<int>(sh.cnt0[qp - 1])) : 0;
+          above_p = qp > 0 ? sgpr_f64(sh.mass0[qp - 1]) : 0.0;
+          const int cnt_p = sgpr_i32(static_cast<int>(sh.cnt0[qp]));
+          if (cnt_p < keep && cnt_p - ra_p <= LC) {
+            f = first_bucket(u * above_p);
+            wave_claim_min(&sh.fb[1], f < kGenBuckets, f);
+            f = first_bucket(u * sgpr_f64(sh.mass0[qp]) * (1.0 + 1e-12));  // slack: tot's sum order differs
+            wave_claim_min(&sh.fb[2], f < kGenBuckets, f);
+            __syncthreads();
+            d_lo = sgpr_i32(sh.fb[1]);
+            d_hi = sgpr_i32(sh.fb[2]);
+            plan = true;
+          }
+        }
+      } else if (!listed && !cut && u * tot > 0.0) {
+        target = u * tot;
+        const int f = first_bucket(target);
+        wave_claim_min(&sh.fb[1], f < kGenBuckets, f);
+        __syncthreads();
+        d_lo = d_hi = sgpr_i32(sh.fb[1]);
+        plan = true;
+      }
+      const int base_d = d_lo > 0 && d_lo < kGenBuckets ? sgpr_i32(static_cast<int>(sh.cnt0[d_lo - 1])) : 0;
+      plan = plan && d_hi < kGenBuckets && sgpr_i32(static_cast<int>(sh.cnt0[min(d_hi, kGenBuckets - 1)])) - base_d <= LC;
+      if (!plan) {
+        // the min-p prefix, which k_gen_hist listed, or a plan whose lists do not fit: one workgroup
+        // ends the row
+        if (part.part != 0) return;
+        alone = true;
+        __syncthreads();
+        if (tid < 4) sh.fb[tid] = kGenBuckets;
+        if (tid == 0) sh.ints[4] = nlist;
+        if (listed && nlist == static_cast<int>(cntm))
+          gen_gather<NT>(a, row, 1, 0, sh.list, kGenCap, part_off[0]);
+        else
+          __syncthreads();
+      } else {
+        part_each(pv, pnibs, [&](int q, uint64_t ck) {
+          if (q == qp) append(&sh.ints[4], 0, LC, ck);
+          if (q >= d_lo && q <= d_hi) append(&sh.ints[7], LC, LC, ck);
+        });
+        if (!hand_over()) return;
+        alone = true;
+        uint64_t* listA = sh.list;
+        uint64_t* listB = sh.list + LC;
+        double* lprA = sh.lpr;
+        double* lprB = sh.lpr + LC;
+        if (w < 2) gen_offsets(a, row, kGenPartListA + w, part_off[w]);
+        if (tid < 4) sh.fb[tid] = kGenBuckets;
+        if (tid < 2) sh.ints[tid] = LC;
+        __syncthreads();
+        const int mA = min(sgpr_i32(part_off[0][64]), LC), mB = min(sgpr_i32(part_off[1][64]), LC);
+        const uint64_t xA = tid < mA ? gen_entry(a, row, 0, part_off[0], tid) : 0ull;
+        const uint64_t xB = tid < mB ? gen_entry(a, row, LC, part_off[1], tid) : 0ull;
+        listA[tid] = xA;
+        listB[tid] = xB;
+        __syncthreads();
+        if (max(mA, mB) <= kGenRankMax) {
+          int rA = 0, rB = 0;
+          if (tid < mA) rA = rank_count(listA, mA, xA);
+          if (tid < mB) rB = rank_count(listB, mB, xB);
+          const double wA = numer_g(g, comp_val(xA)), wB = numer_g(g, comp_val(xB));
+          __syncthreads();
+          if (tid < mA) {
+            listA[rA] = xA;
+            lprA[rA] = wA;
+          }
+          if (tid < mB) {
+            listB[rB] = xB;
+            lprB[rB] = wB;
+          }
+        } else {
+          bitonic_desc<NT>(listA, LC);
+          bitonic_desc<NT>(listB, LC);
+          lprA[tid] = numer_g(g, comp_val(listA[tid]));
+          lprB[tid] = numer_g(g, comp_val(listB[tid]));
+        }
+        __syncthreads();
+        // running sums through both lists, and the first entry of each that reaches its target
+        const double above_d = d_lo > 0 ? sgpr_f64(sh.mass0[d_lo - 1]) : 0.0;
+        double iA = wave_incl_scan_f64(tid < mA ? lprA[tid] : 0.0);
+        double iB = wave_incl_scan_f64(tid < mB ? lprB[tid] : 0.0);
+        if (lane == 63) {
+          sh.wm[w] = iA;
+          sh.rd[w] = iB;
+        }
+        __syncthreads();
+        double pA = above_p, pB = above_d;
+        for (int i = 0; i < w; ++i) {
+          pA += sh.wm[i];
+          pB += sh.rd[i];
+        }
+        iA += pA;
+        iB += pB;
+        lprA[tid] = iA;
+        lprB[tid] = iB;
+        if (cut) {
+          wave_claim_min(&sh.ints[0], tid < mA && iA >= tgt, tid);
+          __syncthreads();
+          int j = sgpr_i32(sh.ints[0]);
+          Sel s;
+          s.found = j < mA;
+          if (!s.found) j = mA - 1;  // rounding left the target just past the list
+          s.ck = sgpr_u64(listA[j]);
+          s.rank = ra_p + j;
+          s.before = j > 0 ? sgpr_f64(lprA[j - 1]) : above_p;
+          s.incl = sgpr_f64(lprA[j]);
+          apply_topp(s);
+          target = u * tot;
+          flags |= VSMP_FLAG_ONE_PASS;
+        }
+        wave_claim_min(&sh.ints[1], tid < mB && iB >= target, tid);
+        __syncthreads();
+        const int j = sgpr_i32(sh.ints[1]);
+        if (j < mB) {  // (not so: rounding at the list's end; a select of its own below)
+          d.found = true;
+          d.ck = sgpr_u64(listB[j]);
+          d.rank = base_d + j;
+          d.before = j > 0 ? sgpr_f64(lprB[j - 1]) : above_d;
+          d.incl = sgpr_f64(lprB[j]);
+          drawn = true;
+        }
+        shared = true;
+      }
+    }
+  }
+  if (!shared && minp && cntm >= 1u && cntm <= static_cast<uint32_t>(kGenCap)) {
     // the main pass's list holds the prefix when every element it counted was collected there (not
     // so for a capped row whose overflow bucket a tiny min-p threshold keeps); otherwise a pass
     // collects every element above a float floor just below the min-p threshold
@@ -2335,6 +3062,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
   }
   margin = tot > 0.0 ? margin / tot : 0.0;
   if (margin < kNearDraw) flags |= VSMP_FLAG_DRAW_NEAR;
+  if constexpr (SPLIT)
+    if (a.info) count_pen();
   if (tid == 0) {
     if (a.x_flag) {
       a.x_flag[row] = (flags & VSMP_FLAG_TOPP_NEAR) ? 1 : 0;
@@ -4356,6 +5085,13 @@ void launch_rows(const KArgs& a, hipStream_t st) {
   static DynLdsOnce configured;
   allow_dyn_lds(configured, {reinterpret_cast<const void*>(k_rows)}, static_cast<int>(kRowMaxDynLds));
   hipLaunchKernelGGL(k_rows, dim3(a.B), dim3(kRowNT), dyn, st, a);
+}
+
+void launch_general_split(const KArgs& a, hipStream_t st) {
+  const dim3 grid(static_cast<unsigned>(a.B * a.P)), nt(kGsNT);
+  hipLaunchKernelGGL(k_gen_max, grid, nt, 0, st, a);
+  hipLaunchKernelGGL(k_gen_hist, grid, nt, 0, st, a);
+  hipLaunchKernelGGL((k_general<kGsNT, true>), grid, nt, 0, st, a);
 }
 
 void launch_general_exact(const KArgs& a, int slots, hipStream_t st) {
