@@ -236,24 +236,29 @@ int topk_parts(int B, int V, int cus, int k, bool forced, long long forced_p) {
 // 30.2 against 69.4 us, 16 rows 42.6 / 74.1, 64 rows 66.3 / 79.8, 128 rows 89.4 / 83.0; 49,152 logits
 // 1 row 27.9 / 38.5, 32 rows 36.8 / 40.7, 64 rows 43.3 / 40.8. The line between lies near B = V / 1600;
 // the split is taken to V / 2000.
-GenParts general_parts(int B, int V, bool forced, long long forced_p) {
+// per_row: the greedy and small-k rows among them are cut into the same parts (k_topk_split's, so
+// register-held ones, at most 16), and a batch that cannot be takes no split.
+GenParts general_parts(int B, int V, bool per_row, bool forced, long long forced_p) {
   const long long V4 = (static_cast<long long>(V) + 3) / 4;
   const long long most = static_cast<long long>(kGenPartChunk) * kGenPartChunks;
   const long long pmin = (V4 + most - 1) / most;
   const long long pmax = std::max(pmin, std::min<long long>(kGenMaxParts, V4 / 256));
+  const long long tmin = (V4 + kSplitMaxPartGroups - 1) / kSplitMaxPartGroups, tmax = kMergeCap / kKmax;
   if (pmin > kGenMaxParts || static_cast<long long>(B) * kGenMaxParts > INT32_MAX / kGenPartList) return {};
   const long long want = forced_p > 0 ? forced_p : std::llround(std::sqrt(V / (64.0 * B)));
-  const long long P = std::min(std::max(want, pmin), pmax);
+  long long P = std::min(std::max(want, pmin), pmax);
+  if (per_row && tmin > tmax) P = 0;
+  if (per_row && P > 0) P = std::min(std::max(P, tmin), tmax);
   if (forced) return {static_cast<int>(P), static_cast<size_t>(B), static_cast<size_t>(B * P)};
   const long long rows = std::min<long long>(B, V / 2000);
   if (rows < 1 || pmax < 2) return {};
-  const long long slots = std::max({rows * pmin, rows * P, static_cast<long long>(std::sqrt(rows * (V / 64.0)) + 0.5 * rows) + 1});
+  const long long slots = std::max({rows * std::max(pmin, std::min(tmin, tmax)), rows * P, static_cast<long long>(std::sqrt(rows * (V / 64.0)) + 0.5 * rows) + 1});
   return {rows == B && P >= 2 ? static_cast<int>(P) : 0, static_cast<size_t>(rows), static_cast<size_t>(slots)};
 }
 
 // Where the split general rows' scratch lies in its allocation, 16-byte aligned.
 struct SplitScratch {
-  size_t list, hfix, max, mass, cnt, min, bits, tick, bytes;
+  size_t list, hfix, max, mass, cnt, min, bits, tick, cand, tcnt, tpen, bytes;
 };
 SplitScratch split_scratch(const GenParts& gp, int words) {
   const size_t rows = gp.rows, slots = gp.slots;
@@ -272,6 +277,9 @@ SplitScratch split_scratch(const GenParts& gp, int words) {
   s.min = take(slots * sizeof(unsigned));
   s.bits = take(rows * static_cast<size_t>(words) * sizeof(unsigned));
   s.tick = take(rows * sizeof(unsigned));
+  s.cand = take(slots * kKmax * sizeof(uint64_t));
+  s.tcnt = take(slots * sizeof(int));
+  s.tpen = take(slots * sizeof(int));
   s.bytes = at;
   return s;
 }
@@ -325,11 +333,15 @@ Plan plan(const vsmp_ctx* ctx, int B, int V, const vsmp_params* hostp) {
     // leaves those rows alone), on a stream forked from the caller's: the few long general rows
     // then overlap the row kernel instead of following it.
     pl.side_general = !hostp;
-    // k <= kGenCap or top-k off: k_general's split takes the row (with per-row parameters it leaves
-    // other rows to one of their workgroups)
+    // k <= kGenCap or top-k off: the split takes the row (with per-row parameters it leaves other
+    // general rows to one of their workgroups)
     if (pl.any_general && fm != 1) {
-      pl.gen = general_parts(B, V, fm == 2, ctx->split_p);
+      pl.gen = general_parts(B, V, !hostp, fm == 2, ctx->split_p);
       pl.gen_split = pl.gen.P > 0 && (!hostp || hostp->top_k <= kGenCap || hostp->top_k >= V);
+      if (pl.gen_split) {  // one workgroup per part of every row, on the caller's stream
+        pl.side_general = false;
+        pl.no_rows_kernel = true;
+      }
     }
     pl.any_smallk = false;
     pl.any_finish = false;
@@ -490,6 +502,9 @@ int launch_batch(vsmp_ctx* ctx, const float* logits, int B, int V, long long ld,
     a.s_min = reinterpret_cast<unsigned*>(ctx->p_scr + ss.min);
     a.s_bits = reinterpret_cast<unsigned*>(ctx->p_scr + ss.bits);
     a.g_tick = reinterpret_cast<unsigned*>(ctx->p_scr + ss.tick);
+    a.s_cand = reinterpret_cast<unsigned long long*>(ctx->p_scr + ss.cand);
+    a.s_cnt = reinterpret_cast<int*>(ctx->p_scr + ss.tcnt);
+    a.s_npen = reinterpret_cast<int*>(ctx->p_scr + ss.tpen);
   }
   a.gen_fused = pl.rows ? 1 : 0;
   a.x_flag = exact ? ctx->x_flag : nullptr;
@@ -514,10 +529,7 @@ int launch_batch(vsmp_ctx* ctx, const float* logits, int B, int V, long long ld,
     if (!hip_ok(hipEventRecord(ctx->fork_ev, st), "hipEventRecord") ||
         !hip_ok(hipStreamWaitEvent(ctx->side, ctx->fork_ev, 0), "hipStreamWaitEvent"))
       return -1;
-    if (pl.gen_split)
-      launch_general_split(a, ctx->side);
-    else
-      launch_general(a, ctx->cus, ctx->side);
+    launch_general(a, ctx->cus, ctx->side);
     bool ok = hip_ok(hipGetLastError(), "general-path launch");
     if (ok && exact) {
       launch_general_exact(a, exact_slots(a.x_n, B), ctx->side);

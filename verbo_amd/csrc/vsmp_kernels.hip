@@ -26,7 +26,8 @@
 //            row, with histograms in LDS. In row mode it takes the row's maximum pass and penalty
 //            bitmap itself.
 //  k_gen_max, k_gen_hist, k_general<512, true>  the same for a batch of few general rows: each row cut
-//            into parts over several CUs, one launch per pass.
+//            into parts over several CUs, one launch per pass; with per-row parameters the last launch
+//            takes the greedy and small-k rows as well, as k_topk_split does.
 //  k_general_exact  after k_general: the rows it marked (a top-p cut at rounding distance of
 //            top_p) redone in the reference's order and sequential sums.
 //  k_read_probe  a plain streaming read, for the attainable-bandwidth measurement.
@@ -1768,6 +1769,332 @@ __device__ __forceinline__ Sel refine_select(const GenCtx& g, GenShared<NT>& sh,
   return scan_sorted<MASS>(g, sh, sh.list, sh.lpr, m, rank_above, above, target);
 }
 
+constexpr int kRowBins = 2048;
+// One wave searches 2048 bins from the top (bucket 2047 first) for the first bucket whose running
+// count reaches `need` (such a bucket is never empty). Lane l first sums buckets 2047-32l down to
+// 2016-32l; a scan over lanes finds the 32 buckets holding the crossing, and a second scan over
+// those (one per lane) the bucket. out[0] = bucket (-1 when the bins hold fewer than `need`),
+// out[1] = count above it, out[2] = its own count.
+__device__ void wave_find_bucket(const uint32_t* bins, int need, int* out) {
+  const int lane = threadIdx.x & 63;
+  const int lo = kRowBins - 32 * (lane + 1);
+  const uint4* p = reinterpret_cast<const uint4*>(bins + lo);
+  uint32_t s = 0;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const uint4 v = p[j];
+    s += v.x + v.y + v.z + v.w;
+  }
+  const uint32_t incl = wave_incl_scan(s);
+  const uint64_t m = __ballot(static_cast<int>(incl) >= need);
+  if (m == 0ull) {
+    if (lane == 0) {
+      out[0] = -1;
+      out[1] = 0;
+      out[2] = 0;
+    }
+    return;
+  }
+  const int L = __ffsll(static_cast<long long>(m)) - 1;
+  const int exL = __builtin_amdgcn_readlane(static_cast<int>(incl - s), L);
+  const int loL = kRowBins - 32 * (L + 1);
+  const uint32_t c = lane < 32 ? bins[loL + 31 - lane] : 0u;
+  const uint32_t in2 = wave_incl_scan(c);
+  const uint64_t m2 = __ballot(lane < 32 && exL + static_cast<int>(in2) >= need);
+  const int t = __ffsll(static_cast<long long>(m2)) - 1;
+  if (lane == t) {
+    out[0] = loL + 31 - t;
+    out[1] = exL + static_cast<int>(in2 - c);
+    out[2] = static_cast<int>(c);
+  }
+}
+
+// ---- split top-k rows: a small batch of small-k rows, each row cut into parts in one launch -------
+//
+// The counterpart of k_greedy_split for rows with 0 < k <= 256 (src/sampler.cpp:71-108): row r's
+// 16-byte groups are cut into P contiguous parts, one 512-thread workgroup each. A part holds its
+// elements as penalised order keys in registers (all its loads in flight at once), bounds its
+// ks-th key from below by the ks-th largest of its 512 lane maxima (two 2048-bin histogram levels
+// in LDS), selects its exact top-ks composites among the keys above that bound with further
+// histogram passes over the registers, and writes them, sorted, with device-scope stores. The part
+// that takes the row's last device-scope ticket merges the P lists and runs the reference epilogue
+// (finish_smallk, as k_finish does after slices), then clears the ticket for the next call.
+
+constexpr int kTkNT = 512;
+constexpr int kTkW = kTkNT / 64;
+constexpr int kTkU = 8;                     // 16-byte loads per thread: the whole part in flight
+static_assert(kTkNT * kTkU == kSplitMaxPartGroups, "the planner sizes parts by kSplitMaxPartGroups");
+
+struct __align__(16) TkShared {
+  uint32_t bins[2][kRowBins];                // row-bound and select histograms (read as uint4)
+  uint32_t bits[kSplitMaxPartGroups / 8];    // the part's penalty bitmap (4 elements per group)
+  uint64_t top[kKmax];                       // the part's top-ks; the merged top-k
+  int rank[kKmax];
+  uint64_t red64[kTkW];
+  uint32_t red32[kTkW];
+  int ints[16];
+  int off[kMaxMergeSlices + 1];
+  uint64_t mbuf[kMergeCap];                  // the last part's merge and epilogue workspace
+};
+static_assert(kEpiWs + kKmax <= kMergeCap, "the epilogue's workspace and numerators live in mbuf");
+
+// Takes the row's ticket once every store of this part has completed; true in the part that takes the
+// last one, with the ticket cleared for the next call.
+__device__ __forceinline__ bool topk_last_part(const KArgs& a, int row, int* flag) {
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const unsigned t = __hip_atomic_fetch_add(&a.g_tick[row], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const bool last = t == static_cast<unsigned>(a.P - 1);
+    // The last part: every other part's lists and counts were stored with agent-scope stores and had
+    // completed (vmcnt(0)) before that part's ticket, whose read-modify-write returned P - 1 to this
+    // part only after all of them. An agent-scope acquire here, as k_greedy_split's last part takes,
+    // drops what this CU's and this XCD's caches hold of them, so the merge that follows (agent-scope
+    // loads, ordered after it by the barrier) cannot be served a line read before the ticket.
+    if (last) {
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+      __hip_atomic_store(&a.g_tick[row], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    *flag = last;
+  }
+  __syncthreads();
+  return *flag != 0;
+}
+
+// Part `part` of a small-k row (k_topk_split), or of a greedy row in k_general<kTkNT, true, true>,
+// whose parts hand over their first maximum only.
+__device__ __forceinline__ void topk_part(const KArgs& a, TkShared& sh, const vsmp_params& P, int row, int part,
+                                          bool greedy = false) {
+  const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
+  const int V = a.V;
+  const int V4 = (V + 3) >> 2;
+  const int G = (V4 + a.P - 1) / a.P;
+  const int g0 = min(V4, part * G), g1 = min(V4, g0 + G);
+  const int lo = 4 * g0;  // the part's elements: [lo, hi)
+  const int hi = min(V, 4 * g1);
+  const int ks = min(top_k_of(P, V), max(0, hi - lo));
+  const size_t slot = static_cast<size_t>(row) * a.P + part;
+
+  int h0, h1;
+  row_hist(a, row, h0, h1);
+  const int H = h1 - h0;
+  const bool pen = (P.repeat != 1.0f) && H > 0;
+  const int hfrom = h0 + ((P.repeat_last > 0 && H > P.repeat_last) ? H - P.repeat_last : 0);
+  constexpr int HQ = 4;
+  int hid[HQ];
+  if (pen) {
+#pragma unroll
+    for (int q = 0; q < HQ; ++q) hid[q] = a.hist[min(hfrom + q * kTkNT + tid, h1 - 1)];
+  }
+  const uint4* rp4 = reinterpret_cast<const uint4*>(a.logits + static_cast<size_t>(row) * static_cast<size_t>(a.ld));
+  const int glast = g1 > g0 ? g1 - 1 : V4 - 1;
+  uint4 v[kTkU];
+#pragma unroll
+  for (int u = 0; u < kTkU; ++u) v[u] = stream_ld(rp4 + min(g0 + u * kTkNT + tid, glast));
+
+  for (int i = tid; i < 2 * kRowBins; i += kTkNT) (&sh.bins[0][0])[i] = 0u;
+  if (tid == 0) sh.ints[8] = 0;
+  // penalty bitmap of the part (src/sampler.cpp:53-65)
+  const int words = (hi - lo + 31) >> 5;
+  if (pen) {
+    for (int i = tid; i < words; i += kTkNT) sh.bits[i] = 0u;
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < HQ; ++q) {
+      const int id = hid[q];
+      if (hfrom + q * kTkNT + tid < h1 && id >= lo && id < hi) atomicOr(&sh.bits[(id - lo) >> 5], 1u << ((id - lo) & 31));
+    }
+    for (int i = hfrom + HQ * kTkNT + tid; i < h1; i += kTkNT) {
+      const int id = a.hist[i];
+      if (id >= lo && id < hi) atomicOr(&sh.bits[(id - lo) >> 5], 1u << ((id - lo) & 31));
+    }
+  }
+  __syncthreads();
+  if (a.pen_bits && pen) or_pen_ids<kTkNT>(a, row, lo, sh.bits, words);
+
+  // penalised order keys in place (0: past the part), the lane maximum and the part's maximum
+  uint32_t lm = 0u;
+  uint64_t mxc = 0ull;
+#pragma unroll
+  for (int u = 0; u < kTkU; ++u) {
+    const int f = g0 + u * kTkNT + tid;
+    const int e = 4 * f;
+    float x[4] = {__uint_as_float(v[u].x), __uint_as_float(v[u].y), __uint_as_float(v[u].z), __uint_as_float(v[u].w)};
+    if (pen && f < g1) {
+      const uint32_t nib = (sh.bits[(e - lo) >> 5] >> ((e - lo) & 31)) & 0xFu;
+      if (nib) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+          if (nib & (1u << c)) x[c] = penalise(x[c], P.repeat);
+      }
+    }
+    uint32_t kk[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      kk[c] = (f < g1 && e + c < V) ? ord_key(x[c]) : 0u;
+      lm = max(lm, kk[c]);
+      if (kk[c]) mxc = max64(mxc, comp(kk[c], static_cast<uint32_t>(e + c)));
+    }
+    v[u] = make_uint4(kk[0], kk[1], kk[2], kk[3]);
+  }
+  mxc = block_max64<kTkNT>(mxc, sh.red64);
+
+  if (greedy) {  // src/sampler.cpp:66-70
+    uint32_t np = 0;
+    if (a.info && pen) {
+      for (int i = tid; i < words; i += kTkNT) np += __popc(sh.bits[i]);
+      np = block_sum_u32<kTkNT>(np, sh.red32);
+    }
+    if (tid == 0) {
+      __hip_atomic_store(&a.s_cand[slot * kKmax], static_cast<unsigned long long>(mxc), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_store(&a.s_npen[slot], static_cast<int>(np), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    if (!topk_last_part(a, row, &sh.ints[9]) || w != 0) return;
+    const size_t s0 = static_cast<size_t>(row) * a.P;
+    uint64_t m = lane < a.P ? __hip_atomic_load(&a.s_cand[(s0 + lane) * kKmax], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0ull;
+    int n = lane < a.P ? __hip_atomic_load(&a.s_npen[s0 + lane], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
+    for (int o = 32; o > 0; o >>= 1) {
+      m = max64(m, __shfl_xor(m, o));
+      n += __shfl_xor(n, o);
+    }
+    if (lane == 0) {
+      const int id = comp_idx(m);
+      a.out[row] = id;
+      if (a.info) {
+        vsmp_row_info inf = {};
+        inf.id = id;
+        inf.path = kPathGreedy;
+        inf.k = inf.keep_minp = inf.keep = 1;
+        inf.last_id = id;
+        inf.mx = comp_val(m);
+        inf.n_pen = n;
+        a.info[row] = inf;
+      }
+    }
+    return;
+  }
+
+  // row bound T (to 2^10 keys): the ks-th largest lane maximum, from two histogram levels
+  uint32_t T = 0u;
+  if (ks > 0) {
+    atomicAdd(&sh.bins[0][lm >> 21], 1u);
+    __syncthreads();
+    if (w == 0) wave_find_bucket(sh.bins[0], ks, sh.ints);
+    __syncthreads();
+    const int b1 = sh.ints[0];
+    if (static_cast<int>(lm >> 21) == b1) atomicAdd(&sh.bins[1][(lm >> 10) & 2047u], 1u);
+    __syncthreads();
+    if (w == 0) wave_find_bucket(sh.bins[1], ks - sh.ints[1], sh.ints + 4);
+    __syncthreads();
+    const int b2 = sh.ints[4];
+    T = (b1 >= 0 && b2 >= 0) ? ((static_cast<uint32_t>(b1) << 21) | (static_cast<uint32_t>(b2) << 10)) : 0u;
+    T = __builtin_amdgcn_readfirstlane(T);
+    for (int i = tid; i < 2 * kRowBins; i += kTkNT) (&sh.bins[0][0])[i] = 0u;
+    __syncthreads();
+  }
+
+  // the part's list: every composite >= clo, collected in LDS (at most kKmax kept)
+  auto collect = [&](uint64_t clo) {
+#pragma unroll
+    for (int u = 0; u < kTkU; ++u) {
+      const uint32_t kk[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
+      const int e = 4 * (g0 + u * kTkNT + tid);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const uint64_t cc = kk[c] ? comp(kk[c], static_cast<uint32_t>(e + c)) : 0ull;
+        const bool t = ks > 0 && kk[c] != 0u && cc >= clo;
+        const uint64_t m = __ballot(t);
+        if (m) {
+          int base = 0;
+          if (lane == 0) base = atomicAdd(&sh.ints[8], __popcll(m));
+          base = __builtin_amdgcn_readfirstlane(base);  // lane 0: every lane is active here
+          const int pos = base + static_cast<int>(__builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(m >> 32),
+                                                                            __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(m), 0u)));
+          if (t && pos < kKmax) sh.top[pos] = cc;
+        }
+      }
+    }
+  };
+  // Usually the keys above the bound fit the list: it is kept whole (the merge takes the row's top
+  // k from the union of the lists, each sorted). Otherwise the exact ks-th largest composite is found
+  // first: 2048-bin passes over the composites >= T << 32 in registers, each narrowing [clo, chi]
+  // to the bucket that holds it, until the bucket is taken whole; the list is then exactly ks long.
+  uint32_t nabove = 0;
+#pragma unroll
+  for (int u = 0; u < kTkU; ++u)
+    nabove += (v[u].x >= T && v[u].x != 0u) + (v[u].y >= T && v[u].y != 0u) + (v[u].z >= T && v[u].z != 0u) +
+              (v[u].w >= T && v[u].w != 0u);
+  nabove = block_sum_u32<kTkNT>(nabove, sh.red32);
+  uint64_t clo = static_cast<uint64_t>(T) << 32;
+  if (ks > 0 && nabove > static_cast<uint32_t>(kKmax)) {
+  uint64_t chi = mxc;
+  int need = ks;
+  for (int pass = 0; clo != chi && pass < 9; ++pass) {
+    const uint64_t R = chi - clo;
+    const int sft = R < static_cast<uint64_t>(kRowBins) ? 0 : 53 - __clzll(static_cast<long long>(R));
+    uint32_t* bins = sh.bins[pass & 1];
+    for (int i = tid; i < kRowBins; i += kTkNT) sh.bins[(pass + 1) & 1][i] = 0u;
+#pragma unroll
+    for (int u = 0; u < kTkU; ++u) {
+      const uint32_t kk[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
+      const int e = 4 * (g0 + u * kTkNT + tid);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        if (kk[c] < T || kk[c] == 0u) continue;
+        const uint64_t cc = comp(kk[c], static_cast<uint32_t>(e + c));
+        if (cc >= clo && cc <= chi) atomicAdd(&bins[(cc - clo) >> sft], 1u);
+      }
+    }
+    __syncthreads();
+    if (w == 0) wave_find_bucket(bins, need, sh.ints);
+    __syncthreads();
+    const int b = sh.ints[0];
+    const int inb = sh.ints[2];
+    need -= sh.ints[1];
+    __syncthreads();
+    if (b < 0) break;  // unreachable: ks composites lie at or above T << 32
+    const uint64_t nlo = clo + (static_cast<uint64_t>(b) << sft);
+    const uint64_t wdt = sft == 0 ? 0ull : (1ull << sft) - 1ull;
+    chi = (chi - nlo < wdt) ? chi : nlo + wdt;
+    clo = nlo;
+    if (inb == need) chi = clo;  // the whole bucket is taken: the top ks are the composites >= clo
+  }
+  }
+  collect(clo);
+  if (tid < kKmax) sh.rank[tid] = 0;
+  __syncthreads();
+  const int nt = min(sh.ints[8], kKmax);
+  {
+    const int parts = nt <= 64 ? kTkW : kTkNT / max(nt, 1);
+    const int pw = nt <= 64 ? w : tid / max(nt, 1);
+    const int ci = nt <= 64 ? lane : tid % max(nt, 1);
+    if (nt > 0 && pw < parts && ci < nt) {
+      const int chunk = (nt + parts - 1) / parts;
+      const uint64_t x = sh.top[ci];
+      int r = 0;
+      const int j1 = min(nt, (pw + 1) * chunk);
+      for (int j = pw * chunk; j < j1; ++j) r += sh.top[j] > x;
+      if (r) atomicAdd(&sh.rank[ci], r);
+    }
+  }
+  __syncthreads();
+  for (int i = tid; i < nt; i += kTkNT)
+    __hip_atomic_store(&a.s_cand[slot * kKmax + sh.rank[i]], sh.top[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  uint32_t np = 0;
+  if (a.info && pen) {
+    for (int i = tid; i < words; i += kTkNT) np += __popc(sh.bits[i]);
+    np = block_sum_u32<kTkNT>(np, sh.red32);
+  }
+  if (tid == 0) {
+    __hip_atomic_store(&a.s_cnt[slot], nt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(&a.s_npen[slot], static_cast<int>(np), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  if (!topk_last_part(a, row, &sh.ints[9])) return;
+  finish_smallk<kTkNT, true>(a, row, P, a.P, sh.mbuf, sh.top, sh.red64, sh.ints, sh.off);
+}
+
 // ---- split general rows: a small batch's general rows, each cut into parts over several CUs -------
 //
 // With fewer general rows than CUs, k_general's one workgroup per row leaves most of the chip idle
@@ -1871,6 +2198,7 @@ __global__ __launch_bounds__(kGsNT) void k_gen_max(KArgs a) {
   __shared__ uint64_t red[kGsNT / 64];
   const GenPart t = gen_part(a);
   const int tid = threadIdx.x, V = a.V, row = t.row;
+  if (t.part == 0 && tid == 0) a.g_tick[row] = 0u;
   const vsmp_params P = sgpr_params(row_params(a, row));
   if (path_of(P, V, a.smallk_ok) != kPathGeneral) return;
   int h0, h1;
@@ -1891,10 +2219,7 @@ __global__ __launch_bounds__(kGsNT) void k_gen_max(KArgs a) {
   gen_part_load(rp, V, t, t.g0, v);
   for (int b = t.part * kGenBuckets / a.P + tid; b < (t.part + 1) * kGenBuckets / a.P; b += kGsNT)
     a.p_hfix[static_cast<size_t>(row) * kGenBuckets + b] = 0ull;
-  if (t.part == 0 && tid == 0) {
-    a.x_u[row] = draw_u(a, row, P);
-    a.g_tick[row] = 0u;
-  }
+  if (t.part == 0 && tid == 0) a.x_u[row] = draw_u(a, row, P);
   if (R.pen) {  // src/sampler.cpp:53-65
     const int words = (t.hi - t.lo + 31) >> 5;
     for (int i = tid; i < words; i += kGsNT) bits[i] = 0u;
@@ -2111,7 +2436,9 @@ __device__ __forceinline__ bool gen_last_part(const KArgs& a, int row, int* flag
 // NT threads per workgroup: 1024, or 512 (two workgroups per CU, each holding its row's passes
 // while the other's wait on memory) for batches with more general rows than CUs. SPLIT: a workgroup
 // per part of a row, after k_gen_max and k_gen_hist.
-template <int NT, bool SPLIT = false>
+// MIXED: a batch with per-row parameters, whose greedy and small-k rows' parts are k_topk_split's,
+// taken in the last launch, so that the batch needs no other kernel and no second stream.
+template <int NT, bool SPLIT = false, bool MIXED = false>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_general(KArgs a) {
   constexpr int kGenThreads = NT;
   __shared__ GenShared<NT> sh;
@@ -2143,6 +2470,14 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
   }
   // the row, so its parameters and history window, are the same in every lane: scalar registers
   const vsmp_params P = sgpr_params(row_params(a, row));
+  if constexpr (MIXED) {
+    static_assert(NT == kTkNT && sizeof(TkShared) <= sizeof(GenShared<NT>), "the parts share the general rows' LDS");
+    const int path = path_of(P, V, a.smallk_ok);
+    if (path != kPathGeneral) {
+      topk_part(a, reinterpret_cast<TkShared&>(sh), P, row, static_cast<int>(blockIdx.x) - row * a.P, path == kPathGreedy);
+      return;
+    }
+  }
   if (path_of(P, V, a.smallk_ok) != kPathGeneral) return;
   const int S = a.S;
   exp_tab_fill();  // ordered before its first use by the barriers of the reductions below
@@ -3532,7 +3867,6 @@ constexpr int kRowNT = 1024;
 constexpr int kRowW = kRowNT / 64;
 constexpr int kRowU = 4;
 constexpr int kWaveCap = 512;
-constexpr int kRowBins = 2048;
 
 static_assert(kEpiWs <= 16 * 512, "k_rows lends its candidate buffers to the epilogue");
 
@@ -3593,45 +3927,6 @@ __device__ __forceinline__ uint64_t wave_max_u64(uint64_t v) {
   const uint32_t lo = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), 63));
   const uint32_t hi = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v >> 32), 63));
   return (static_cast<uint64_t>(hi) << 32) | lo;
-}
-
-// One wave searches 2048 bins from the top (bucket 2047 first) for the first bucket whose running
-// count reaches `need` (such a bucket is never empty). Lane l first sums buckets 2047-32l down to
-// 2016-32l; a scan over lanes finds the 32 buckets holding the crossing, and a second scan over
-// those (one per lane) the bucket. out[0] = bucket (-1 when the bins hold fewer than `need`),
-// out[1] = count above it, out[2] = its own count.
-__device__ void wave_find_bucket(const uint32_t* bins, int need, int* out) {
-  const int lane = threadIdx.x & 63;
-  const int lo = kRowBins - 32 * (lane + 1);
-  const uint4* p = reinterpret_cast<const uint4*>(bins + lo);
-  uint32_t s = 0;
-#pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    const uint4 v = p[j];
-    s += v.x + v.y + v.z + v.w;
-  }
-  const uint32_t incl = wave_incl_scan(s);
-  const uint64_t m = __ballot(static_cast<int>(incl) >= need);
-  if (m == 0ull) {
-    if (lane == 0) {
-      out[0] = -1;
-      out[1] = 0;
-      out[2] = 0;
-    }
-    return;
-  }
-  const int L = __ffsll(static_cast<long long>(m)) - 1;
-  const int exL = __builtin_amdgcn_readlane(static_cast<int>(incl - s), L);
-  const int loL = kRowBins - 32 * (L + 1);
-  const uint32_t c = lane < 32 ? bins[loL + 31 - lane] : 0u;
-  const uint32_t in2 = wave_incl_scan(c);
-  const uint64_t m2 = __ballot(lane < 32 && exL + static_cast<int>(in2) >= need);
-  const int t = __ffsll(static_cast<long long>(m2)) - 1;
-  if (lane == t) {
-    out[0] = loL + 31 - t;
-    out[1] = exL + static_cast<int>(in2 - c);
-    out[2] = static_cast<int>(c);
-  }
 }
 
 // Wave-local: penalise the not yet penalised history entries [from, cnt) of a buffer.
@@ -4162,249 +4457,10 @@ __global__ __launch_bounds__(kRowNT) void k_rows(KArgs a) {
   }
 }
 
-// ---- split top-k rows: a small batch of small-k rows, each row cut into parts in one launch -------
-//
-// The counterpart of k_greedy_split for rows with 0 < k <= 256 (src/sampler.cpp:71-108): row r's
-// 16-byte groups are cut into P contiguous parts, one 512-thread workgroup each. A part holds its
-// elements as penalised order keys in registers (all its loads in flight at once), bounds its
-// ks-th key from below by the ks-th largest of its 512 lane maxima (two 2048-bin histogram levels
-// in LDS), selects its exact top-ks composites among the keys above that bound with further
-// histogram passes over the registers, and writes them, sorted, with device-scope stores. The part
-// that takes the row's last device-scope ticket merges the P lists and runs the reference epilogue
-// (finish_smallk, as k_finish does after slices), then clears the ticket for the next call.
-
-constexpr int kTkNT = 512;
-constexpr int kTkW = kTkNT / 64;
-constexpr int kTkU = 8;                     // 16-byte loads per thread: the whole part in flight
-static_assert(kTkNT * kTkU == kSplitMaxPartGroups, "the planner sizes parts by kSplitMaxPartGroups");
-
-struct __align__(16) TkShared {
-  uint32_t bins[2][kRowBins];                // row-bound and select histograms (read as uint4)
-  uint32_t bits[kSplitMaxPartGroups / 8];    // the part's penalty bitmap (4 elements per group)
-  uint64_t top[kKmax];                       // the part's top-ks; the merged top-k
-  int rank[kKmax];
-  uint64_t red64[kTkW];
-  uint32_t red32[kTkW];
-  int ints[16];
-  int off[kMaxMergeSlices + 1];
-  uint64_t mbuf[kMergeCap];                  // the last part's merge and epilogue workspace
-};
-static_assert(kEpiWs + kKmax <= kMergeCap, "the epilogue's workspace and numerators live in mbuf");
-
 __global__ __launch_bounds__(kTkNT) void k_topk_split(KArgs a) {
   __shared__ TkShared sh;
   const int row = static_cast<int>(blockIdx.x) / a.P;
-  const int part = static_cast<int>(blockIdx.x) - row * a.P;
-  const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
-  const vsmp_params& P = a.shared;
-  const int V = a.V;
-  const int V4 = (V + 3) >> 2;
-  const int G = (V4 + a.P - 1) / a.P;
-  const int g0 = min(V4, part * G), g1 = min(V4, g0 + G);
-  const int lo = 4 * g0;  // the part's elements: [lo, hi)
-  const int hi = min(V, 4 * g1);
-  const int ks = min(top_k_of(P, V), max(0, hi - lo));
-  const size_t slot = static_cast<size_t>(row) * a.P + part;
-
-  int h0, h1;
-  row_hist(a, row, h0, h1);
-  const int H = h1 - h0;
-  const bool pen = (P.repeat != 1.0f) && H > 0;
-  const int hfrom = h0 + ((P.repeat_last > 0 && H > P.repeat_last) ? H - P.repeat_last : 0);
-  constexpr int HQ = 4;
-  int hid[HQ];
-  if (pen) {
-#pragma unroll
-    for (int q = 0; q < HQ; ++q) hid[q] = a.hist[min(hfrom + q * kTkNT + tid, h1 - 1)];
-  }
-  const uint4* rp4 = reinterpret_cast<const uint4*>(a.logits + static_cast<size_t>(row) * static_cast<size_t>(a.ld));
-  const int glast = g1 > g0 ? g1 - 1 : V4 - 1;
-  uint4 v[kTkU];
-#pragma unroll
-  for (int u = 0; u < kTkU; ++u) v[u] = stream_ld(rp4 + min(g0 + u * kTkNT + tid, glast));
-
-  for (int i = tid; i < 2 * kRowBins; i += kTkNT) (&sh.bins[0][0])[i] = 0u;
-  if (tid == 0) sh.ints[8] = 0;
-  // penalty bitmap of the part (src/sampler.cpp:53-65)
-  const int words = (hi - lo + 31) >> 5;
-  if (pen) {
-    for (int i = tid; i < words; i += kTkNT) sh.bits[i] = 0u;
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < HQ; ++q) {
-      const int id = hid[q];
-      if (hfrom + q * kTkNT + tid < h1 && id >= lo && id < hi) atomicOr(&sh.bits[(id - lo) >> 5], 1u << ((id - lo) & 31));
-    }
-    for (int i = hfrom + HQ * kTkNT + tid; i < h1; i += kTkNT) {
-      const int id = a.hist[i];
-      if (id >= lo && id < hi) atomicOr(&sh.bits[(id - lo) >> 5], 1u << ((id - lo) & 31));
-    }
-  }
-  __syncthreads();
-  if (a.pen_bits && pen) or_pen_ids<kTkNT>(a, row, lo, sh.bits, words);
-
-  // penalised order keys in place (0: past the part), the lane maximum and the part's maximum
-  uint32_t lm = 0u;
-  uint64_t mxc = 0ull;
-#pragma unroll
-  for (int u = 0; u < kTkU; ++u) {
-    const int f = g0 + u * kTkNT + tid;
-    const int e = 4 * f;
-    float x[4] = {__uint_as_float(v[u].x), __uint_as_float(v[u].y), __uint_as_float(v[u].z), __uint_as_float(v[u].w)};
-    if (pen && f < g1) {
-      const uint32_t nib = (sh.bits[(e - lo) >> 5] >> ((e - lo) & 31)) & 0xFu;
-      if (nib) {
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-          if (nib & (1u << c)) x[c] = penalise(x[c], P.repeat);
-      }
-    }
-    uint32_t kk[4];
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      kk[c] = (f < g1 && e + c < V) ? ord_key(x[c]) : 0u;
-      lm = max(lm, kk[c]);
-      if (kk[c]) mxc = max64(mxc, comp(kk[c], static_cast<uint32_t>(e + c)));
-    }
-    v[u] = make_uint4(kk[0], kk[1], kk[2], kk[3]);
-  }
-  mxc = block_max64<kTkNT>(mxc, sh.red64);
-
-  // row bound T (to 2^10 keys): the ks-th largest lane maximum, from two histogram levels
-  uint32_t T = 0u;
-  if (ks > 0) {
-    atomicAdd(&sh.bins[0][lm >> 21], 1u);
-    __syncthreads();
-    if (w == 0) wave_find_bucket(sh.bins[0], ks, sh.ints);
-    __syncthreads();
-    const int b1 = sh.ints[0];
-    if (static_cast<int>(lm >> 21) == b1) atomicAdd(&sh.bins[1][(lm >> 10) & 2047u], 1u);
-    __syncthreads();
-    if (w == 0) wave_find_bucket(sh.bins[1], ks - sh.ints[1], sh.ints + 4);
-    __syncthreads();
-    const int b2 = sh.ints[4];
-    T = (b1 >= 0 && b2 >= 0) ? ((static_cast<uint32_t>(b1) << 21) | (static_cast<uint32_t>(b2) << 10)) : 0u;
-    T = __builtin_amdgcn_readfirstlane(T);
-    for (int i = tid; i < 2 * kRowBins; i += kTkNT) (&sh.bins[0][0])[i] = 0u;
-    __syncthreads();
-  }
-
-  // the part's list: every composite >= clo, collected in LDS (at most kKmax kept)
-  auto collect = [&](uint64_t clo) {
-#pragma unroll
-    for (int u = 0; u < kTkU; ++u) {
-      const uint32_t kk[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
-      const int e = 4 * (g0 + u * kTkNT + tid);
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        const uint64_t cc = kk[c] ? comp(kk[c], static_cast<uint32_t>(e + c)) : 0ull;
-        const bool t = ks > 0 && kk[c] != 0u && cc >= clo;
-        const uint64_t m = __ballot(t);
-        if (m) {
-          int base = 0;
-          if (lane == 0) base = atomicAdd(&sh.ints[8], __popcll(m));
-          base = __builtin_amdgcn_readfirstlane(base);  // lane 0: every lane is active here
-          const int pos = base + static_cast<int>(__builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(m >> 32),
-                                                                            __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(m), 0u)));
-          if (t && pos < kKmax) sh.top[pos] = cc;
-        }
-      }
-    }
-  };
-  // Usually the keys above the bound fit the list: it is kept whole (the merge takes the row's top
-  // k from the union of the lists, each sorted). Otherwise the exact ks-th largest composite is found
-  // first: 2048-bin passes over the composites >= T << 32 in registers, each narrowing [clo, chi]
-  // to the bucket that holds it, until the bucket is taken whole; the list is then exactly ks long.
-  uint32_t nabove = 0;
-#pragma unroll
-  for (int u = 0; u < kTkU; ++u)
-    nabove += (v[u].x >= T && v[u].x != 0u) + (v[u].y >= T && v[u].y != 0u) + (v[u].z >= T && v[u].z != 0u) +
-              (v[u].w >= T && v[u].w != 0u);
-  nabove = block_sum_u32<kTkNT>(nabove, sh.red32);
-  uint64_t clo = static_cast<uint64_t>(T) << 32;
-  if (ks > 0 && nabove > static_cast<uint32_t>(kKmax)) {
-  uint64_t chi = mxc;
-  int need = ks;
-  for (int pass = 0; clo != chi && pass < 9; ++pass) {
-    const uint64_t R = chi - clo;
-    const int sft = R < static_cast<uint64_t>(kRowBins) ? 0 : 53 - __clzll(static_cast<long long>(R));
-    uint32_t* bins = sh.bins[pass & 1];
-    for (int i = tid; i < kRowBins; i += kTkNT) sh.bins[(pass + 1) & 1][i] = 0u;
-#pragma unroll
-    for (int u = 0; u < kTkU; ++u) {
-      const uint32_t kk[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
-      const int e = 4 * (g0 + u * kTkNT + tid);
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        if (kk[c] < T || kk[c] == 0u) continue;
-        const uint64_t cc = comp(kk[c], static_cast<uint32_t>(e + c));
-        if (cc >= clo && cc <= chi) atomicAdd(&bins[(cc - clo) >> sft], 1u);
-      }
-    }
-    __syncthreads();
-    if (w == 0) wave_find_bucket(bins, need, sh.ints);
-    __syncthreads();
-    const int b = sh.ints[0];
-    const int inb = sh.ints[2];
-    need -= sh.ints[1];
-    __syncthreads();
-    if (b < 0) break;  // unreachable: ks composites lie at or above T << 32
-    const uint64_t nlo = clo + (static_cast<uint64_t>(b) << sft);
-    const uint64_t wdt = sft == 0 ? 0ull : (1ull << sft) - 1ull;
-    chi = (chi - nlo < wdt) ? chi : nlo + wdt;
-    clo = nlo;
-    if (inb == need) chi = clo;  // the whole bucket is taken: the top ks are the composites >= clo
-  }
-  }
-  collect(clo);
-  if (tid < kKmax) sh.rank[tid] = 0;
-  __syncthreads();
-  const int nt = min(sh.ints[8], kKmax);
-  {
-    const int parts = nt <= 64 ? kTkW : kTkNT / max(nt, 1);
-    const int pw = nt <= 64 ? w : tid / max(nt, 1);
-    const int ci = nt <= 64 ? lane : tid % max(nt, 1);
-    if (nt > 0 && pw < parts && ci < nt) {
-      const int chunk = (nt + parts - 1) / parts;
-      const uint64_t x = sh.top[ci];
-      int r = 0;
-      const int j1 = min(nt, (pw + 1) * chunk);
-      for (int j = pw * chunk; j < j1; ++j) r += sh.top[j] > x;
-      if (r) atomicAdd(&sh.rank[ci], r);
-    }
-  }
-  __syncthreads();
-  for (int i = tid; i < nt; i += kTkNT)
-    __hip_atomic_store(&a.s_cand[slot * kKmax + sh.rank[i]], sh.top[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  uint32_t np = 0;
-  if (a.info && pen) {
-    for (int i = tid; i < words; i += kTkNT) np += __popc(sh.bits[i]);
-    np = block_sum_u32<kTkNT>(np, sh.red32);
-  }
-  if (tid == 0) {
-    __hip_atomic_store(&a.s_cnt[slot], nt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __hip_atomic_store(&a.s_npen[slot], static_cast<int>(np), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  }
-  // every store of this part has completed before its ticket is taken
-  __atomic_signal_fence(__ATOMIC_SEQ_CST);
-  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-  __atomic_signal_fence(__ATOMIC_SEQ_CST);
-  __syncthreads();
-  if (tid == 0) {
-    const unsigned t = __hip_atomic_fetch_add(&a.g_tick[row], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const bool last = t == static_cast<unsigned>(a.P - 1);
-    // The last part: every other part's lists and counts were stored with agent-scope stores and had
-    // completed (vmcnt(0)) before that part's ticket, whose read-modify-write returned P - 1 to this
-    // part only after all of them. An agent-scope acquire here, as k_greedy_split's last part takes,
-    // drops what this CU's and this XCD's caches hold of them, so the merge below (agent-scope loads,
-    // ordered after it by the barrier) cannot be served a line read before the ticket.
-    if (last) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-    sh.ints[9] = last;
-  }
-  __syncthreads();
-  if (!sh.ints[9]) return;
-  if (tid == 0) __hip_atomic_store(&a.g_tick[row], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  finish_smallk<kTkNT, true>(a, row, P, a.P, sh.mbuf, sh.top, sh.red64, sh.ints, sh.off);
+  topk_part(a, sh, a.shared, row, static_cast<int>(blockIdx.x) - row * a.P);
 }
 
 // ---- split greedy rows: a small greedy batch, each row cut into parts over several CUs ----------
@@ -5091,7 +5147,10 @@ void launch_general_split(const KArgs& a, hipStream_t st) {
   const dim3 grid(static_cast<unsigned>(a.B * a.P)), nt(kGsNT);
   hipLaunchKernelGGL(k_gen_max, grid, nt, 0, st, a);
   hipLaunchKernelGGL(k_gen_hist, grid, nt, 0, st, a);
-  hipLaunchKernelGGL((k_general<kGsNT, true>), grid, nt, 0, st, a);
+  if (a.params)
+    hipLaunchKernelGGL((k_general<kGsNT, true, true>), grid, nt, 0, st, a);
+  else
+    hipLaunchKernelGGL((k_general<kGsNT, true>), grid, nt, 0, st, a);
 }
 
 void launch_general_exact(const KArgs& a, int slots, hipStream_t st) {
