@@ -116,13 +116,12 @@ struct vsmp_ctx {
   size_t n_min = 0;
   unsigned int* s_bits = nullptr;
   size_t n_bits = 0;
-  // split greedy rows: per-row slot, ticket and penalised-id count, zero between calls
-  unsigned long long* g_slot = nullptr;
-  size_t n_slot = 0;
-  unsigned int* g_tick = nullptr;
-  size_t n_tick = 0;
-  unsigned int* g_npen = nullptr;
-  size_t n_gnpen = 0;
+  // split greedy and small-k rows: per-row slot, ticket and penalised-id count, zero between calls,
+  // 16 bytes per row; the parts' lists and counts
+  unsigned long long* g_rows = nullptr;
+  size_t n_grows = 0;
+  unsigned long long* t_scr = nullptr;
+  size_t n_tscr = 0;
   // split general rows: one allocation (split_scratch); every call fills what it reads
   unsigned char* p_scr = nullptr;
   size_t n_pscr = 0;
@@ -181,8 +180,8 @@ struct Plan {
 };
 
 // VSMP_MODE=rows|slices|split pins the decomposition (testing and tuning); default: split parts
-// for a greedy batch of at most half as many rows as CUs, or a small-k batch of at most 24 long rows
-// (topk_parts), else rows whenever the vocabulary fits the row kernel (V <= 2^19), slices beyond.
+// for a greedy batch of at most half as many rows as CUs, or a small-k batch whose parts fit the chip
+// at once (topk_parts), else rows whenever the vocabulary fits the row kernel (V <= 2^19), slices beyond.
 // split applies to greedy and small-k batches with shared parameters only; other batches take the
 // default.
 int env_mode() {
@@ -219,11 +218,16 @@ int topk_parts(int B, int V, int cus, int k, bool forced, long long forced_p) {
   const long long pmax = std::min<long long>({std::max(pmin, V4 / 512), kMaxMergeSlices, kMergeCap / kKmax});
   if (pmin > pmax) return 0;
   const long long P = forced_p > 0 ? std::min(std::max(forced_p, pmin), pmax) : pmin;
-  // Measured against row mode (top-k 40, V = 151936): faster up to B = 24 (1: 17.9 against 21.5,
-  // 8: 18.6 / 22.8, 16: 20.7 / 22.6, 24: 20.5 / 23.1 us), even at 32 (22.8 / 23.0); slower at any B
-  // when the row is short (one workgroup streams it quickly: V = 49152, 17.8 against 14.0 us).
-  // Default: B <= 24, P >= 8.
-  if (!forced && (B > 24 || P < 8)) return 0;
+  // Measured against row mode (top-k 40, back to back): 151,936 logits in 10 parts 13.4 against 20.4 us
+  // at 1 row, 16.4 / 21.6 at 24, 19.3 / 21.6 at 48, 24.4 / 22.0 at 64; 49,152 in 3 parts 11.6 / 12.9 at
+  // 1 row, 13.4 / 13.9 at 64, 15.5 / 14.1 at 96; 262,144 in 16 parts 15.0 / 27.1 at 1 row, 26.4 / 29.1
+  // at 32, 33.9 / 29.7 at 48: ahead while the parts fit the chip at once (two per CU) and, on short
+  // rows, up to about V / 250 parts. Longer lists cost the split more than row mode: k = 100 at 1 and
+  // 24 rows 18.4-21.0 / 24.6 and 23.0 / 26.4 us at 151,936, but 15.9 / 14.4 at 1 row of 49,152 and 50.1
+  // / 36.4 at 24 rows of 262,144; and from k of about 190 a part's first bound lets more keys through
+  // than a list holds (256), whose select passes take 56.3 / 33.9 us at 1 row of 151,936, k = 256.
+  const long long parts = k <= 64 ? std::min<long long>(2LL * cus, V / 250) : (k <= 100 && P >= 8 ? cus : 0);
+  if (!forced && (P < 2 || B * P > parts)) return 0;
   if (static_cast<long long>(B) * P > INT32_MAX) return 0;
   return static_cast<int>(std::max<long long>(P, 1));
 }
@@ -455,12 +459,13 @@ int launch_batch(vsmp_ctx* ctx, const float* logits, int B, int V, long long ld,
   const size_t slots = static_cast<size_t>(B) * static_cast<size_t>(pl.S);
   if (slots > static_cast<size_t>(INT32_MAX) / kKmax) return set_error("vsmp: batch too large");
   const int words = a.words;
-  if (!pl.rows && (!grow(ctx->s_cnt, ctx->n_cnt, slots, false, "scratch", st) ||  // row mode uses none of these
-                   !grow(ctx->s_npen, ctx->n_npen, slots, false, "scratch", st) ||
-                   !grow(ctx->s_max, ctx->n_max, slots, false, "scratch", st) ||
-                   !grow(ctx->s_min, ctx->n_min, slots, false, "scratch", st)))
+  const bool slices = !pl.rows && !pl.split;
+  if (slices && (!grow(ctx->s_cnt, ctx->n_cnt, slots, false, "scratch", st) ||
+                 !grow(ctx->s_npen, ctx->n_npen, slots, false, "scratch", st) ||
+                 !grow(ctx->s_max, ctx->n_max, slots, false, "scratch", st) ||
+                 !grow(ctx->s_min, ctx->n_min, slots, false, "scratch", st)))
     return -1;
-  if (pl.any_smallk && !grow(ctx->s_cand, ctx->n_cand, slots * kKmax, false, "scratch", st)) return -1;
+  if (slices && pl.any_smallk && !grow(ctx->s_cand, ctx->n_cand, slots * kKmax, false, "scratch", st)) return -1;
   // General rows marked near a top-p tie are redone exactly (rows up to kExactMaxVocab). The scratch
   // is sized whenever a batch may hold general rows, whatever its parameters, so that one call at a
   // shape sizes it for every later call at that shape (graph capture); the launch is skipped for
@@ -492,33 +497,25 @@ int launch_batch(vsmp_ctx* ctx, const float* logits, int B, int V, long long ld,
   a.s_max = ctx->s_max;
   a.s_min = ctx->s_min;
   a.s_bits = ctx->s_bits;
-  if (pl.gen_split) {
-    a.P = pl.gen.P;
-    a.p_list = reinterpret_cast<unsigned long long*>(ctx->p_scr + ss.list);
-    a.p_hfix = reinterpret_cast<unsigned long long*>(ctx->p_scr + ss.hfix);
-    a.s_max = reinterpret_cast<unsigned long long*>(ctx->p_scr + ss.max);
-    a.p_mass = reinterpret_cast<double*>(ctx->p_scr + ss.mass);
-    a.p_cnt = reinterpret_cast<int*>(ctx->p_scr + ss.cnt);
-    a.s_min = reinterpret_cast<unsigned*>(ctx->p_scr + ss.min);
-    a.s_bits = reinterpret_cast<unsigned*>(ctx->p_scr + ss.bits);
-    a.g_tick = reinterpret_cast<unsigned*>(ctx->p_scr + ss.tick);
-    a.s_cand = reinterpret_cast<unsigned long long*>(ctx->p_scr + ss.cand);
-    a.s_cnt = reinterpret_cast<int*>(ctx->p_scr + ss.tcnt);
-    a.s_npen = reinterpret_cast<int*>(ctx->p_scr + ss.tpen);
-  }
   a.gen_fused = pl.rows ? 1 : 0;
   a.x_flag = exact ? ctx->x_flag : nullptr;
   a.x_u = ctx->x_u;
   a.x_buf = ctx->x_buf;
   if (pl.split) {
-    if (!grow(ctx->g_slot, ctx->n_slot, static_cast<size_t>(B), true, "scratch", st) ||
-        !grow(ctx->g_tick, ctx->n_tick, static_cast<size_t>(B), true, "scratch", st) ||
-        !grow(ctx->g_npen, ctx->n_gnpen, static_cast<size_t>(B), true, "scratch", st))
-      return -1;
+    // per row, zero between calls, at the allocation's own capacity (a later, wider batch finds the
+    // words that it takes for its own untouched): slot, ticket, penalised-id count
+    if (!grow(ctx->g_rows, ctx->n_grows, 2 * static_cast<size_t>(B), true, "scratch", st)) return -1;
+    const size_t cap = ctx->n_grows / 2;
     a.P = pl.P;
-    a.g_slot = ctx->g_slot;
-    a.g_tick = ctx->g_tick;
-    a.g_npen = ctx->g_npen;
+    a.g_slot = ctx->g_rows;
+    a.g_tick = reinterpret_cast<unsigned int*>(ctx->g_rows + cap);
+    a.g_npen = a.g_tick + cap;
+    if (pl.topk) {  // the parts' lists, then their counts and penalised-id counts, written before they are read
+      if (!grow(ctx->t_scr, ctx->n_tscr, slots * (kKmax + 1), false, "scratch", st)) return -1;
+      a.s_cand = ctx->t_scr;
+      a.s_cnt = reinterpret_cast<int*>(ctx->t_scr + slots * kKmax);
+      a.s_npen = a.s_cnt + slots;
+    }
     if (pl.topk)
       launch_topk_split(a, st);
     else
@@ -558,10 +555,25 @@ int launch_batch(vsmp_ctx* ctx, const float* logits, int B, int V, long long ld,
     if (!hip_ok(hipGetLastError(), "finish launch")) return -1;
   }
   if (pl.any_general) {
-    if (pl.gen_split)
-      launch_general_split(a, st);
-    else
+    if (pl.gen_split) {
+      SplitArgs g;
+      static_cast<KArgs&>(g) = a;
+      g.P = pl.gen.P;
+      g.p_list = reinterpret_cast<unsigned long long*>(ctx->p_scr + ss.list);
+      g.p_hfix = reinterpret_cast<unsigned long long*>(ctx->p_scr + ss.hfix);
+      g.s_max = reinterpret_cast<unsigned long long*>(ctx->p_scr + ss.max);
+      g.p_mass = reinterpret_cast<double*>(ctx->p_scr + ss.mass);
+      g.p_cnt = reinterpret_cast<int*>(ctx->p_scr + ss.cnt);
+      g.s_min = reinterpret_cast<unsigned*>(ctx->p_scr + ss.min);
+      g.s_bits = reinterpret_cast<unsigned*>(ctx->p_scr + ss.bits);
+      g.g_tick = reinterpret_cast<unsigned*>(ctx->p_scr + ss.tick);
+      g.s_cand = reinterpret_cast<unsigned long long*>(ctx->p_scr + ss.cand);
+      g.s_cnt = reinterpret_cast<int*>(ctx->p_scr + ss.tcnt);
+      g.s_npen = reinterpret_cast<int*>(ctx->p_scr + ss.tpen);
+      launch_general_split(g, st);
+    } else {
       launch_general(a, ctx->cus, st);
+    }
     if (!hip_ok(hipGetLastError(), "general-path launch")) return -1;
     if (exact) {
       launch_general_exact(a, exact_slots(a.x_n, B), st);
@@ -867,7 +879,7 @@ void vsmp_ctx_free(vsmp_ctx* c) {
   vsmp::DeviceScope scope(c->device);
   (void)hipDeviceSynchronize();
   void* bufs[] = {c->x_flag, c->x_u,    c->x_buf,    c->s_cand, c->s_cnt,   c->s_npen,   c->s_max,
-                  c->s_min,  c->s_bits, c->g_slot,   c->g_tick, c->g_npen,  c->h_probe,  c->h_full,
+                  c->s_min,  c->s_bits, c->g_rows,   c->t_scr,  c->h_probe,  c->h_full,
                   c->h_tk,   c->h_rmode, c->h_rcand, c->h_rcnt, c->p_scr};
   for (void* p : bufs)
     if (p) (void)hipFree(p);

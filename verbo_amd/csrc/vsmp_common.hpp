@@ -80,7 +80,11 @@ struct KArgs {
   unsigned long long* g_slot;
   unsigned int* g_tick;
   unsigned int* g_npen;
-  // split general rows: P parts per row, the tickets above, per row the level-0 histogram's raw sums,
+};
+
+// Arguments of the split general rows' kernels (apart, so that the other kernels' stay as short).
+struct SplitArgs : KArgs {
+  // P parts per row, the tickets above; per row the level-0 histogram's raw sums,
   // per part its min-p prefix's mass and its overflow bucket's, kGenPartCnt counts and a list
   unsigned long long* p_hfix;  // [B][kGenBuckets]
   double* p_mass;              // [B*P][2]
@@ -96,7 +100,7 @@ void launch_rows(const KArgs& a, hipStream_t st);
 // cus: the device's CUs (0: unknown), which sets the workgroup size for large general batches.
 void launch_general(const KArgs& a, int cus, hipStream_t st);
 // General rows cut into a.P parts each: k_gen_max, k_gen_hist and k_general<512, true>.
-void launch_general_split(const KArgs& a, hipStream_t st);
+void launch_general_split(const SplitArgs& a, hipStream_t st);
 void launch_general_exact(const KArgs& a, int slots, hipStream_t st);
 void launch_numer_probe(const float* d, double* y, long long n, float temp, float qs, bool fixed_point, hipStream_t st);
 // Workgroups (and scratch slots of 2 * x_n entries) of k_general_exact for a batch of B rows: one

@@ -14,7 +14,7 @@
 //  k_greedy_split  a greedy batch of at most half as many rows as CUs: each row cut into parts
 //            over several CUs; the part that takes the row's last device-scope ticket writes the
 //            id (every cross-workgroup value travels in a device-scope atomic).
-//  k_topk_split  the same for a small-k batch of at most 24 long rows: each part selects its exact
+//  k_topk_split  the same for a small-k batch whose parts fit the chip at once: each part selects its exact
 //            top-k; the last part merges the parts' lists and runs the epilogue.
 //  k_stage1  larger vocabularies (V > 2^19), grid = rows x slices. Each workgroup loads one slice
 //            of one row into registers (the single HBM pass), applies the penalty and writes its
@@ -1088,6 +1088,21 @@ __device__ void finish_smallk(const KArgs& a, int row, const vsmp_params& P, int
   // only entries at or above it can be in the top k. Wave 0 reads the S <= 64 slice counts and
   // m-th entries in parallel (one lane each) and scans the offsets.
   const int m = (k + S - 1) / S;
+  double u = 0.0;  // the draw, asked for first
+  if (tid == 0) u = draw_u(a, row, P);
+  // COHERENT: at most kMergeCap / kKmax lists, read whole before their counts are known (one round
+  // trip to memory instead of two); what lies past a list's count is dropped below
+  constexpr int PF = 8;
+  static_assert(!COHERENT || PF * NT == kMergeCap, "every list entry in flight");
+  uint64_t vals[PF];
+  if constexpr (COHERENT) {
+#pragma unroll
+    for (int j = 0; j < PF; ++j) {
+      const int i = j * NT + tid;
+      vals[j] = 0ull;
+      if (i < S * kKmax) vals[j] = ld(&a.s_cand[static_cast<size_t>(row) * S * kKmax + i]);
+    }
+  }
   if (tid < 64) {
     int c = 0, np = 0;
     uint64_t mth = ~0ull;
@@ -1120,11 +1135,19 @@ __device__ void finish_smallk(const KArgs& a, int row, const vsmp_params& P, int
   const int M = sm_off[S];
   const uint64_t lb = sm_red64[0];
   __syncthreads();
+  if constexpr (COHERENT) {
+#pragma unroll
+    for (int j = 0; j < PF; ++j) {
+      const int i = j * NT + tid, l = i / kKmax;
+      if (i < S * kKmax && (i & (kKmax - 1)) < sm_off[l + 1] - sm_off[l] && vals[j] >= lb) {
+        const int pos = atomicAdd(&sm_int[7], 1);
+        if (pos < kMergeCap) sm_buf[pos] = vals[j];
+      }
+    }
+  }
   // the entries >= lb: entry i of the concatenated lists lies in list s2 with off[s2] <= i <
   // off[s2 + 1] (binary search); eight loads per thread go out together
-  constexpr int PF = 8;
-  for (int i0 = 0; i0 < M; i0 += NT * PF) {
-    uint64_t vals[PF];
+  for (int i0 = 0; i0 < (COHERENT ? 0 : M); i0 += NT * PF) {
 #pragma unroll
     for (int j = 0; j < PF; ++j) {
       const int i = i0 + j * NT + tid;
@@ -1166,8 +1189,6 @@ __device__ void finish_smallk(const KArgs& a, int row, const vsmp_params& P, int
   }
   __syncthreads();
   if (tid < 64) {
-    double u = 0.0;
-    if (tid == 0) u = draw_u(a, row, P);
     double* spr = reinterpret_cast<double*>(sm_buf) + kEpiWs;  // src/sampler.cpp:79-83
     const float mx = comp_val(sm_top[0]);
     for (int i = tid; i < k; i += 64) spr[i] = numer(comp_val(sm_top[i]), mx, P.temp);
@@ -1809,6 +1830,12 @@ __device__ void wave_find_bucket(const uint32_t* bins, int need, int* out) {
   }
 }
 
+// Order key without branches; +0.0f turns -0 into +0 first.
+__device__ __forceinline__ uint32_t key_of(uint32_t bits) {
+  const uint32_t b = __float_as_uint(__uint_as_float(bits) + 0.0f);
+  return b ^ (static_cast<uint32_t>(static_cast<int32_t>(b) >> 31) | 0x80000000u);
+}
+
 // ---- split top-k rows: a small batch of small-k rows, each row cut into parts in one launch -------
 //
 // The counterpart of k_greedy_split for rows with 0 < k <= 256 (src/sampler.cpp:71-108): row r's
@@ -1914,34 +1941,47 @@ __device__ __forceinline__ void topk_part(const KArgs& a, TkShared& sh, const vs
   __syncthreads();
   if (a.pen_bits && pen) or_pen_ids<kTkNT>(a, row, lo, sh.bits, words);
 
-  // penalised order keys in place (0: past the part), the lane maximum and the part's maximum
+  // the penalty bits of the thread's groups (group d of the part: word d >> 3), read from LDS together
+  // before any load is waited for; a group past g1 reads a word that may be stale, and is not used
+  uint32_t nibs = 0u;
+  if (pen) {
+#pragma unroll
+    for (int u = 0; u < kTkU; ++u) {
+      const int d = u * kTkNT + tid;
+      nibs |= ((sh.bits[d >> 3] >> ((4 * d) & 31)) & 0xFu) << (4 * u);
+    }
+  }
+  // penalised order keys in place (0: past the part) and the lane maximum
   uint32_t lm = 0u;
-  uint64_t mxc = 0ull;
 #pragma unroll
   for (int u = 0; u < kTkU; ++u) {
     const int f = g0 + u * kTkNT + tid;
-    const int e = 4 * f;
     float x[4] = {__uint_as_float(v[u].x), __uint_as_float(v[u].y), __uint_as_float(v[u].z), __uint_as_float(v[u].w)};
-    if (pen && f < g1) {
-      const uint32_t nib = (sh.bits[(e - lo) >> 5] >> ((e - lo) & 31)) & 0xFu;
-      if (nib) {
+    const uint32_t nib = (nibs >> (4 * u)) & 0xFu;
+    if (nib) {
 #pragma unroll
-        for (int c = 0; c < 4; ++c)
-          if (nib & (1u << c)) x[c] = penalise(x[c], P.repeat);
-      }
+      for (int c = 0; c < 4; ++c)
+        if (nib & (1u << c)) x[c] = penalise(x[c], P.repeat);
     }
-    uint32_t kk[4];
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      kk[c] = (f < g1 && e + c < V) ? ord_key(x[c]) : 0u;
-      lm = max(lm, kk[c]);
-      if (kk[c]) mxc = max64(mxc, comp(kk[c], static_cast<uint32_t>(e + c)));
-    }
-    v[u] = make_uint4(kk[0], kk[1], kk[2], kk[3]);
+    const int n = f < g1 ? V - 4 * f : 0;  // the group's elements inside the row (four or more: all)
+    v[u].x = n > 0 ? key_of(__float_as_uint(x[0])) : 0u;
+    v[u].y = n > 1 ? key_of(__float_as_uint(x[1])) : 0u;
+    v[u].z = n > 2 ? key_of(__float_as_uint(x[2])) : 0u;
+    v[u].w = n > 3 ? key_of(__float_as_uint(x[3])) : 0u;
+    lm = max(lm, max(max(v[u].x, v[u].y), max(v[u].z, v[u].w)));
   }
-  mxc = block_max64<kTkNT>(mxc, sh.red64);
 
   if (greedy) {  // src/sampler.cpp:66-70
+    uint64_t m0 = 0ull;
+#pragma unroll
+    for (int u = kTkU - 1; u >= 0; --u) {  // the lane's first element of its largest key
+      const uint32_t e = 4u * static_cast<uint32_t>(g0 + u * kTkNT + tid);
+      if (v[u].w == lm) m0 = comp(lm, e + 3);
+      if (v[u].z == lm) m0 = comp(lm, e + 2);
+      if (v[u].y == lm) m0 = comp(lm, e + 1);
+      if (v[u].x == lm) m0 = comp(lm, e);
+    }
+    const uint64_t mxc = block_max64<kTkNT>(lm ? m0 : 0ull, sh.red64);
     uint32_t np = 0;
     if (a.info && pen) {
       for (int i = tid; i < words; i += kTkNT) np += __popc(sh.bits[i]);
@@ -2018,18 +2058,45 @@ __device__ __forceinline__ void topk_part(const KArgs& a, TkShared& sh, const vs
     }
   };
   // Usually the keys above the bound fit the list: it is kept whole (the merge takes the row's top
-  // k from the union of the lists, each sorted). Otherwise the exact ks-th largest composite is found
-  // first: 2048-bin passes over the composites >= T << 32 in registers, each narrowing [clo, chi]
-  // to the bucket that holds it, until the bucket is taken whole; the list is then exactly ks long.
-  uint32_t nabove = 0;
+  // k from the union of the lists, each sorted). Each lane marks its keys in a mask, a wave's take
+  // their places by a scan of the counts and one LDS atomic. Otherwise the exact ks-th largest
+  // composite is found first: 2048-bin passes over the composites >= T << 32 in registers, each
+  // narrowing [clo, chi] to the bucket that holds it, until the bucket is taken whole; the list is
+  // then exactly ks long.
+  uint32_t hit = 0u;
+  {
+    const uint32_t t1 = max(T, 1u);  // 0 marks a place past the part
 #pragma unroll
-  for (int u = 0; u < kTkU; ++u)
-    nabove += (v[u].x >= T && v[u].x != 0u) + (v[u].y >= T && v[u].y != 0u) + (v[u].z >= T && v[u].z != 0u) +
-              (v[u].w >= T && v[u].w != 0u);
-  nabove = block_sum_u32<kTkNT>(nabove, sh.red32);
+    for (int u = 0; u < kTkU; ++u)
+      hit |= (static_cast<uint32_t>(v[u].x >= t1) | static_cast<uint32_t>(v[u].y >= t1) << 1 |
+              static_cast<uint32_t>(v[u].z >= t1) << 2 | static_cast<uint32_t>(v[u].w >= t1) << 3)
+             << (4 * u);
+  }
+  static_assert(4 * kTkU <= 32, "one mask bit per key");
+  if (ks == 0) hit = 0u;
+  int place;
+  {
+    const uint32_t n = __popc(hit);
+    const uint32_t incl = wave_incl_scan(n);
+    int base = 0;
+    if (lane == 63 && incl) base = atomicAdd(&sh.ints[8], static_cast<int>(incl));
+    place = __builtin_amdgcn_readlane(base, 63) + static_cast<int>(incl - n);
+  }
+  __syncthreads();
+  const int nabove = sh.ints[8];
+  if (nabove <= kKmax) {
+#pragma unroll
+    for (int u = 0; u < kTkU; ++u) {
+      if (((hit >> (4 * u)) & 0xFu) == 0u) continue;
+      const uint32_t kk[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        if ((hit >> (4 * u + c)) & 1u) sh.top[place++] = comp(kk[c], static_cast<uint32_t>(4 * (g0 + u * kTkNT + tid) + c));
+    }
+  } else {
   uint64_t clo = static_cast<uint64_t>(T) << 32;
-  if (ks > 0 && nabove > static_cast<uint32_t>(kKmax)) {
-  uint64_t chi = mxc;
+  uint64_t chi = block_max64<kTkNT>((static_cast<uint64_t>(lm) << 32) | 0xFFFFFFFFull, sh.red64);  // at or above every key
+  if (tid == 0) sh.ints[8] = 0;
   int need = ks;
   for (int pass = 0; clo != chi && pass < 9; ++pass) {
     const uint64_t R = chi - clo;
@@ -2061,8 +2128,8 @@ __device__ __forceinline__ void topk_part(const KArgs& a, TkShared& sh, const vs
     clo = nlo;
     if (inb == need) chi = clo;  // the whole bucket is taken: the top ks are the composites >= clo
   }
-  }
   collect(clo);
+  }
   if (tid < kKmax) sh.rank[tid] = 0;
   __syncthreads();
   const int nt = min(sh.ints[8], kKmax);
@@ -2193,7 +2260,7 @@ __device__ __forceinline__ void gen_part_range(const KArgs& a, int row, uint64_t
 // A row whose k-th element the split selects: top-k off, or a top-k whose elements fit one list.
 __device__ __forceinline__ bool gen_split_row(int k, int V) { return k == V || k <= kGenCap; }
 
-__global__ __launch_bounds__(kGsNT) void k_gen_max(KArgs a) {
+__global__ __launch_bounds__(kGsNT) void k_gen_max(SplitArgs a) {
   __shared__ uint32_t bits[kGenPartChunks * kGsChunk / 8];
   __shared__ uint64_t red[kGsNT / 64];
   const GenPart t = gen_part(a);
@@ -2273,7 +2340,7 @@ __global__ __launch_bounds__(kGsNT) void k_gen_max(KArgs a) {
   }
 }
 
-__global__ __launch_bounds__(kGsNT) void k_gen_hist(KArgs a) {
+__global__ __launch_bounds__(kGsNT) void k_gen_hist(SplitArgs a) {
   __shared__ unsigned long long fix0[kGenBuckets];
   __shared__ uint64_t list[kGenCap];
   __shared__ uint64_t red[kGsNT / 64];
@@ -2387,7 +2454,7 @@ __global__ __launch_bounds__(kGsNT) void k_gen_hist(KArgs a) {
 }
 
 // Entry i of the parts' lists of a row laid end to end (off: where each part's starts).
-__device__ __forceinline__ uint64_t gen_entry(const KArgs& a, int row, int at, const int* off, int i) {
+__device__ __forceinline__ uint64_t gen_entry(const SplitArgs& a, int row, int at, const int* off, int i) {
   int p = 0;  // the last part whose entries start at or before i
 #pragma unroll
   for (int s = 32; s > 0; s >>= 1)
@@ -2396,7 +2463,7 @@ __device__ __forceinline__ uint64_t gen_entry(const KArgs& a, int row, int at, c
                            __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 // off[0, 64] from the parts' counts number `which`, by one wave.
-__device__ __forceinline__ void gen_offsets(const KArgs& a, int row, int which, int* off) {
+__device__ __forceinline__ void gen_offsets(const SplitArgs& a, int row, int which, int* off) {
   const int lane = threadIdx.x & 63;
   const int n = lane < a.P ? __hip_atomic_load(&a.p_cnt[kGenPartCnt * (static_cast<size_t>(row) * a.P + lane) + which],
                                                __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
@@ -2407,7 +2474,7 @@ __device__ __forceinline__ void gen_offsets(const KArgs& a, int row, int which, 
 // The lists that the parts of a row handed over (count `which` of each part, entries from `at` of
 // its list), one after the other into dst (at most cap). Returns the number of entries.
 template <int NT>
-__device__ __forceinline__ int gen_gather(const KArgs& a, int row, int which, int at, uint64_t* dst, int cap, int* off) {
+__device__ __forceinline__ int gen_gather(const SplitArgs& a, int row, int which, int at, uint64_t* dst, int cap, int* off) {
   const int tid = threadIdx.x;
   if (tid < 64) gen_offsets(a, row, which, off);
   __syncthreads();
@@ -2439,7 +2506,8 @@ __device__ __forceinline__ bool gen_last_part(const KArgs& a, int row, int* flag
 // MIXED: a batch with per-row parameters, whose greedy and small-k rows' parts are k_topk_split's,
 // taken in the last launch, so that the batch needs no other kernel and no second stream.
 template <int NT, bool SPLIT = false, bool MIXED = false>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_general(KArgs a) {
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_general(
+    std::conditional_t<SPLIT, SplitArgs, KArgs> a) {
   constexpr int kGenThreads = NT;
   __shared__ GenShared<NT> sh;
   __shared__ int part_off[2][SPLIT ? kGenMaxParts + 1 : 1];
@@ -2717,6 +2785,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
   unsigned long long* plist = nullptr;
   auto hand_over = [&]() -> bool {
     __syncthreads();
+    if constexpr (SPLIT)
     if (tid < 2)
       __hip_atomic_store(&a.p_cnt[kGenPartCnt * (static_cast<size_t>(row) * a.P + part.part) + kGenPartListA + tid], sh.ints[tid == 0 ? 4 : 7],
                          __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -3884,12 +3953,6 @@ struct __align__(16) RowShared {
   int ints[16];
 };
 
-// Order key without branches; +0.0f turns -0 into +0 first.
-__device__ __forceinline__ uint32_t key_of(uint32_t bits) {
-  const uint32_t b = __float_as_uint(__uint_as_float(bits) + 0.0f);
-  return b ^ (static_cast<uint32_t>(static_cast<int32_t>(b) >> 31) | 0x80000000u);
-}
-
 __device__ __forceinline__ bool bit_of(const uint32_t* bits, int e) { return (bits[e >> 5] >> (e & 31)) & 1u; }
 
 
@@ -4457,7 +4520,7 @@ __global__ __launch_bounds__(kRowNT) void k_rows(KArgs a) {
   }
 }
 
-__global__ __launch_bounds__(kTkNT) void k_topk_split(KArgs a) {
+__global__ __launch_bounds__(kTkNT) __attribute__((amdgpu_waves_per_eu(4))) void k_topk_split(KArgs a) {
   __shared__ TkShared sh;
   const int row = static_cast<int>(blockIdx.x) / a.P;
   topk_part(a, sh, a.shared, row, static_cast<int>(blockIdx.x) - row * a.P);
@@ -5143,7 +5206,7 @@ void launch_rows(const KArgs& a, hipStream_t st) {
   hipLaunchKernelGGL(k_rows, dim3(a.B), dim3(kRowNT), dyn, st, a);
 }
 
-void launch_general_split(const KArgs& a, hipStream_t st) {
+void launch_general_split(const SplitArgs& a, hipStream_t st) {
   const dim3 grid(static_cast<unsigned>(a.B * a.P)), nt(kGsNT);
   hipLaunchKernelGGL(k_gen_max, grid, nt, 0, st, a);
   hipLaunchKernelGGL(k_gen_hist, grid, nt, 0, st, a);
