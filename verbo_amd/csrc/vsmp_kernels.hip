@@ -2219,21 +2219,23 @@ __device__ __forceinline__ GenPart gen_part(const KArgs& a) {
 }
 // The 16-byte groups of the part's chunk that starts at group c0, all loads in flight at once (past
 // the part: its last group, or the row's).
-__device__ __forceinline__ void gen_part_load(const float* rp, int V, const GenPart& t, int c0, float4 (&v)[kGsU]) {
+template <int U>
+__device__ __forceinline__ void gen_part_load(const float* rp, int V, const GenPart& t, int c0, float4 (&v)[U]) {
   const float4* rp4 = reinterpret_cast<const float4*>(rp);
   const int glast = (t.g1 > t.g0 ? t.g1 : (V + 3) >> 2) - 1;
 #pragma unroll
-  for (int u = 0; u < kGsU; ++u) v[u] = rp4[min(c0 + u * kGsNT + static_cast<int>(threadIdx.x), glast)];
+  for (int u = 0; u < U; ++u) v[u] = rp4[min(c0 + u * kGsNT + static_cast<int>(threadIdx.x), glast)];
 }
 // The penalty bits of the thread's groups of that chunk, four bits each. bits: the bitmap from the
 // row's start, in global memory, or (base > 0 possible) from group `base` on.
+template <int U = kGsU>
 __device__ __forceinline__ uint32_t gen_part_nibs(const uint32_t* bits, const GenPart& t, int c0, int base = 0) {
-  uint32_t w[kGsU], nibs = 0u;
+  uint32_t w[U], nibs = 0u;
   const int glast = max(t.g1 - 1, t.g0);
 #pragma unroll
-  for (int u = 0; u < kGsU; ++u) w[u] = bits[(min(c0 + u * kGsNT + static_cast<int>(threadIdx.x), glast) - base) >> 3];
+  for (int u = 0; u < U; ++u) w[u] = bits[(min(c0 + u * kGsNT + static_cast<int>(threadIdx.x), glast) - base) >> 3];
 #pragma unroll
-  for (int u = 0; u < kGsU; ++u) {
+  for (int u = 0; u < U; ++u) {
     const int f = c0 + u * kGsNT + static_cast<int>(threadIdx.x);
     nibs |= ((w[u] >> (4 * (f & 7))) & 0xFu) << (4 * u);
   }
@@ -2566,6 +2568,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
   ulonglong2 hraw[SPLIT ? kGenBuckets / NT / 2 : 1];
   int4 pcnt = {};
   double2 pmass = {};
+  double pu = 0.0;  // the draw, which k_gen_max took
   if constexpr (SPLIT) {
     static_assert(NT == kGsNT, "a part's elements are held by its threads");
     part = gen_part(a);
@@ -2580,6 +2583,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
       pcnt = *reinterpret_cast<const int4*>(&a.p_cnt[kGenPartCnt * slot]);
       pmass = *reinterpret_cast<const double2*>(&a.p_mass[2 * slot]);
     }
+    pu = a.x_u[row];
     if (tid < 8) sh.ints[tid] = tid == 0 ? kGenBuckets : 0;
     if (tid < 4) sh.fb[tid] = kGenBuckets;
     uint32_t mn;
@@ -2735,14 +2739,18 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
       em += im - ms;
       ec += ic - cs;
       int first = kGenBuckets;
+      double pm[2];  // written as 16-byte vectors: a thread's buckets are consecutive
+      uint32_t pc[4];
 #pragma unroll
       for (int i = 0; i < BP; ++i) {
         em += rm[i];
         const uint32_t n = rc[i];
         ec += n;
         rm[i] = n ? em : -1.0;  // no target is found in an empty bucket
-        sh.mass0[b0 + i] = em;
-        sh.cnt0[b0 + i] = ec;
+        pm[i & 1] = em;
+        pc[i & 3] = ec;
+        if ((i & 1) == 1) *reinterpret_cast<double2*>(&sh.mass0[b0 + i - 1]) = make_double2(pm[0], pm[1]);
+        if ((i & 3) == 3) *reinterpret_cast<uint4*>(&sh.cnt0[b0 + i - 3]) = make_uint4(pc[0], pc[1], pc[2], pc[3]);
         if (first == kGenBuckets && ec >= static_cast<uint32_t>(k)) first = b0 + i;
       }
       if (k < V) wave_claim_min(&sh.ints[0], first < kGenBuckets, first);
@@ -2762,27 +2770,65 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
       }
     }
   }
-  // f(bucket, composite) for each of this part's elements; pv, pnibs: the part's first chunk.
-  auto part_each = [&](float4 (&pv)[kGsU], uint32_t pnibs, auto&& f) {
-    for (int c0 = part.g0; c0 < part.g1; c0 += kGsChunk) {
+  // Stores this part's elements of the buckets that inA and inB take in its lists A (at most capA) and
+  // B (at most kGenCap / 2, from that place on), counted in ints[4] and ints[7]. pv, pnibs: the part's
+  // first chunk. A lane marks its elements in two masks; a wave's take their places by one scan of the
+  // packed counts and one LDS atomic per list, not one per element.
+  unsigned long long* plist = nullptr;
+  if constexpr (SPLIT) plist = a.p_list + (static_cast<size_t>(row) * a.P + part.part) * kGenPartList;
+  constexpr int LU = 4;  // 16-byte groups held at once here (8 made the kernel spill)
+  auto part_lists = [&](float4 (&pv)[LU], uint32_t pnibs, int capA, auto&& inA, auto&& inB) {
+    for (int c0 = part.g0; c0 < part.g1; c0 += LU * kGsNT) {
       if (c0 != part.g0) {
         gen_part_load(g.R.rp, V, part, c0, pv);
-        pnibs = g.R.pen ? gen_part_nibs(g.R.bits, part, c0) : 0u;
+        pnibs = g.R.pen ? gen_part_nibs<LU>(g.R.bits, part, c0) : 0u;
       }
+      uint32_t hA = 0u, hB = 0u;
 #pragma unroll
-      for (int u = 0; u < kGsU; ++u) {
-        const int e = 4 * (c0 + u * kGenThreads + tid);
-        if (e >= part.hi) continue;
+      for (int u = 0; u < LU; ++u) {
+        const int n = part.hi - 4 * (c0 + u * kGenThreads + tid);  // the group's elements inside the part
         float x[4] = {pv[u].x, pv[u].y, pv[u].z, pv[u].w};
         gen_part_penalise(g.R, (pnibs >> (4 * u)) & 0xFu, x);
+        pv[u] = make_float4(x[0], x[1], x[2], x[3]);
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (e + i < V) f(q_of(g, x[i]), comp(ord_key(x[i]), static_cast<uint32_t>(e + i)));
+        for (int i = 0; i < 4; ++i) {
+          const int q = q_of(g, x[i]);
+          hA |= static_cast<uint32_t>(i < n && inA(q)) << (4 * u + i);
+          hB |= static_cast<uint32_t>(i < n && inB(q)) << (4 * u + i);
+        }
+      }
+      static_assert(4 * LU <= 32, "one mask bit per element");
+      if (__ballot((hA | hB) != 0u) == 0ull) continue;
+      const uint32_t mine = __popc(hA) | __popc(hB) << 16, incl = wave_incl_scan(mine);
+      int bA = 0, bB = 0;
+      if ((tid & 63) == 63) {
+        if (incl & 0xFFFFu) bA = atomicAdd(&sh.ints[4], static_cast<int>(incl & 0xFFFFu));
+        if (incl >> 16) bB = atomicAdd(&sh.ints[7], static_cast<int>(incl >> 16));
+      }
+      int pA = __builtin_amdgcn_readlane(bA, 63) + static_cast<int>((incl - mine) & 0xFFFFu);
+      int pB = __builtin_amdgcn_readlane(bB, 63) + static_cast<int>((incl - mine) >> 16);
+#pragma unroll
+      for (int u = 0; u < LU; ++u) {
+        if ((((hA | hB) >> (4 * u)) & 0xFu) == 0u) continue;
+        const float x[4] = {pv[u].x, pv[u].y, pv[u].z, pv[u].w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          if (((hA | hB) >> (4 * u + i)) & 1u) {
+            const unsigned long long ck = comp(ord_key(x[i]), static_cast<uint32_t>(4 * (c0 + u * kGenThreads + tid) + i));
+            if ((hA >> (4 * u + i)) & 1u) {
+              if (pA < capA) __hip_atomic_store(&plist[pA], ck, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+              ++pA;
+            }
+            if ((hB >> (4 * u + i)) & 1u) {
+              if (pB < kGenCap / 2) __hip_atomic_store(&plist[kGenCap / 2 + pB], ck, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+              ++pB;
+            }
+          }
+        }
       }
     }
   };
   // hands this part's two lists over; false: another part ends the row
-  unsigned long long* plist = nullptr;
   auto hand_over = [&]() -> bool {
     __syncthreads();
     if constexpr (SPLIT)
@@ -2791,11 +2837,6 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
                          __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     return gen_last_part(a, row, &sh.ints[6]);
   };
-  auto append = [&](int* n, int at, int cap, uint64_t ck) {
-    const int p = atomicAdd(n, 1);
-    if (p < cap) __hip_atomic_store(&plist[at + p], static_cast<unsigned long long>(ck), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  };
-  if constexpr (SPLIT) plist = a.p_list + (static_cast<size_t>(row) * a.P + part.part) * kGenPartList;
   if (alone && k < V) {
     auto all_v = [](float) { return true; };
     auto all_c = [](uint64_t) { return true; };
@@ -3114,7 +3155,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
   // usual case below, the top-p cut and the draw share one pass over the row.
   if (!SPLIT && tid == 0) sh.dbls[1] = draw_u(a, row, P);
   if (!SPLIT) __syncthreads();
-  const double u = SPLIT ? a.x_u[row] : sgpr_f64(sh.dbls[1]);  // SPLIT: k_gen_max drew it
+  const double u = SPLIT ? sgpr_f64(pu) : sgpr_f64(sh.dbls[1]);
   const bool topp = P.top_p > 0.0f && P.top_p < 1.0f;
   const double tp = static_cast<double>(P.top_p);
   const double near_tp = near_topp(k);
@@ -3145,11 +3186,10 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
       // parts and put in order by the last one (each bucket's entries at its count prefix, then
       // ranked within the bucket), in the histogram's mass array, read no more. The sum, the cuts and
       // the draw are taken on the sorted list.
-      float4 pv[kGsU];
+      float4 pv[LU];
       gen_part_load(g.R.rp, V, part, part.g0, pv);
-      part_each(pv, g.R.pen ? gen_part_nibs(g.R.bits, part, part.g0) : 0u, [&](int q, uint64_t ck) {
-        if (q <= qk) append(&sh.ints[4], 0, kGenPartList, ck);
-      });
+      part_lists(pv, g.R.pen && part.hi > part.lo ? gen_part_nibs<LU>(g.R.bits, part, part.g0) : 0u, kGenPartList,
+                 [qk](int q) { return q <= qk; }, [](int) { return false; });
       if (!hand_over()) return;
       alone = true;
       uint64_t* big = reinterpret_cast<uint64_t*>(sh.mass0);            // kGenPartList entries
@@ -3201,9 +3241,9 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
       constexpr int LC = kGenCap / 2;
       static_assert(LC == NT, "one entry of each list per thread");
       const int lane = tid & 63, w = tid >> 6;
-      float4 pv[kGsU];
+      float4 pv[LU];
       gen_part_load(g.R.rp, V, part, part.g0, pv);
-      const uint32_t pnibs = g.R.pen && part.hi > part.lo ? gen_part_nibs(g.R.bits, part, part.g0) : 0u;
+      const uint32_t pnibs = g.R.pen && part.hi > part.lo ? gen_part_nibs<LU>(g.R.bits, part, part.g0) : 0u;
       auto first_bucket = [&](double t) {
         int f = kGenBuckets;
 #pragma unroll
@@ -3260,10 +3300,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
         else
           __syncthreads();
       } else {
-        part_each(pv, pnibs, [&](int q, uint64_t ck) {
-          if (q == qp) append(&sh.ints[4], 0, LC, ck);
-          if (q >= d_lo && q <= d_hi) append(&sh.ints[7], LC, LC, ck);
-        });
+        part_lists(pv, pnibs, LC, [qp](int q) { return q == qp; }, [d_lo, d_hi](int q) { return q >= d_lo && q <= d_hi; });
         if (!hand_over()) return;
         alone = true;
         uint64_t* listA = sh.list;
@@ -3275,12 +3312,31 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
         if (tid < 2) sh.ints[tid] = LC;
         __syncthreads();
         const int mA = min(sgpr_i32(part_off[0][64]), LC), mB = min(sgpr_i32(part_off[1][64]), LC);
-        const uint64_t xA = tid < mA ? gen_entry(a, row, 0, part_off[0], tid) : 0ull;
-        const uint64_t xB = tid < mB ? gen_entry(a, row, LC, part_off[1], tid) : 0ull;
-        listA[tid] = xA;
-        listB[tid] = xB;
-        __syncthreads();
-        if (max(mA, mB) <= kGenRankMax) {
+        // Lists that half the threads hold are ranked side by side, longer ones one after the other
+        // (counting all 512 is still faster than a bitonic sort's 45 barriers).
+        const double above_d = d_lo > 0 ? sgpr_f64(sh.mass0[d_lo - 1]) : 0.0;
+        const bool second = tid >= NT / 2;
+        if (max(mA, mB) <= NT / 2) {
+          uint64_t* list = second ? listB : listA;
+          double* lpr = second ? lprB : lprA;
+          const int m = second ? mB : mA, i = tid & (NT / 2 - 1);
+          const uint64_t x = i < m ? gen_entry(a, row, second ? LC : 0, part_off[second ? 1 : 0], i) : 0ull;
+          list[i] = x;
+          __syncthreads();
+          int r = 0;
+          if (i < m) r = rank_count(list, m, x);
+          const double wt = numer_g(g, comp_val(x));
+          __syncthreads();
+          if (i < m) {
+            list[r] = x;
+            lpr[r] = wt;
+          }
+        } else {
+          const uint64_t xA = tid < mA ? gen_entry(a, row, 0, part_off[0], tid) : 0ull;
+          const uint64_t xB = tid < mB ? gen_entry(a, row, LC, part_off[1], tid) : 0ull;
+          listA[tid] = xA;
+          listB[tid] = xB;
+          __syncthreads();
           int rA = 0, rB = 0;
           if (tid < mA) rA = rank_count(listA, mA, xA);
           if (tid < mB) rB = rank_count(listB, mB, xB);
@@ -3294,15 +3350,9 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
             listB[rB] = xB;
             lprB[rB] = wB;
           }
-        } else {
-          bitonic_desc<NT>(listA, LC);
-          bitonic_desc<NT>(listB, LC);
-          lprA[tid] = numer_g(g, comp_val(listA[tid]));
-          lprB[tid] = numer_g(g, comp_val(listB[tid]));
         }
         __syncthreads();
         // running sums through both lists, and the first entry of each that reaches its target
-        const double above_d = d_lo > 0 ? sgpr_f64(sh.mass0[d_lo - 1]) : 0.0;
         double iA = wave_incl_scan_f64(tid < mA ? lprA[tid] : 0.0);
         double iB = wave_incl_scan_f64(tid < mB ? lprB[tid] : 0.0);
         if (lane == 63) {
@@ -3753,6 +3803,9 @@ __global__ __launch_bounds__(kGenThreads) void k_general_exact(KArgs a) {
   __shared__ int xi[4];
   __shared__ uint32_t xk[2];  // the row's smallest and largest penalised order key
   __shared__ __align__(16) uint64_t blk[kXBlock];  // sort blocks; staged chunks of the chains
+  // A workgroup with one row leaves on that row's mark: most calls mark none, and their launch should
+  // cost no more than it must.
+  if (gridDim.x >= static_cast<unsigned>(a.B) && a.x_flag[blockIdx.x] == 0) return;
   double* stage = reinterpret_cast<double*>(blk);
   const int tid = threadIdx.x;
   const int V = a.V, n2 = a.x_n;
