@@ -829,3 +829,40 @@ def test_general_split_parts(monkeypatch, parts, Vv):
         states.append(st.cpu())
         ids.append(torch.stack(out))
     assert torch.equal(states[0], states[1]) and torch.equal(ids[0], ids[1])
+
+
+def test_graph_capture_after_a_larger_warm_up():
+    """The split kernels' scratch is sized by any call at a shape or a larger one: after one call of a
+    wide batch on another path, smaller batches of every split path are captured and replayed."""
+    import torch
+
+    ctx = V.Context(0)
+    Vv = 49152
+    g = torch.Generator(device="cuda").manual_seed(3)
+    big = torch.randn(96, Vv, generator=g, device="cuda")
+    off = V.Params(temp=1.0, top_k=2000, top_p=0.9, min_p=0.0, repeat=1.0, repeat_last=0, seed=4)  # one workgroup per row
+    ctx.pick_batch(big, off)
+    torch.cuda.synchronize()
+    cases = [(24, dict(temp=0.8, top_k=40, top_p=0.9)), (1, dict(temp=0.8, top_k=64, top_p=0.95)), (32, dict(temp=1.0, top_k=0, top_p=0.95)),
+             (3, dict(temp=1.0, top_k=700, top_p=0.9, min_p=0.01)), (16, dict(temp=0.0, top_k=0, top_p=1.0)), (48, dict(temp=0.9, top_k=0, top_p=0.9))]
+    for B, f in cases:
+        pr = V.Params(**{"min_p": 0.0, "repeat": 1.0, "repeat_last": 0, "seed": 11, **f})
+        if B == 48:  # per-row parameters beyond the split: k_rows, and k_general on the forked stream
+            rows = V.params_array(n=B, temp=0.9, top_k=40, top_p=0.9, repeat=1.0, repeat_last=0, seed=1)
+            rows["top_k"][::3] = 0
+            pr = V.to_device_params(rows)
+        x = torch.randn(B, Vv, generator=g, device="cuda")
+        out = torch.empty(B, dtype=torch.int32, device="cuda")
+        torch.cuda.synchronize()
+        st, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+        with torch.cuda.stream(st):
+            with torch.cuda.graph(graph, stream=st):
+                ctx.pick_batch(x, pr, out=out, stream=st)
+        torch.cuda.synchronize()
+        for step in range(3):
+            log("capture after a larger warm-up", B, f, step)
+            x.copy_(torch.randn(B, Vv, generator=g, device="cuda"))
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, mode_ctx("rows").pick_batch(x, pr)), (B, f, step)

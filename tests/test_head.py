@@ -18,8 +18,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.fixture(params=["auto", "fused"])
 def ctx(request):
-    """vsmp_head_pick's route by batch size (fused for 16 to 64 rows, the head's logits written and
-    the batched pick otherwise), and the fused route pinned for every batch."""
+    """vsmp_head_pick's own route by shape (fused, or the head's logits written and the batched pick),
+    and the fused route pinned for every batch."""
     import torch
 
     assert torch.cuda.is_available(), "the gpu tests need a ROCm device"

@@ -234,12 +234,13 @@ int topk_parts(int B, int V, int cus, int k, bool forced, long long forced_p) {
 
 // Parts per general row of a small batch. 0: one workgroup per row. A part costs the histogram's
 // global atomics (up to 4,096 whatever its elements) and its own elements, so the best number falls as
-// the square root of the batch: measured (top-k off, top-p .95) 48, 24, 10, 8 and 6 parts at 1, 4, 16,
-// 32 and 64 rows of 151,936, 28, 16, 6 and 5 at 1, 4, 16 and 32 of 49,152, which sqrt(V / (64 B))
-// meets. Against one workgroup per row, whose time hardly grows with the batch: 151,936 logits 1 row
-// 30.2 against 69.4 us, 16 rows 42.6 / 74.1, 64 rows 66.3 / 79.8, 128 rows 89.4 / 83.0; 49,152 logits
-// 1 row 27.9 / 38.5, 32 rows 36.8 / 40.7, 64 rows 43.3 / 40.8. The line between lies near B = V / 1600;
-// the split is taken to V / 2000.
+// the square root of the batch: measured (top-k off, top-p .95, nearly flat rows) 48, 24, 10, 8 and 6-8
+// parts at 1, 4, 16, 32 and 64 rows of 151,936, 24, 16, 6 and 6 at 1, 4, 16 and 32 of 49,152, which
+// sqrt(V / (64 B)) meets. Against one workgroup per row, whose time hardly grows with the batch:
+// 151,936 logits 1 row 28.1 against 69.2 us, 16 rows 39.8 / 72.7, 64 rows 63.0 / 78.8, 128 rows 85.0 /
+// 82.8; 49,152 logits 1 row 26.3 / 37.6, 32 rows 34.0 / 39.1, 64 rows 40.2 / 39.2. The line between
+// lies near B = V / 1200; the split is taken to V / kGenSplitLogits.
+constexpr int kGenSplitLogits = 1500;
 // per_row: the greedy and small-k rows among them are cut into the same parts (k_topk_split's, so
 // register-held ones, at most 16), and a batch that cannot be takes no split.
 GenParts general_parts(int B, int V, bool per_row, bool forced, long long forced_p) {
@@ -254,7 +255,7 @@ GenParts general_parts(int B, int V, bool per_row, bool forced, long long forced
   if (per_row && tmin > tmax) P = 0;
   if (per_row && P > 0) P = std::min(std::max(P, tmin), tmax);
   if (forced) return {static_cast<int>(P), static_cast<size_t>(B), static_cast<size_t>(B * P)};
-  const long long rows = std::min<long long>(B, V / 2000);
+  const long long rows = std::min<long long>(B, V / kGenSplitLogits);
   if (rows < 1 || pmax < 2) return {};
   const long long slots = std::max({rows * std::max(pmin, std::min(tmin, tmax)), rows * P, static_cast<long long>(std::sqrt(rows * (V / 64.0)) + 0.5 * rows) + 1});
   return {rows == B && P >= 2 ? static_cast<int>(P) : 0, static_cast<size_t>(rows), static_cast<size_t>(slots)};
@@ -448,6 +449,16 @@ KArgs batch_args(const float* logits, int B, int V, long long ld, const vsmp_par
   return a;
 }
 
+// The split kernels' scratch. Which batches they take depends on k as well as on the shape, so every
+// call sizes it for whatever split the device can be given by default (about 1 MiB): a call at a shape,
+// with any parameters, then serves a graph capture at that shape or a smaller one. rows, slots: what a
+// call itself needs beyond that (pinned modes).
+bool split_rows_scratch(vsmp_ctx* ctx, size_t rows, size_t slots, hipStream_t st) {
+  const size_t most = 2 * static_cast<size_t>(ctx->cus);
+  return grow(ctx->g_rows, ctx->n_grows, 2 * std::max(rows, most), true, "scratch", st) &&
+         grow(ctx->t_scr, ctx->n_tscr, std::max(slots, most) * (kKmax + 1), false, "scratch", st);
+}
+
 int launch_batch(vsmp_ctx* ctx, const float* logits, int B, int V, long long ld, const vsmp_params* params,
                  int params_per_row, const int* hist, const int* hist_off, int u_mode, const double* u,
                  unsigned long long* rng_state, unsigned long long counter, int* out, const vsmp_debug* dbg,
@@ -460,6 +471,7 @@ int launch_batch(vsmp_ctx* ctx, const float* logits, int B, int V, long long ld,
   if (slots > static_cast<size_t>(INT32_MAX) / kKmax) return set_error("vsmp: batch too large");
   const int words = a.words;
   const bool slices = !pl.rows && !pl.split;
+  if (!slices && !split_rows_scratch(ctx, pl.split ? static_cast<size_t>(B) : 0, pl.split && pl.topk ? slots : 0, st)) return -1;
   if (slices && (!grow(ctx->s_cnt, ctx->n_cnt, slots, false, "scratch", st) ||
                  !grow(ctx->s_npen, ctx->n_npen, slots, false, "scratch", st) ||
                  !grow(ctx->s_max, ctx->n_max, slots, false, "scratch", st) ||
@@ -504,14 +516,12 @@ int launch_batch(vsmp_ctx* ctx, const float* logits, int B, int V, long long ld,
   if (pl.split) {
     // per row, zero between calls, at the allocation's own capacity (a later, wider batch finds the
     // words that it takes for its own untouched): slot, ticket, penalised-id count
-    if (!grow(ctx->g_rows, ctx->n_grows, 2 * static_cast<size_t>(B), true, "scratch", st)) return -1;
     const size_t cap = ctx->n_grows / 2;
     a.P = pl.P;
     a.g_slot = ctx->g_rows;
     a.g_tick = reinterpret_cast<unsigned int*>(ctx->g_rows + cap);
     a.g_npen = a.g_tick + cap;
     if (pl.topk) {  // the parts' lists, then their counts and penalised-id counts, written before they are read
-      if (!grow(ctx->t_scr, ctx->n_tscr, slots * (kKmax + 1), false, "scratch", st)) return -1;
       a.s_cand = ctx->t_scr;
       a.s_cnt = reinterpret_cast<int*>(ctx->t_scr + slots * kKmax);
       a.s_npen = a.s_cnt + slots;
@@ -671,15 +681,21 @@ int head_pick(vsmp_ctx* ctx, const void* hidden, long long ldh, const void* head
   if (cand_cap > kGenCap) return set_error("vsmp: cand_cap is at most " + std::to_string(kGenCap));
 
   const bool shared_general = !params_per_row && path_host(*params, V, true) == kPathGeneral;
-  // The route. Fused, the call pays fixed stages (the probe's product, the bound, the finish: 25-31
-  // us at 151,936 x 896) against the logits it does not write and the sampler's read of them it
-  // saves; measured on MI355X (top-k 50, bf16 head of 151,936 x 896) that wins for batches of 16 to
-  // 64 rows (64 rows: 80.5 against 88.3 us; 16 rows: 71.3 against 73.0 us) and loses outside (1 row:
-  // 66.6 against 62.8 us, a tie at 12; 80 rows: 110.0 against 106.4 us; 256 rows: 157.4 against
-  // 150.0 us). Whole, the head's logits are written and the batched pick runs on them: the same ids
-  // and diagnostics, as the fused route is built to give.
-  constexpr int kHeadFuseMin = 16, kHeadFuseMax = 64;
-  const bool fused = ctx->head_route == 1 || (ctx->head_route < 0 && B >= kHeadFuseMin && B <= kHeadFuseMax);
+  // The route. Fused, the call pays fixed stages (the probe's product, the bound, the finish: about 25
+  // us) against the logits it does not write and the sampler's read of them it saves; whole, the
+  // head's logits are written and the batched pick runs on them: the same ids and diagnostics, as the
+  // fused route is built to give. Measured (fused / whole, us, D = 896, top-k 20, 64 and 100, shared
+  // parameters): 151,936 columns 24 rows 74.2 / 69.9, 76.1 / 75.4, 81.0 / 79.3; 32 rows 75.0 / 73.6, 77.0
+  // / 78.5, 81.7 / 83.2; 64 rows 81.0 / 85.6, 83.0 / 89.0, 88.7 / 93.1; 96 rows at top-k 50 106.4 / 102.9;
+  // 110,000 columns 16 to 64 rows 62.6 to 74.5 / 52.3 to 73.5, and whole further ahead on fewer (50,257:
+  // 42.5 to 51.6 / 32.0 to 43.7). So fused for 31 to 64 rows of 151,936 columns and in proportion, not
+  // below 120,000. It does not depend on k, so that a call at a shape sizes its scratch. With per-row
+  // parameters (some rows general or not) it is taken for 16 to 64 rows.
+  constexpr int kHeadFuseMin = 16, kHeadFuseMax = 64, kHeadFuseV = 120000;
+  constexpr long long kHeadFuseLogits = 4600000;
+  const bool fuse_shape = B >= kHeadFuseMin && B <= kHeadFuseMax &&
+                          (params_per_row || (V >= kHeadFuseV && static_cast<long long>(B) * V >= kHeadFuseLogits));
+  const bool fused = ctx->head_route == 1 || (ctx->head_route < 0 && fuse_shape);
   const bool whole = shared_general || !fused;
   // logits written whole: the caller's, or (general rows possible, none kept by the caller) scratch
   float* full = logits;
@@ -703,6 +719,13 @@ int head_pick(vsmp_ctx* ctx, const void* hidden, long long ldh, const void* head
   }
   const int n0 = std::min(kHeadProbe, V);
   const int tile = head_tile(B, false);
+  // fewer rows of this head take the other route: its logits and the pick's scratch, sized here too
+  if (!params_per_row && ctx->head_route < 0) {
+    const size_t rows = static_cast<size_t>(kHeadFuseLogits / V);
+    if (!grow(ctx->h_full, ctx->n_full, rows * static_cast<size_t>((V + 3) & ~3), false, "head scratch", st) ||
+        !split_rows_scratch(ctx, 0, 0, st))
+      return -1;
+  }
   if (!grow(ctx->h_tk, ctx->n_tk, static_cast<size_t>(B), false, "head scratch", st) ||
       !grow(ctx->h_rmode, ctx->n_rmode, static_cast<size_t>(B), false, "head scratch", st) ||
       !grow(ctx->h_rcand, ctx->n_rcand, static_cast<size_t>(B) * static_cast<size_t>(V), false, "head scratch", st) ||

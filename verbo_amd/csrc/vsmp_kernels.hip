@@ -2094,41 +2094,41 @@ __device__ __forceinline__ void topk_part(const KArgs& a, TkShared& sh, const vs
         if ((hit >> (4 * u + c)) & 1u) sh.top[place++] = comp(kk[c], static_cast<uint32_t>(4 * (g0 + u * kTkNT + tid) + c));
     }
   } else {
-  uint64_t clo = static_cast<uint64_t>(T) << 32;
-  uint64_t chi = block_max64<kTkNT>((static_cast<uint64_t>(lm) << 32) | 0xFFFFFFFFull, sh.red64);  // at or above every key
-  if (tid == 0) sh.ints[8] = 0;
-  int need = ks;
-  for (int pass = 0; clo != chi && pass < 9; ++pass) {
-    const uint64_t R = chi - clo;
-    const int sft = R < static_cast<uint64_t>(kRowBins) ? 0 : 53 - __clzll(static_cast<long long>(R));
-    uint32_t* bins = sh.bins[pass & 1];
-    for (int i = tid; i < kRowBins; i += kTkNT) sh.bins[(pass + 1) & 1][i] = 0u;
+    uint64_t clo = static_cast<uint64_t>(T) << 32;
+    uint64_t chi = block_max64<kTkNT>((static_cast<uint64_t>(lm) << 32) | 0xFFFFFFFFull, sh.red64);  // at or above every key
+    if (tid == 0) sh.ints[8] = 0;
+    int need = ks;
+    for (int pass = 0; clo != chi && pass < 9; ++pass) {
+      const uint64_t R = chi - clo;
+      const int sft = R < static_cast<uint64_t>(kRowBins) ? 0 : 53 - __clzll(static_cast<long long>(R));
+      uint32_t* bins = sh.bins[pass & 1];
+      for (int i = tid; i < kRowBins; i += kTkNT) sh.bins[(pass + 1) & 1][i] = 0u;
 #pragma unroll
-    for (int u = 0; u < kTkU; ++u) {
-      const uint32_t kk[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
-      const int e = 4 * (g0 + u * kTkNT + tid);
+      for (int u = 0; u < kTkU; ++u) {
+        const uint32_t kk[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
+        const int e = 4 * (g0 + u * kTkNT + tid);
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        if (kk[c] < T || kk[c] == 0u) continue;
-        const uint64_t cc = comp(kk[c], static_cast<uint32_t>(e + c));
-        if (cc >= clo && cc <= chi) atomicAdd(&bins[(cc - clo) >> sft], 1u);
+        for (int c = 0; c < 4; ++c) {
+          if (kk[c] < T || kk[c] == 0u) continue;
+          const uint64_t cc = comp(kk[c], static_cast<uint32_t>(e + c));
+          if (cc >= clo && cc <= chi) atomicAdd(&bins[(cc - clo) >> sft], 1u);
+        }
       }
+      __syncthreads();
+      if (w == 0) wave_find_bucket(bins, need, sh.ints);
+      __syncthreads();
+      const int b = sh.ints[0];
+      const int inb = sh.ints[2];
+      need -= sh.ints[1];
+      __syncthreads();
+      if (b < 0) break;  // unreachable: ks composites lie at or above T << 32
+      const uint64_t nlo = clo + (static_cast<uint64_t>(b) << sft);
+      const uint64_t wdt = sft == 0 ? 0ull : (1ull << sft) - 1ull;
+      chi = (chi - nlo < wdt) ? chi : nlo + wdt;
+      clo = nlo;
+      if (inb == need) chi = clo;  // the whole bucket is taken: the top ks are the composites >= clo
     }
-    __syncthreads();
-    if (w == 0) wave_find_bucket(bins, need, sh.ints);
-    __syncthreads();
-    const int b = sh.ints[0];
-    const int inb = sh.ints[2];
-    need -= sh.ints[1];
-    __syncthreads();
-    if (b < 0) break;  // unreachable: ks composites lie at or above T << 32
-    const uint64_t nlo = clo + (static_cast<uint64_t>(b) << sft);
-    const uint64_t wdt = sft == 0 ? 0ull : (1ull << sft) - 1ull;
-    chi = (chi - nlo < wdt) ? chi : nlo + wdt;
-    clo = nlo;
-    if (inb == need) chi = clo;  // the whole bucket is taken: the top ks are the composites >= clo
-  }
-  collect(clo);
+    collect(clo);
   }
   if (tid < kKmax) sh.rank[tid] = 0;
   __syncthreads();
@@ -2831,10 +2831,12 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
   // hands this part's two lists over; false: another part ends the row
   auto hand_over = [&]() -> bool {
     __syncthreads();
-    if constexpr (SPLIT)
-    if (tid < 2)
-      __hip_atomic_store(&a.p_cnt[kGenPartCnt * (static_cast<size_t>(row) * a.P + part.part) + kGenPartListA + tid], sh.ints[tid == 0 ? 4 : 7],
-                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if constexpr (SPLIT) {
+      if (tid < 2) {
+        int* counts = a.p_cnt + kGenPartCnt * (static_cast<size_t>(row) * a.P + part.part) + kGenPartListA;
+        __hip_atomic_store(&counts[tid], sh.ints[tid == 0 ? 4 : 7], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+    }
     return gen_last_part(a, row, &sh.ints[6]);
   };
   if (alone && k < V) {
@@ -2849,17 +2851,19 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
   // relative to the table points, numer_fix, in the mass array's 8-byte slots until the prefix
   // below turns them into fp64 masses)
   uint64_t* fix0 = reinterpret_cast<uint64_t*>(sh.mass0);
-  if (alone)
-  for (int i = tid; i < kGenBuckets; i += kGenThreads) {
-    sh.cnt0[i] = 0u;
-    fix0[i] = 0ull;
+  if (alone) {
+    for (int i = tid; i < kGenBuckets; i += kGenThreads) {
+      sh.cnt0[i] = 0u;
+      fix0[i] = 0ull;
+    }
   }
   // the main pass's table (numer_tab), in the refinement histograms, which are free until the
   // prefix below has used it
   double* etab = sh.rmass;
   const double wq = table_width(g.qs, P.temp);
-  if (alone)
-  for (int j = tid; j < kGenBuckets / 2; j += kGenThreads) etab[j] = exp_tab(-static_cast<double>(2 * j + 1) * wq);
+  if (alone) {
+    for (int j = tid; j < kGenBuckets / 2; j += kGenThreads) etab[j] = exp_tab(-static_cast<double>(2 * j + 1) * wq);
+  }
   const FixCoef fc = fix_coef(wq, P.temp, g.inv_temp);
   // The main pass also collects the min-p prefix (its elements' exact numerators are taken there)
   // into the list, which aliases the refinement counts, idle until the pass ends.
@@ -5042,6 +5046,19 @@ __global__ __launch_bounds__(kHfNT) void k_head_finish(KArgs a, HeadArgs h) {
   const bool pen = (P.repeat != 1.0f) && H > 0;
   const int hfrom = h0 + ((P.repeat_last > 0 && H > P.repeat_last) ? H - P.repeat_last : 0);
   const int words = (V + 31) >> 5;
+  // the row's candidates: its list holds n of them (the probe's, then the main product's); the first
+  // round's and the draw are asked for ahead of the bitmap
+  const int n = static_cast<int>(min(static_cast<long long>(h.rcnt[row]), h.rcap));
+  const uint64_t* list = reinterpret_cast<const uint64_t*>(h.rcand) + static_cast<long long>(row) * h.rcap;
+  constexpr int PF = (kHeadRound + kHfNT - 1) / kHfNT;  // a round's loads per thread, all in flight
+  uint64_t v0[PF];
+#pragma unroll
+  for (int u = 0; u < PF; ++u) {
+    const int i = u * kHfNT + tid;
+    v0[u] = i < min(n, kHeadRound) ? list[i] : 0ull;
+  }
+  double u0 = 0.0;
+  if (tid == 0 && path == kPathSmallK) u0 = draw_u(a, row, P);
   uint32_t np = 0;
   if (pen) {  // src/sampler.cpp:53-65
     for (int i = tid; i < words; i += kHfNT) bits[i] = 0u;
@@ -5051,13 +5068,11 @@ __global__ __launch_bounds__(kHfNT) void k_head_finish(KArgs a, HeadArgs h) {
       if (id >= 0 && id < V) atomicOr(&bits[id >> 5], 1u << (id & 31));
     }
     __syncthreads();
-    for (int i = tid; i < words; i += kHfNT) np += __popc(bits[i]);
+    if (a.info)
+      for (int i = tid; i < words; i += kHfNT) np += __popc(bits[i]);
     if (a.pen_bits) store_pen_words<kHfNT>(a, row, 0, bits, words);
   }
-  const int n_pen = static_cast<int>(block_sum_u32<kHfNT>(np, red32));
-  // the row's candidates: its list holds n of them (the probe's, then the main product's)
-  const int n = static_cast<int>(min(static_cast<long long>(h.rcnt[row]), h.rcap));
-  const uint64_t* list = reinterpret_cast<const uint64_t*>(h.rcand) + static_cast<long long>(row) * h.rcap;
+  const int n_pen = a.info ? static_cast<int>(block_sum_u32<kHfNT>(np, red32)) : 0;
 
   if (path == kPathGreedy) {  // src/sampler.cpp:66-70: the first maximum
     uint64_t b = 0ull;
@@ -5101,19 +5116,16 @@ __global__ __launch_bounds__(kHfNT) void k_head_finish(KArgs a, HeadArgs h) {
     const int end = min(n, base + kHeadRound);
     if (tid == 0) sint[3] = 0;
     __syncthreads();
-    for (int i0 = base; i0 < end; i0 += kHfNT * kHfPF) {  // kHfPF loads in flight per thread
-      uint64_t v[kHfPF];
 #pragma unroll
-      for (int u = 0; u < kHfPF; ++u) {
-        const int i = i0 + u * kHfNT + tid;
-        v[u] = i < end ? list[i] : 0ull;
-      }
+    for (int u = 0; u < PF; ++u) {
+      const int i = base + u * kHfNT + tid;
+      if (base > 0) v0[u] = i < end ? list[i] : 0ull;
+    }
 #pragma unroll
-      for (int u = 0; u < kHfPF; ++u) {
-        if (i0 + u * kHfNT + tid >= end) continue;
-        const uint64_t x = head_pen(v[u], pen, bits, P.repeat);
-        if (x > bound) buf[have + atomicAdd(&sint[3], 1)] = x;
-      }
+    for (int u = 0; u < PF; ++u) {
+      if (base + u * kHfNT + tid >= end) continue;
+      const uint64_t x = head_pen(v0[u], pen, bits, P.repeat);
+      if (x > bound) buf[have + atomicAdd(&sint[3], 1)] = x;
     }
     __syncthreads();
     const int m = have + sint[3];
@@ -5136,16 +5148,14 @@ __global__ __launch_bounds__(kHfNT) void k_head_finish(KArgs a, HeadArgs h) {
   __syncthreads();
   // -- src/sampler.cpp:79-108 on the sorted top-k (kk == k: the probe alone holds k candidates)
   if (tid < 64) {
-    double u = 0.0;
-    if (tid == 0) u = draw_u(a, row, P);
     double* spr = reinterpret_cast<double*>(buf) + kEpiWs;
     const float mx = comp_val(top[0]);
     for (int i = tid; i < kk; i += 64) spr[i] = numer(comp_val(top[i]), mx, P.temp);
     wave_lds_sync();
     if (kk <= 64)
-      epilogue_wave<1>(a, row, P, top, spr, kk, n_pen, 0, readlane_f64(u, 0), reinterpret_cast<double*>(buf));
+      epilogue_wave<1>(a, row, P, top, spr, kk, n_pen, 0, readlane_f64(u0, 0), reinterpret_cast<double*>(buf));
     else
-      epilogue_wave<kEpiJ>(a, row, P, top, spr, kk, n_pen, 0, readlane_f64(u, 0), reinterpret_cast<double*>(buf));
+      epilogue_wave<kEpiJ>(a, row, P, top, spr, kk, n_pen, 0, readlane_f64(u0, 0), reinterpret_cast<double*>(buf));
   }
 }
 
