@@ -241,6 +241,12 @@ int topk_parts(int B, int V, int cus, int k, bool forced, long long forced_p) {
 // 82.8; 49,152 logits 1 row 26.3 / 37.6, 32 rows 34.0 / 39.1, 64 rows 40.2 / 39.2. The line between
 // lies near B = V / 1200; the split is taken to V / kGenSplitLogits.
 constexpr int kGenSplitLogits = 1500;
+// Per-row parameters (against k_rows beside k_general, us; rows all top-k 40 / all top-p / half of each):
+// 24 rows of 50,257 18.8 / 38.6, 32.8 / 62.7, 31.4 / 62.3; 64 of 151,936 (640 parts) 30.2 / 39.0, 73.7 / 94.5,
+// 56.1 / 94.2; 100 of 151,936 38.9 / 38.6, 95.1 / 95.3, 75.6 / 94.7; 100 of 262,144 (1,600 parts) 65.0 /
+// 41.3, 147.2 / 128.8, 120.7 / 128.1. Rows with k of 200 (lists overflow) or above 1,024 (one workgroup)
+// are the split's worst: 46-59 / 39-41 and 100-203 / 105-174 up to 33 rows.
+constexpr long long kMixedParts = 640;
 // per_row: the greedy and small-k rows among them are cut into the same parts (k_topk_split's, so
 // register-held ones, at most 16), and a batch that cannot be takes no split.
 GenParts general_parts(int B, int V, bool per_row, bool forced, long long forced_p) {
@@ -258,7 +264,8 @@ GenParts general_parts(int B, int V, bool per_row, bool forced, long long forced
   const long long rows = std::min<long long>(B, V / kGenSplitLogits);
   if (rows < 1 || pmax < 2) return {};
   const long long slots = std::max({rows * std::max(pmin, std::min(tmin, tmax)), rows * P, static_cast<long long>(std::sqrt(rows * (V / 64.0)) + 0.5 * rows) + 1});
-  return {rows == B && P >= 2 ? static_cast<int>(P) : 0, static_cast<size_t>(rows), static_cast<size_t>(slots)};
+  const bool fits = !per_row || B * P <= kMixedParts;
+  return {rows == B && P >= 2 && fits ? static_cast<int>(P) : 0, static_cast<size_t>(rows), static_cast<size_t>(slots)};
 }
 
 // Where the split general rows' scratch lies in its allocation, 16-byte aligned.
