@@ -710,6 +710,54 @@ def test_topk_split_parts(dmode):
         assert (dst.cpu().numpy().view(np.uint64) == st).all()
 
 
+@pytest.mark.parametrize("parts", [4, 9, 16])
+@pytest.mark.parametrize("per_row", [False, True])
+def test_topk_split_lists(monkeypatch, parts, per_row):
+    """Small-k and greedy rows cut into parts whose lists hold more than k keys: k up to 256, where the
+    bound lets more than 256 keys through, and rows whose keys tie by the thousand at the k-th (a
+    grammar's mask of -inf, equal values, steps of 1/4), which the parts select by bisection. Once with
+    shared parameters and once with every row's own, in one batch."""
+    monkeypatch.setenv("VSMP_MODE", "split")
+    monkeypatch.setenv("VSMP_SPLIT_P", str(parts))
+    ctx = V.Context(0)
+    Vv = 49153  # 12,289 groups, the last of one element
+    ks = [1, 20, 64, 65, 128, 200, 255, 256]
+    rng = np.random.default_rng(parts)
+    kinds = ["normal", "mask", "equal", "steps", "rising", "two"]
+    lg = rng.normal(0, 2.0, (len(kinds), Vv)).astype(np.float32)
+    for r, kind in enumerate(kinds):
+        if kind == "mask":  # 30 finite values, as many rows of 0 to 30 per part
+            keep = rng.permutation(Vv)[:30]
+            v = lg[r, keep].copy()
+            lg[r] = -np.inf
+            lg[r, keep] = v
+        elif kind == "equal":
+            lg[r] = -0.25
+        elif kind == "steps":
+            lg[r] = np.round(lg[r] * 4) / 4
+        elif kind == "rising":
+            lg[r] = np.arange(Vv, dtype=np.float32) * 1e-4
+        elif kind == "two":  # two values, the larger one 300 times
+            lg[r] = 1.0
+            lg[r, rng.permutation(Vv)[:300]] = 2.0
+    hists = [rng.integers(-2, Vv + 2, 700) for _ in kinds]
+    fields = dict(temp=0.9, top_p=0.95, repeat=1.2, repeat_last=0, seed=77)
+    if per_row:
+        rows = [(k, r) for k in ks + [0] for r in range(len(kinds))]  # k = 0 here: a greedy row
+        p = V.params_array(n=len(rows), **fields)
+        p["top_k"] = [k for k, _ in rows]
+        p["temp"][p["top_k"] == 0] = 0.0
+        p["seed"] = np.arange(len(rows)) + 5
+        h, off = csr([hists[r] for _, r in rows])
+        log("top-k split lists, per row", parts, len(rows))
+        assert Run(ctx, lg[[r for _, r in rows]], p, h, off).report()[1] == 0
+        return
+    h, off = csr(hists)
+    for k in ks:
+        log("top-k split lists", parts, k)
+        assert Run(ctx, lg, V.params_array(n=1, top_k=k, **fields), h, off).report()[1] == 0
+
+
 @pytest.mark.parametrize("kind", ["topp", "minp", "topk", "capped", "capped_minp", "flat"])
 def test_general_path_two_workgroups_per_cu(kind):
     """Shared-parameter batches of general rows without a penalty and with more rows than the device

@@ -1843,26 +1843,27 @@ __device__ __forceinline__ uint32_t key_of(uint32_t bits) {
 // 16-byte groups are cut into P contiguous parts, one 512-thread workgroup each. A part holds its
 // elements as penalised order keys in registers (all its loads in flight at once), bounds its
 // ks-th key from below by the ks-th largest of its 512 lane maxima (two 2048-bin histogram levels
-// in LDS), selects its exact top-ks composites among the keys above that bound with further
-// histogram passes over the registers, and writes them, sorted, with device-scope stores. The part
-// that takes the row's last device-scope ticket merges the P lists and runs the reference epilogue
+// in LDS), ranks the keys above that bound in LDS (where very many tie at it, the exact top-ks found
+// by bisection over the registers first), and writes its top-ks composites, sorted, with device-scope
+// stores. The part that takes the row's last device-scope ticket merges the P lists and runs the reference epilogue
 // (finish_smallk, as k_finish does after slices), then clears the ticket for the next call.
 
 constexpr int kTkNT = 512;
 constexpr int kTkW = kTkNT / 64;
 constexpr int kTkU = 8;                     // 16-byte loads per thread: the whole part in flight
+constexpr int kTkList = 2 * kTkNT;          // keys above the row bound that a part ranks as they are
 static_assert(kTkNT * kTkU == kSplitMaxPartGroups, "the planner sizes parts by kSplitMaxPartGroups");
 
 struct __align__(16) TkShared {
-  uint32_t bins[2][kRowBins];                // row-bound and select histograms (read as uint4)
+  uint32_t bins[2][kRowBins];                // row-bound histograms (read as uint4)
   uint32_t bits[kSplitMaxPartGroups / 8];    // the part's penalty bitmap (4 elements per group)
-  uint64_t top[kKmax];                       // the part's top-ks; the merged top-k
-  int rank[kKmax];
+  uint64_t top[kKmax];                       // the merged top-k
   uint64_t red64[kTkW];
   uint32_t red32[kTkW];
+  uint32_t cnt[2][kTkW];                     // a counting step's sums per wave
   int ints[16];
   int off[kMaxMergeSlices + 1];
-  __align__(16) uint64_t mbuf[kMergeCap];    // the last part's merge and epilogue workspace
+  __align__(16) uint64_t mbuf[kMergeCap];    // the part's list; the last part's merge and epilogue workspace
 };
 // rank_count reads it in 16-byte pieces. At 8 bytes off, every such LDS read took several times as
 // long: the merge's ranking 9.8 us at k = 100 in 16 parts (a 4 x 151,936 batch).
@@ -1926,7 +1927,7 @@ __device__ __forceinline__ void topk_part(const KArgs& a, TkShared& sh, const vs
   for (int u = 0; u < kTkU; ++u) v[u] = stream_ld(rp4 + min(g0 + u * kTkNT + tid, glast));
 
   for (int i = tid; i < 2 * kRowBins; i += kTkNT) (&sh.bins[0][0])[i] = 0u;
-  if (tid == 0) sh.ints[8] = 0;
+  if (tid == 0) sh.ints[8] = sh.ints[10] = 0;
   // penalty bitmap of the part (src/sampler.cpp:53-65)
   const int words = (hi - lo + 31) >> 5;
   if (pen) {
@@ -2035,38 +2036,12 @@ __device__ __forceinline__ void topk_part(const KArgs& a, TkShared& sh, const vs
     const int b2 = sh.ints[4];
     T = (b1 >= 0 && b2 >= 0) ? ((static_cast<uint32_t>(b1) << 21) | (static_cast<uint32_t>(b2) << 10)) : 0u;
     T = __builtin_amdgcn_readfirstlane(T);
-    for (int i = tid; i < 2 * kRowBins; i += kTkNT) (&sh.bins[0][0])[i] = 0u;
-    __syncthreads();
   }
 
-  // the part's list: every composite >= clo, collected in LDS (at most kKmax kept)
-  auto collect = [&](uint64_t clo) {
-#pragma unroll
-    for (int u = 0; u < kTkU; ++u) {
-      const uint32_t kk[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
-      const int e = 4 * (g0 + u * kTkNT + tid);
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        const uint64_t cc = kk[c] ? comp(kk[c], static_cast<uint32_t>(e + c)) : 0ull;
-        const bool t = ks > 0 && kk[c] != 0u && cc >= clo;
-        const uint64_t m = __ballot(t);
-        if (m) {
-          int base = 0;
-          if (lane == 0) base = atomicAdd(&sh.ints[8], __popcll(m));
-          base = __builtin_amdgcn_readfirstlane(base);  // lane 0: every lane is active here
-          const int pos = base + static_cast<int>(__builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(m >> 32),
-                                                                            __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(m), 0u)));
-          if (t && pos < kKmax) sh.top[pos] = cc;
-        }
-      }
-    }
-  };
-  // Usually the keys above the bound fit the list: it is kept whole (the merge takes the row's top
-  // k from the union of the lists, each sorted). Each lane marks its keys in a mask, a wave's take
-  // their places by a scan of the counts and one LDS atomic. Otherwise the exact ks-th largest
-  // composite is found first: 2048-bin passes over the composites >= T << 32 in registers, each
-  // narrowing [clo, chi] to the bucket that holds it, until the bucket is taken whole; the list is
-  // then exactly ks long.
+  // Usually the keys above the bound fit the list (about 1.1 to 1.4 ks of them in 16,384 distinct
+  // ones). Each lane marks its keys in a mask, a wave's take their places by a scan of the counts and
+  // one LDS atomic.
+  static_assert(4 * kTkU <= 32, "one mask bit per key");
   uint32_t hit = 0u;
   {
     const uint32_t t1 = max(T, 1u);  // 0 marks a place past the part
@@ -2076,90 +2051,96 @@ __device__ __forceinline__ void topk_part(const KArgs& a, TkShared& sh, const vs
               static_cast<uint32_t>(v[u].z >= t1) << 2 | static_cast<uint32_t>(v[u].w >= t1) << 3)
              << (4 * u);
   }
-  static_assert(4 * kTkU <= 32, "one mask bit per key");
   if (ks == 0) hit = 0u;
-  int place;
-  {
+  auto places = [&](int* count) -> int {  // this lane's first place; *count grows by the wave's keys
     const uint32_t n = __popc(hit);
     const uint32_t incl = wave_incl_scan(n);
     int base = 0;
-    if (lane == 63 && incl) base = atomicAdd(&sh.ints[8], static_cast<int>(incl));
-    place = __builtin_amdgcn_readlane(base, 63) + static_cast<int>(incl - n);
-  }
+    if (lane == 63 && incl) base = atomicAdd(count, static_cast<int>(incl));
+    return __builtin_amdgcn_readlane(base, 63) + static_cast<int>(incl - n);
+  };
+  int place = places(&sh.ints[8]);
   __syncthreads();
-  const int nabove = sh.ints[8];
-  if (nabove <= kKmax) {
-#pragma unroll
-    for (int u = 0; u < kTkU; ++u) {
-      if (((hit >> (4 * u)) & 0xFu) == 0u) continue;
-      const uint32_t kk[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
-#pragma unroll
-      for (int c = 0; c < 4; ++c)
-        if ((hit >> (4 * u + c)) & 1u) sh.top[place++] = comp(kk[c], static_cast<uint32_t>(4 * (g0 + u * kTkNT + tid) + c));
-    }
-  } else {
-    uint64_t clo = static_cast<uint64_t>(T) << 32;
-    uint64_t chi = block_max64<kTkNT>((static_cast<uint64_t>(lm) << 32) | 0xFFFFFFFFull, sh.red64);  // at or above every key
-    if (tid == 0) sh.ints[8] = 0;
-    int need = ks;
-    for (int pass = 0; clo != chi && pass < 9; ++pass) {
-      const uint64_t R = chi - clo;
-      const int sft = R < static_cast<uint64_t>(kRowBins) ? 0 : 53 - __clzll(static_cast<long long>(R));
-      uint32_t* bins = sh.bins[pass & 1];
-      for (int i = tid; i < kRowBins; i += kTkNT) sh.bins[(pass + 1) & 1][i] = 0u;
+  int nt = sh.ints[8];
+  if (nt > kTkList) {
+    // Many keys tie near the ks-th (a grammar's mask, a row of few distinct values): the ks-th largest
+    // key K by bisection, and among the keys equal to it the first by index. A step counts over the
+    // registers with one barrier and no atomics, so it takes as long whatever the keys (0.2 us): 2,048-bin
+    // histogram passes, whose atomics meet on the ties' bins, took 120 us in 32 rows of 151,936 with 30
+    // finite logits each. The ties lie in the bound's bucket as a rule, so the first step tests its top.
+    int step = 0;
+    auto count = [&](auto&& in) -> int {  // the part's elements that `in` takes
+      uint32_t n = 0u;
 #pragma unroll
       for (int u = 0; u < kTkU; ++u) {
-        const uint32_t kk[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
-        const int e = 4 * (g0 + u * kTkNT + tid);
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          if (kk[c] < T || kk[c] == 0u) continue;
-          const uint64_t cc = comp(kk[c], static_cast<uint32_t>(e + c));
-          if (cc >= clo && cc <= chi) atomicAdd(&bins[(cc - clo) >> sft], 1u);
-        }
+        const int d = 4 * (u * kTkNT + tid);
+        n += __popcll(__ballot(in(v[u].x, d))) + __popcll(__ballot(in(v[u].y, d + 1))) +
+             __popcll(__ballot(in(v[u].z, d + 2))) + __popcll(__ballot(in(v[u].w, d + 3)));
       }
+      uint32_t* c = sh.cnt[step++ & 1];  // the step before this one's other half is read behind this barrier
+      if (lane == 0) c[w] = n;
       __syncthreads();
-      if (w == 0) wave_find_bucket(bins, need, sh.ints);
-      __syncthreads();
-      const int b = sh.ints[0];
-      const int inb = sh.ints[2];
-      need -= sh.ints[1];
-      __syncthreads();
-      if (b < 0) break;  // unreachable: ks composites lie at or above T << 32
-      const uint64_t nlo = clo + (static_cast<uint64_t>(b) << sft);
-      const uint64_t wdt = sft == 0 ? 0ull : (1ull << sft) - 1ull;
-      chi = (chi - nlo < wdt) ? chi : nlo + wdt;
-      clo = nlo;
-      if (inb == need) chi = clo;  // the whole bucket is taken: the top ks are the composites >= clo
+      uint32_t all = 0u;
+#pragma unroll
+      for (int i = 0; i < kTkW; ++i) all += c[i];
+      return __builtin_amdgcn_readfirstlane(static_cast<int>(all));
+    };
+    uint32_t klo = max(T, 1u);  // at least ks keys lie at or above klo, fewer above khi
+    uint32_t khi = comp_key(block_max64<kTkNT>(static_cast<uint64_t>(lm) << 32, sh.red64));
+    uint32_t mid = (T | 1023u) < khi ? (T | 1023u) + 1u : khi;
+    int above = 0;  // keys above khi
+    while (klo < khi) {
+      const int n = count([mid](uint32_t kk, int) { return kk >= mid; });
+      if (n >= ks) {
+        klo = mid;
+      } else {
+        khi = mid - 1u;
+        above = n;
+      }
+      mid = klo + (khi - klo + 1u) / 2u;
     }
-    collect(clo);
-  }
-  if (tid < kKmax) sh.rank[tid] = 0;
-  __syncthreads();
-  const int nt = min(sh.ints[8], kKmax);
-  {
-    const int parts = nt <= 64 ? kTkW : kTkNT / max(nt, 1);
-    const int pw = nt <= 64 ? w : tid / max(nt, 1);
-    const int ci = nt <= 64 ? lane : tid % max(nt, 1);
-    if (nt > 0 && pw < parts && ci < nt) {
-      const int chunk = (nt + parts - 1) / parts;
-      const uint64_t x = sh.top[ci];
-      int r = 0;
-      const int j1 = min(nt, (pw + 1) * chunk);
-      for (int j = pw * chunk; j < j1; ++j) r += sh.top[j] > x;
-      if (r) atomicAdd(&sh.rank[ci], r);
+    const int need = ks - above;  // of the keys equal to klo
+    int elo = 0, ehi = 4 * kTkNT * kTkU - 1;  // the first index that takes `need` of them
+    while (elo < ehi) {
+      const int em = (elo + ehi) >> 1;
+      if (count([klo, em](uint32_t kk, int d) { return kk == klo && d <= em; }) >= need)
+        ehi = em;
+      else
+        elo = em + 1;
     }
+    hit = 0u;
+#pragma unroll
+    for (int u = 0; u < kTkU; ++u) {
+      const int d = 4 * (u * kTkNT + tid);
+      auto in = [klo, elo](uint32_t kk, int at) { return static_cast<uint32_t>(kk > klo || (kk == klo && at <= elo)); };
+      hit |= (in(v[u].x, d) | in(v[u].y, d + 1) << 1 | in(v[u].z, d + 2) << 2 | in(v[u].w, d + 3) << 3) << (4 * u);
+    }
+    place = places(&sh.ints[10]);
+    nt = ks;
   }
+#pragma unroll
+  for (int u = 0; u < kTkU; ++u) {
+    if (((hit >> (4 * u)) & 0xFu) == 0u) continue;
+    const uint32_t kk[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+      if ((hit >> (4 * u + c)) & 1u) sh.mbuf[place++] = comp(kk[c], static_cast<uint32_t>(4 * (g0 + u * kTkNT + tid) + c));
+  }
+  pad16(sh.mbuf, nt, tid);
   __syncthreads();
-  for (int i = tid; i < nt; i += kTkNT)
-    __hip_atomic_store(&a.s_cand[slot * kKmax + sh.rank[i]], sh.top[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  // the part's top ks in order, by counting
+  for (int i = tid; i < nt; i += kTkNT) {
+    const uint64_t x = sh.mbuf[i];
+    const int r = rank_count(sh.mbuf, nt, x);
+    if (r < ks) __hip_atomic_store(&a.s_cand[slot * kKmax + r], x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
   uint32_t np = 0;
   if (a.info && pen) {
     for (int i = tid; i < words; i += kTkNT) np += __popc(sh.bits[i]);
     np = block_sum_u32<kTkNT>(np, sh.red32);
   }
   if (tid == 0) {
-    __hip_atomic_store(&a.s_cnt[slot], nt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(&a.s_cnt[slot], ks, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __hip_atomic_store(&a.s_npen[slot], static_cast<int>(np), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
   if (!topk_last_part(a, row, &sh.ints[9])) return;
