@@ -879,6 +879,47 @@ def test_general_split_parts(monkeypatch, parts, Vv):
     assert torch.equal(states[0], states[1]) and torch.equal(ids[0], ids[1])
 
 
+@pytest.mark.parametrize("per_row", [False, True])
+def test_general_topk_from_the_histogram(ctx, mode, per_row):
+    """Rows with 256 < k < V whose k-th element is found in its mass bucket: k from 257 to V - 2, the
+    k-th in a bucket of few elements, among thousands of equal values, among -inf behind a grammar's
+    mask and in a cold row's last bucket; min-p cuts before and behind the k-th, top-p cuts, draws
+    without a cut, flat rows. As one workgroup per row, over slices, and over parts."""
+    Vv = 40009
+    kinds = ["normal", "mask", "ties", "steps", "flat", "cold", "spiky"]
+    opts = [dict(top_k=257, top_p=0.9), dict(top_k=1024, min_p=0.01), dict(top_k=1025, top_p=0.95), dict(top_k=2000, min_p=1e-3),
+            dict(top_k=2000, top_p=0.5, min_p=0.3), dict(top_k=20000, top_p=0.99), dict(top_k=Vv - 2, top_p=1.0), dict(top_k=5000, min_p=1e-30)]
+    rng = np.random.default_rng(12)
+    lg = rng.normal(0, 1.5, (len(kinds), Vv)).astype(np.float32)
+    for r, kind in enumerate(kinds):
+        if kind == "mask":
+            keep = rng.permutation(Vv)[:600]
+            v = lg[r, keep].copy()
+            lg[r] = -np.inf
+            lg[r, keep] = v
+        elif kind == "ties":
+            lg[r, ::6] = 1.25
+        elif kind == "steps":
+            lg[r] = np.round(lg[r] * 8) / 8
+        elif kind == "flat":
+            lg[r] = 0.75
+        elif kind == "spiky":
+            lg[r, rng.integers(0, Vv, 12)] += 9.0
+    hists = [rng.integers(-2, Vv + 2, int(rng.integers(0, 300))) if kind != "flat" else [] for kind in kinds]
+    rows = [(o, r) for o in opts for r in range(len(kinds))]
+    p = V.params_array(rows=[dict(dict(temp=0.05 if kinds[r] == "cold" else 1.1, top_p=1.0, repeat=1.2, repeat_last=0, seed=9 + i), **o)
+                             for i, (o, r) in enumerate(rows)])
+    if per_row:
+        h, off = csr([hists[r] for _, r in rows])
+        log("top-k from the histogram, per row", mode, len(rows))
+        assert Run(ctx, lg[[r for _, r in rows]], p, h, off).report()[1] == 0
+        return
+    h, off = csr(hists)
+    for i in range(0, len(rows), len(kinds)):
+        log("top-k from the histogram", mode, rows[i][0])
+        assert Run(ctx, lg, p[i:i + 1], h, off).report()[1] == 0
+
+
 def test_graph_capture_after_a_larger_warm_up():
     """The split kernels' scratch is sized by any call at a shape or a larger one: after one call of a
     wide batch on another path, smaller batches of every split path are captured and replayed."""

@@ -345,8 +345,8 @@ Plan plan(const vsmp_ctx* ctx, int B, int V, const vsmp_params* hostp) {
     // leaves those rows alone), on a stream forked from the caller's: the few long general rows
     // then overlap the row kernel instead of following it.
     pl.side_general = !hostp;
-    // k <= kGenCap or top-k off: the split takes the row (with per-row parameters it leaves other
-    // general rows to one of their workgroups)
+    // k <= kGenCap or top-k off: the split takes the row (with per-row parameters it leaves a larger
+    // k to one of their workgroups after the histogram)
     if (pl.any_general && fm != 1) {
       pl.gen = general_parts(B, V, !hostp, fm == 2, ctx->split_p);
       pl.gen_split = pl.gen.P > 0 && (!hostp || hostp->top_k <= kGenCap || hostp->top_k >= V);

@@ -2244,9 +2244,6 @@ __device__ __forceinline__ void gen_part_range(const KArgs& a, int row, uint64_t
   mxc = sgpr_u64(m);
   mnk = sgpr_u32(n);
 }
-// A row whose k-th element the split selects: top-k off, or a top-k whose elements fit one list.
-__device__ __forceinline__ bool gen_split_row(int k, int V) { return k == V || k <= kGenCap; }
-
 __global__ __launch_bounds__(kGsNT) void k_gen_max(SplitArgs a) {
   __shared__ uint32_t bits[kGenPartChunks * kGsChunk / 8];
   __shared__ uint64_t red[kGsNT / 64];
@@ -2335,7 +2332,7 @@ __global__ __launch_bounds__(kGsNT) void k_gen_hist(SplitArgs a) {
   const GenPart t = gen_part(a);
   const int tid = threadIdx.x, V = a.V, row = t.row;
   const vsmp_params P = sgpr_params(row_params(a, row));
-  if (path_of(P, V, a.smallk_ok) != kPathGeneral || !gen_split_row(top_k_of(P, V), V)) return;
+  if (path_of(P, V, a.smallk_ok) != kPathGeneral) return;
   int h0, h1;
   row_hist(a, row, h0, h1);
   GenCtx g;
@@ -2659,13 +2656,16 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
   };
   if constexpr (!SPLIT) count_pen();
 
-  // top-k prefix when 256 < k < V: the k-th element by count
-  g.ckk = 0ull;
+  // A flat row: every penalised value the same finite float, as in a padding row of zeros.
+  const bool flat = comp_key(mxc) == static_cast<uint32_t>(mnk) && isfinite(g.mx);
+  // top-k prefix when 256 < k < V: the k-th element's composite, once it is known
+  g.ckk = flat && k < V ? comp(comp_key(mxc), static_cast<uint32_t>(k - 1)) : 0ull;
   // SPLIT: alone = the rest of the row is taken by this workgroup by itself (part 0; the others have
   // returned), pass by pass as without the split. Every part decides it from the same values.
-  bool alone = !SPLIT || !gen_split_row(k, V);
+  bool alone = !SPLIT || flat;
   if constexpr (SPLIT)
     if (alone && part.part != 0) return;
+  bool by_hist = false;  // ... with the parts' histogram, once the k-th element is found in its bucket
   constexpr int BP = kGenBuckets / kGenThreads;
   static_assert(BP % 4 == 0, "a thread's buckets are read as 16-byte vectors");
   const int b0 = BP * tid;
@@ -2747,10 +2747,13 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
       }
     }
     if (!alone) {
-      if (k < V) {  // the elements through the k-th's bucket have to fit one list
-        qk = sgpr_i32(sh.ints[0]);
-        alone = qk >= kGenBuckets || (capped && qk == kGenBuckets - 1) || sgpr_u32(sh.cnt0[min(qk, kGenBuckets - 1)]) > kGenPartList;
-        if (alone && part.part != 0) return;
+      if (k < V) {
+        // The elements through the k-th's bucket fit one list, or one workgroup ends the row with the
+        // parts' histogram (24 x 128,256, per-row top-k 2,000: 85 us, against 180 when it took every pass
+        // and 158 in one workgroup of 1,024 threads that took every pass).
+        qk = min(sgpr_i32(sh.ints[0]), kGenBuckets - 1);
+        by_hist = k > kGenCap || (capped && qk == kGenBuckets - 1) || sgpr_u32(sh.cnt0[qk]) > kGenPartList;
+        if (by_hist && part.part != 0) return;
         __syncthreads();
       }
     }
@@ -2824,14 +2827,6 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
     }
     return gen_last_part(a, row, &sh.ints[6]);
   };
-  if (alone && k < V) {
-    auto all_v = [](float) { return true; };
-    auto all_c = [](uint64_t) { return true; };
-    const Sel s = refine_select<false>(g, sh, all_v, all_c, static_cast<uint64_t>(static_cast<uint32_t>(mnk)) << 32, mxc, V, 0,
-                                       0.0, static_cast<double>(k));
-    g.ckk = s.ck;
-  }
-
   // pass: min-p statistics, level-0 count and mass histograms (the masses as fixed-point sums
   // relative to the table points, numer_fix, in the mass array's 8-byte slots until the prefix
   // below turns them into fp64 masses)
@@ -2862,7 +2857,6 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
   double t_totm = 0.0, t_omass = 0.0;
   uint64_t t_ofix = 0ull;
   uint32_t t_cntm = 0, t_ocnt = 0;
-  const bool cut_k = g.ckk != 0ull;
   // The overflow bucket of a capped row holds elements at least 63.98 temp below the maximum, whose
   // numerators are below 1.6e-28: together under 2e-22 of the sum (the maximum's numerator is 1),
   // which a sum in the reference's order absorbs without a trace. They are counted without a
@@ -2870,10 +2864,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
   const bool ovf_exact = capped && minp && thr < 1e-26;
   // ovf: the overflow bucket (most of a cold row when capped) is counted per thread rather than by
   // atomics that would all hit one address; with_minp: the min-p statistics are taken
-  auto main_pass = [&](auto ovf, auto with_minp, auto with_cut) {
-    auto excluded = [&](int e, float v) {
-      return decltype(with_cut)::value && cut_k && comp(ord_key(v), static_cast<uint32_t>(e)) < g.ckk;
-    };
+  auto main_pass = [&](auto ovf, auto with_minp) {
     auto add = [&](int e, float v, float d, int q, uint64_t f) {
       if (decltype(ovf)::value && q == kGenBuckets - 1) {
         ++t_ocnt;
@@ -2907,7 +2898,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
         [&](int e, float v) {
           const float d = v - g.mx;
           const int q = q_of_d(g, d);
-          if (!excluded(e, v)) add(e, v, d, q, numer_fix(fc, d, q));
+          add(e, v, d, q, numer_fix(fc, d, q));
         },
         // the four masses first, then the four elements' histogram atomics together
         [&](int e, const float (&x)[4]) {
@@ -2921,22 +2912,18 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
             f[c] = numer_fix(fc, d[c], q[c]);
           }
 #pragma unroll
-          for (int c = 0; c < 4; ++c)
-            if (!excluded(e + c, x[c])) add(e + c, x[c], d[c], q[c], f[c]);
+          for (int c = 0; c < 4; ++c) add(e + c, x[c], d[c], q[c], f[c]);
         });
   };
-  // A flat row (every penalised value the same finite float, as in a padding row of zeros) has
-  // every element in bucket 0 with the numerator exp(0) = 1 (fixed point 2^40, numer_fix): its
+  // A flat row has every element in bucket 0 with the numerator exp(0) = 1 (fixed point 2^40, numer_fix): its
   // histogram, min-p count and prefix are known without the pass, whose atomics would all meet on
   // one address (256 x 151,936 zeros, top-p .9: 1,063 to 809 us per call, against 115 us for rows
   // of normal values; the selects after it refine that one bucket over the row's indices).
   // With a top-k cut the kept elements are the first k by index (equal values rank by index).
-  const bool flat = comp_key(mxc) == static_cast<uint32_t>(mnk) && isfinite(g.mx);
-  // one instance per combination without a top-k restriction (the common case: no per-element
-  // branches beyond the ones asked for); rows with one share an instance
+  // one instance per combination: no per-element branches beyond the ones asked for
   if (!alone) {  // SPLIT: k_gen_hist took the pass
   } else if (flat) {
-    const int n_in = cut_k ? k : V;
+    const int n_in = k;  // V with top-k off
     if (tid == 0) {
       sh.cnt0[0] = static_cast<uint32_t>(n_in);
       fix0[0] = static_cast<uint64_t>(n_in) * (kFixRawE + (1ull << 40));  // n_in bits of 4097.0
@@ -2950,16 +2937,14 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
       const uint32_t key = comp_key(mxc);
       for (int i = tid; i < min(n_in, kGenCap); i += kGenThreads) sh.list[i] = comp(key, static_cast<uint32_t>(i));
     }
-  } else if (cut_k)
-    main_pass(std::true_type{}, std::true_type{}, std::true_type{});
-  else if (capped && minp)
-    main_pass(std::true_type{}, std::true_type{}, std::false_type{});
+  } else if (capped && minp)
+    main_pass(std::true_type{}, std::true_type{});
   else if (capped)
-    main_pass(std::true_type{}, std::false_type{}, std::false_type{});
+    main_pass(std::true_type{}, std::false_type{});
   else if (minp)
-    main_pass(std::false_type{}, std::true_type{}, std::false_type{});
+    main_pass(std::false_type{}, std::true_type{});
   else
-    main_pass(std::false_type{}, std::false_type{}, std::false_type{});
+    main_pass(std::false_type{}, std::false_type{});
   if (alone) {
     const uint32_t oc = block_sum_u32<kGenThreads>(t_ocnt, sh.r32);
     const double om = block_sum_f64<kGenThreads>(t_omass, sh.rd);
@@ -2993,7 +2978,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
   // The kept set's smallest composite (its last element in the reference's order), taken by a pass
   // of its own only when it is needed: a draw that falls past the kept set (rounding) or the
   // diagnostics. by_minp: the set is the min-p prefix (numerator >= thr), else the top-k prefix.
-  auto kept_last = [&](bool by_minp) -> uint64_t {
+  auto kept_last = [&](bool by_minp) __attribute__((always_inline)) -> uint64_t {  // a call would put g in scratch
     uint64_t t = ~0ull;
     gen_pass<NT>(g.R, [&](int e, float v) {
       const uint64_t ck = comp(ord_key(v), static_cast<uint32_t>(e));
@@ -3002,6 +2987,19 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
       t = min64(t, ck);
     });
     return block_min64<kGenThreads>(t, sh.r64);
+  };
+  // the composite range of the elements that in_q takes, among the top-k prefix
+  auto bucket_range = [&](auto&& in_q, uint64_t& clo, uint64_t& chi) {
+    uint64_t lo_ = ~0ull, hi_ = 0ull;
+    gen_pass<NT>(g.R, [&](int e, float v) {
+      if (!in_q(v)) return;
+      const uint64_t ck = comp(ord_key(v), static_cast<uint32_t>(e));
+      if (ck < g.ckk) return;
+      lo_ = min64(lo_, ck);
+      hi_ = max64(hi_, ck);
+    });
+    clo = block_min64<kGenThreads>(lo_, sh.r64);
+    chi = block_max64<kGenThreads>(hi_, sh.r64);
   };
   // level-0 inclusive prefixes (BP consecutive buckets per thread, bucket 0 = closest to the maximum)
   if (alone) {
@@ -3031,6 +3029,64 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
       sh.cnt0[b0 + i] = ec;
     }
     if (tid < 4) sh.fb[tid] = kGenBuckets;
+    __syncthreads();
+  }
+  if (k < V && !flat && (alone || by_hist)) {
+    // The k-th element, in the bucket where the counts reach k; the prefixes then end with it, as if the
+    // pass had taken no other. From the whole row instead of its bucket the k-th took two histogram
+    // passes more, and the main pass a compare per element.
+    if (alone) {
+      if (tid == 0) sh.ints[0] = kGenBuckets - 1;
+      __syncthreads();
+      int f = kGenBuckets;
+#pragma unroll
+      for (int i = BP - 1; i >= 0; --i)
+        if (sh.cnt0[b0 + i] >= static_cast<uint32_t>(k)) f = b0 + i;
+      wave_claim_min(&sh.ints[0], f < kGenBuckets, f);
+      __syncthreads();
+      qk = sgpr_i32(sh.ints[0]);
+    }
+    const int ra = qk > 0 ? sgpr_i32(static_cast<int>(sh.cnt0[qk - 1])) : 0;
+    const int n = sgpr_i32(static_cast<int>(sh.cnt0[qk])) - ra;
+    const double above = qk > 0 ? sgpr_f64(sh.mass0[qk - 1]) : 0.0;
+    auto in_q = [&g, qk](float v) { return q_of(g, v) == qk; };
+    uint64_t clo = 0ull, chi = ~0ull;
+    if (n > kGenCap) bucket_range(in_q, clo, chi);
+    __syncthreads();
+    const Sel s = refine_select<false>(g, sh, in_q, [](uint64_t) { return true; }, clo, chi, n, ra, static_cast<double>(ra),
+                                       static_cast<double>(k));
+    g.ckk = s.ck;
+    double m = 0.0;
+    if (n <= kGenCap) {  // all of the bucket, in order
+      for (int i = tid; i < k - ra; i += kGenThreads) m += numer_g(g, comp_val(sh.list[i]));
+    } else if (!capped || qk < kGenBuckets - 1) {  // a capped row's last bucket adds nothing to a sum
+      const uint64_t ckk = g.ckk;
+      gen_pass<NT>(g.R, [&](int e, float v) {
+        if (in_q(v) && comp(ord_key(v), static_cast<uint32_t>(e)) >= ckk) m += numer_g(g, v);
+      });
+    }
+    const double through = above + block_sum_f64<kGenThreads>(m, sh.rd);
+#pragma unroll
+    for (int i = 0; i < BP; ++i) {
+      if (b0 + i < qk) continue;
+      sh.cnt0[b0 + i] = static_cast<uint32_t>(k);
+      sh.mass0[b0 + i] = through;
+    }
+    if (cntm >= static_cast<uint32_t>(k)) {  // min-p cuts behind the k-th
+      cntm = static_cast<uint32_t>(k);
+      totm = through;
+    }
+    if (tid == 0) sh.ints[4] = by_hist ? nlist : -1;  // the refinement took the min-p list's place
+    if constexpr (SPLIT) {
+      if (by_hist) {
+        alone = true;
+#pragma unroll
+        for (int i = 0; i < BP; ++i) rm[i] = 0.0;  // not read again: not held through the passes above
+        if (tid < 4) sh.fb[tid] = kGenBuckets;
+        if (minp && cntm <= static_cast<uint32_t>(kGenCap) && nlist == static_cast<int>(cntm))
+          gen_gather<NT>(a, row, 1, 0, sh.list, kGenCap, part_off[0]);
+      }
+    }
     __syncthreads();
   }
   // the sum over the top-k prefix (src/sampler.cpp:84): the histogram's total
@@ -3123,18 +3179,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
     auto in_q_v = [&g, qb](float v) { return q_of(g, v) == qb; };
     auto in_q_c = [ckk](uint64_t ck) { return ck >= ckk; };
     uint64_t clo = 0ull, chi = ~0ull;
-    if (n > kGenCap) {  // tighten the composite range to the bucket's
-      uint64_t lo_ = ~0ull, hi_ = 0ull;
-      gen_pass<NT>(g.R, [&](int e, float v) {
-        if (!in_q_v(v)) return;
-        const uint64_t ck = comp(ord_key(v), static_cast<uint32_t>(e));
-        if (!in_q_c(ck)) return;
-        lo_ = min64(lo_, ck);
-        hi_ = max64(hi_, ck);
-      });
-      clo = block_min64<kGenThreads>(lo_, sh.r64);
-      chi = block_max64<kGenThreads>(hi_, sh.r64);
-    }
+    if (n > kGenCap) bucket_range(in_q_v, clo, chi);  // tighten the composite range to the bucket's
     __syncthreads();
     s = refine_select<true>(g, sh, in_q_v, in_q_c, clo, chi, n, rank_above, above, target);
     return s;
