@@ -920,6 +920,41 @@ def test_general_topk_from_the_histogram(ctx, mode, per_row):
         assert Run(ctx, lg, p[i:i + 1], h, off).report()[1] == 0
 
 
+@pytest.mark.parametrize("parts", [3, 16, 64])
+def test_general_split_large_buckets(monkeypatch, parts):
+    """Split general rows with thousands of elements in one mass bucket, whose count the raw sums hold only
+    modulo 4,096: 3,900 to 40,000 equal values at the top, in the bulk and in the tail, two such buckets,
+    all values in steps, and flat rows, with top-p cuts, top-k, min-p and draws without a cut, in rows
+    whose buckets are narrow (a warm row) and as wide as they get (a cold row, capped)."""
+    monkeypatch.setenv("VSMP_MODE", "split")
+    monkeypatch.setenv("VSMP_SPLIT_P", str(parts))
+    ctx = V.Context(0)
+    Vv = 70001
+    rng = np.random.default_rng(parts)
+    lg, temps = [], []
+    for n in (3900, 4031, 4032, 4096, 6000, 8192, 40000):
+        for value in (6.5, 0.3, -5.0):
+            x = rng.normal(0, 1.5, Vv).astype(np.float32)
+            x[rng.permutation(Vv)[:n]] = value
+            lg.append(x)
+            temps.append(1.0 if value != 0.3 else 0.06)
+    x = rng.normal(0, 1.5, Vv).astype(np.float32)
+    x[::9], x[1::9] = 1.0, -0.5
+    lg += [x, (np.round(rng.normal(0, 1.5, Vv) * 4) / 4).astype(np.float32), np.full(Vv, -3.25, np.float32)]
+    temps += [0.9, 0.9, 0.9]
+    lg = np.stack(lg)
+    hists = [rng.integers(0, Vv, 100) if r % 2 else [] for r in range(len(lg))]
+    h, off = csr(hists)
+    for f in (dict(top_p=0.95), dict(top_p=0.3), dict(), dict(top_p=0.9, min_p=0.02), dict(top_k=900, top_p=0.9), dict(top_k=30000)):
+        p = V.params_array(rows=[dict(dict(temp=t, top_k=0, top_p=1.0, repeat=1.1, repeat_last=0, seed=31 + i), **f) for i, t in enumerate(temps)])
+        log("general split, large buckets, per row", parts, f)
+        assert Run(ctx, lg, p, h, off).report()[1] == 0
+        if "top_k" in f and f["top_k"] > 1024:
+            continue  # shared parameters: not a split batch
+        log("general split, large buckets", parts, f)
+        assert Run(ctx, lg, V.params_array(n=1, **dict(dict(temp=0.8, top_k=0, top_p=1.0, repeat=1.1, repeat_last=0, seed=3), **f)), h, off).report()[1] == 0
+
+
 def test_graph_capture_after_a_larger_warm_up():
     """The split kernels' scratch is sized by any call at a shape or a larger one: after one call of a
     wide batch on another path, smaller batches of every split path are captured and replayed."""

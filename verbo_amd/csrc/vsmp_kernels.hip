@@ -1670,33 +1670,29 @@ __device__ __forceinline__ Sel refine_select(const GenCtx& g, GenShared<NT>& sh,
       if (ck < clo || ck > chi || !pred_c(ck)) return -1;
       return static_cast<int>((ck - clo) >> shift);
     };
-    // Four neighbours in one bucket (as in a row of equal values, whose buckets are ranges of
-    // indices) add with one atomic pair rather than four on one address.
-    gen_pass_groups<NT, 1>(
-        g.R,
-        [&](int e, float v) {
-          const int d = bucket(e, v);
-          if (d < 0) return;
-          atomicAdd(&sh.rcnt[d], 1u);
-          if (MASS) atomicAdd(&sh.rmass[d], numer_g(g, v));
-        },
-        [&](int e, const float (&x)[4]) {
-          int d[4];
-#pragma unroll
-          for (int c = 0; c < 4; ++c) d[c] = bucket(e + c, x[c]);
-          if (d[0] >= 0 && d[0] == d[1] && d[0] == d[2] && d[0] == d[3]) {
-            atomicAdd(&sh.rcnt[d[0]], 4u);
-            if (MASS)
-              atomicAdd(&sh.rmass[d[0]], ((numer_g(g, x[0]) + numer_g(g, x[1])) + numer_g(g, x[2])) + numer_g(g, x[3]));
-            return;
-          }
-#pragma unroll
-          for (int c = 0; c < 4; ++c) {
-            if (d[c] < 0) continue;
-            atomicAdd(&sh.rcnt[d[c]], 1u);
-            if (MASS) atomicAdd(&sh.rmass[d[c]], numer_g(g, x[c]));
-          }
-        });
+    // A thread's successive elements of one bucket add with one atomic pair: where thousands of equal
+    // values share a bucket, the atomics on its address are what the pass waits for.
+    int run_d = -1;
+    uint32_t run_n = 0u;
+    double run_m = 0.0;
+    auto flush = [&]() {
+      if (run_d < 0) return;
+      atomicAdd(&sh.rcnt[run_d], run_n);
+      if (MASS) atomicAdd(&sh.rmass[run_d], run_m);
+    };
+    gen_pass<NT>(g.R, [&](int e, float v) {
+      const int d = bucket(e, v);
+      if (d < 0) return;
+      if (d != run_d) {
+        flush();
+        run_d = d;
+        run_n = 0u;
+        run_m = 0.0;
+      }
+      ++run_n;
+      if (MASS) run_m += numer_g(g, v);
+    });
+    flush();
     __syncthreads();
     // scan buckets from the top (largest composites first): position p <-> bucket kRefBuckets-1-p,
     // RP consecutive positions per thread
@@ -2171,8 +2167,9 @@ __device__ __forceinline__ void topk_part(const KArgs& a, TkShared& sh, const vs
 // within e^(+-1/64) of 2^40), so the top 12 bits are n kFixRawE's, an odd multiple of n mod 4096, and
 // give n back (gen_raw_count). A larger bucket decodes to something else; a decoded count above
 // kRawCountMax is taken as 0, so a bucket that is not decoded exactly is decoded too low, and the
-// counts of a row add up to its elements only when all are exact. Otherwise (rows of very many
-// equal values) one workgroup takes the row by itself, counting as k_general does.
+// counts of a row add up to its elements only when all are exact. Otherwise gen_raw_count_any looks
+// closer, and where that is not enough (several buckets of many thousands) one workgroup takes the
+// row by itself, counting as k_general does.
 constexpr int kGsNT = 512;
 constexpr int kGsU = 8;
 constexpr int kGsChunk = kGsNT * kGsU;  // 16-byte groups a part holds in registers at once
@@ -2183,6 +2180,32 @@ static_assert(((kFixRawE >> 52) * kRawInv) % 4096 == 1 && (kFixRawE << 12) == 0,
 __device__ __forceinline__ uint32_t gen_raw_count(uint64_t raw) {
   const uint32_t n = (static_cast<uint32_t>(raw >> 52) * kRawInv) & 4095u;
   return n <= kRawCountMax ? n : 0u;
+}
+
+// The same for a larger bucket, by what else the sum says of n: its terms lie within e^(+-w) of 2^40 (w:
+// one bucket's width, and a little for the bucket index's rounding), so f = F 2^52 + (its low 52 bits)
+// puts n into an interval of 2 w f 2^-40, and the top 12 bits, n (kFixRawE >> 52) + F mod 4,096, name it
+// there for each F. missing: how many elements the counts above leave out, which bounds n. With one F that
+// fits, n is exact. With none or several 0 is returned, and a count that is not exact is again too low (one
+// of at most kRawCountMax at F = 0 lies below the 4,030 that any larger F implies).
+__device__ __forceinline__ uint32_t gen_raw_count_any(uint64_t raw, double w, uint32_t missing) {
+  if (raw == 0ull) return 0u;
+  const double lo = 1.0 - 1.001 * w, hi = 1.0 + 1.02 * w;  // about e^(+-w), w <= 1/64
+  const double low = static_cast<double>(raw & ((1ull << 52) - 1ull)) * kFixUnit;
+  const uint32_t top = static_cast<uint32_t>(raw >> 52);
+  const uint32_t most = missing + gen_raw_count(raw);
+  uint32_t n = 0u;
+  int found = 0;
+  for (uint32_t F = 0u; F <= (most >> 12) + 1u; ++F) {  // f 2^-40 below 1.017 n, n below 2^18
+    const double f = low + 4096.0 * F;
+    const uint32_t from = static_cast<uint32_t>(fmax(f * lo - 1.0, 1.0)), to = min(static_cast<uint32_t>(f * hi + 1.0), most);
+    const uint32_t c = from + (((top - F) * kRawInv - from) & 4095u);
+    if (c > to) continue;
+    if (F == 0u && c <= kRawCountMax) return c;
+    n = c;
+    ++found;
+  }
+  return found == 1 ? n : 0u;
 }
 
 struct GenPart {
@@ -2687,8 +2710,28 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
         }
       }
       const double wq = table_width(g.qs, P.temp);
-      double ms = 0.0;
-      uint32_t cs = 0;
+      double ms = 0.0, im, em;
+      uint32_t cs = 0, ic, ec, total;
+      auto totals = [&]() __attribute__((always_inline)) {  // over the row's buckets, and before this thread's
+        im = wave_incl_scan_f64(ms);
+        ic = wave_incl_scan(cs);
+        if (lane == 63) {
+          sh.wm[w] = im;
+          sh.wc[w] = ic;
+        }
+        __syncthreads();
+        em = ms_before = 0.0;
+        ec = total = 0u;
+#pragma unroll
+        for (int i = 0; i < GenShared<NT>::kGenNW; ++i) {
+          if (i == w) {
+            em = ms_before;
+            ec = total;
+          }
+          ms_before += sh.wm[i];
+          total += sh.wc[i];
+        }
+      };
 #pragma unroll
       for (int i = 0; i < BP; ++i) {
         const int b = b0 + i;
@@ -2703,23 +2746,29 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
         ms += rm[i];
         cs += rc[i];
       }
-      const double im = wave_incl_scan_f64(ms);
-      const uint32_t ic = wave_incl_scan(cs);
-      if (lane == 63) {
-        sh.wm[w] = im;
-        sh.wc[w] = ic;
-      }
-      __syncthreads();
-      double em = 0.0;
-      uint32_t ec = 0u, total = 0u;
-#pragma unroll
-      for (int i = 0; i < GenShared<NT>::kGenNW; ++i) {
-        if (i == w) {
-          em = ms_before;
-          ec = total;
+      totals();
+      if (__builtin_expect(sgpr_u32(total) != static_cast<uint32_t>(V), 0)) {
+        // a bucket of thousands: every count from all that its sum says, a bucket at a time through LDS
+        const unsigned long long* hr = a.p_hfix + static_cast<size_t>(row) * kGenBuckets;
+        const uint32_t missing = static_cast<uint32_t>(V) - sgpr_u32(total);
+        for (int b = b0; b < b0 + BP; ++b) {
+          const uint64_t raw = hr[b];
+          const bool last = capped && b == kGenBuckets - 1;
+          const uint32_t n = last ? static_cast<uint32_t>(oc) : gen_raw_count_any(raw, wq, missing);
+          sh.cnt0[b] = n;
+          sh.mass0[b] = last ? om : exp_tab(-static_cast<double>(b | 1) * wq) * (static_cast<double>(raw - n * kFixRawE) * kFixUnit);
         }
-        ms_before += sh.wm[i];
-        total += sh.wc[i];
+        ms = 0.0;
+        cs = 0u;
+#pragma unroll
+        for (int i = 0; i < BP; ++i) {
+          rc[i] = sh.cnt0[b0 + i];
+          rm[i] = sh.mass0[b0 + i];
+          ms += rm[i];
+          cs += rc[i];
+        }
+        __syncthreads();
+        totals();
       }
       em += im - ms;
       ec += ic - cs;
@@ -2740,7 +2789,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
       }
       if (k < V) wave_claim_min(&sh.ints[0], first < kGenBuckets, first);
       __syncthreads();
-      if (sgpr_u32(total) != static_cast<uint32_t>(V)) {  // a bucket's count was not decoded
+      if (sgpr_u32(total) != static_cast<uint32_t>(V)) {  // a bucket's count is still not known
         alone = true;
         if (part.part != 0) return;
         __syncthreads();
@@ -2917,8 +2966,9 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
   };
   // A flat row has every element in bucket 0 with the numerator exp(0) = 1 (fixed point 2^40, numer_fix): its
   // histogram, min-p count and prefix are known without the pass, whose atomics would all meet on
-  // one address (256 x 151,936 zeros, top-p .9: 1,063 to 809 us per call, against 115 us for rows
-  // of normal values; the selects after it refine that one bucket over the row's indices).
+  // one address, and so is the element that a running mass reaches (256 x 151,936 zeros, top-p .9: 337
+  // us per call when the selects refined that one bucket over the row's indices, 37 now; 91 for rows of
+  // normal values).
   // With a top-k cut the kept elements are the first k by index (equal values rank by index).
   // one instance per combination: no per-element branches beyond the ones asked for
   if (!alone) {  // SPLIT: k_gen_hist took the pass
@@ -3163,6 +3213,16 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
   auto mass_select = [&](double target) -> Sel {
     Sel s;
     if (!(target > 0.0)) return first_element();
+    if (flat) {  // element j, of index j, brings the weight to j + 1
+      const int n = sgpr_i32(static_cast<int>(sh.cnt0[0]));
+      const int j = static_cast<int>(fmin(ceil(target), static_cast<double>(n))) - 1;
+      s.found = target <= static_cast<double>(n);
+      s.ck = comp(comp_key(mxc), static_cast<uint32_t>(j));
+      s.rank = j;
+      s.before = static_cast<double>(j);
+      s.incl = static_cast<double>(j + 1);
+      return s;
+    }
     const int qb = find_bucket(target);
     if (qb == kGenBuckets) {
       s.found = false;
