@@ -955,9 +955,11 @@ def test_general_split_large_buckets(monkeypatch, parts):
         assert Run(ctx, lg, V.params_array(n=1, **dict(dict(temp=0.8, top_k=0, top_p=1.0, repeat=1.1, repeat_last=0, seed=3), **f)), h, off).report()[1] == 0
 
 
-def test_graph_capture_after_a_larger_warm_up():
-    """The split kernels' scratch is sized by any call at a shape or a larger one: after one call of a
-    wide batch on another path, smaller batches of every split path are captured and replayed."""
+@pytest.mark.parametrize("warm", ["larger", "same"])
+def test_graph_capture_after_a_larger_warm_up(warm):
+    """After one call of a wide batch on another path, smaller batches are captured and replayed: as they
+    are (larger: the split kernels have no scratch, which a capture cannot allocate, so the call takes
+    its route without them), and after a call of their own (same: every split path is captured)."""
     import torch
 
     ctx = V.Context(0)
@@ -977,6 +979,8 @@ def test_graph_capture_after_a_larger_warm_up():
             pr = V.to_device_params(rows)
         x = torch.randn(B, Vv, generator=g, device="cuda")
         out = torch.empty(B, dtype=torch.int32, device="cuda")
+        if warm == "same":
+            ctx.pick_batch(x, pr, out=out)
         torch.cuda.synchronize()
         st, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
         with torch.cuda.stream(st):
@@ -984,9 +988,41 @@ def test_graph_capture_after_a_larger_warm_up():
                 ctx.pick_batch(x, pr, out=out, stream=st)
         torch.cuda.synchronize()
         for step in range(3):
-            log("capture after a larger warm-up", B, f, step)
+            log("capture after a larger warm-up", warm, B, f, step)
             x.copy_(torch.randn(B, Vv, generator=g, device="cuda"))
             torch.cuda.synchronize()
             graph.replay()
             torch.cuda.synchronize()
             assert torch.equal(out, mode_ctx("rows").pick_batch(x, pr)), (B, f, step)
+
+
+def test_scratch_on_demand():
+    """A context holds the split kernels' scratch only once a call has taken them: the first call of a
+    batch too wide for a split allocates the exact redo's sort slots (256 of 1 MiB here) and nothing
+    of the 13 MB that a split of the largest batch it could take at this vocabulary would need, and the
+    fused head pick allocates its lists and no logits of the other route's smaller batches."""
+    import torch
+
+    B, Vv = 256, 65536
+    x = torch.randn(B, Vv, device="cuda")
+    out = torch.empty(B, dtype=torch.int32, device="cuda")
+
+    def taken(call):
+        ctx = V.Context(0)
+        torch.cuda.synchronize()
+        free = torch.cuda.mem_get_info()[0]
+        call(ctx)
+        torch.cuda.synchronize()
+        return free - torch.cuda.mem_get_info()[0]
+
+    off = V.Params(temp=1.0, top_k=0, top_p=0.95, min_p=0.0, repeat=1.0, repeat_last=0, seed=4)
+    log("scratch on demand, general rows")
+    assert taken(lambda c: c.pick_batch(x, off, out=out)) <= (256 << 20) + (4 << 20)
+    small = V.Params(temp=1.0, top_k=50, top_p=0.95, min_p=0.0, repeat=1.0, repeat_last=0, seed=4)
+    log("scratch on demand, row mode")
+    assert taken(lambda c: c.pick_batch(x, small, out=out)) == 0
+    hidden = torch.randn(64, 64, device="cuda").bfloat16()
+    head = (torch.randn(131072, 64, device="cuda") * 0.3).bfloat16()
+    o = torch.empty(64, dtype=torch.int32, device="cuda")
+    log("scratch on demand, fused head")
+    assert taken(lambda c: c.head_pick(hidden, head, small, out=o)) <= 64 * 131072 * 8 + (6 << 20)

@@ -162,7 +162,7 @@ namespace {
 struct GenParts {
   int P;         // 0: no split
   size_t rows;   // what the scratch is sized for: the rows and parts of this batch or of any smaller one
-  size_t slots;  // at this vocabulary, so that a context warmed up at a batch can serve smaller ones
+  size_t slots;  // at this vocabulary, whatever its parameters
 };
 
 struct Plan {
@@ -174,8 +174,7 @@ struct Plan {
   bool any_general, any_smallk, any_finish;
   bool no_rows_kernel;  // row mode with every row general: k_general alone takes the batch
   bool side_general;    // row mode with per-row parameters: k_general next to k_rows, on a side stream
-  GenParts gen;         // row mode: parts per general row at this shape; its scratch is sized whatever
-                        // the parameters, as the exact redo's is
+  GenParts gen;         // row mode: parts per general row at this shape
   bool gen_split;       // ... taken by this call's general rows
 };
 
@@ -263,7 +262,8 @@ GenParts general_parts(int B, int V, bool per_row, bool forced, long long forced
   if (forced) return {static_cast<int>(P), static_cast<size_t>(B), static_cast<size_t>(B * P)};
   const long long rows = std::min<long long>(B, V / kGenSplitLogits);
   if (rows < 1 || pmax < 2) return {};
-  const long long slots = std::max({rows * std::max(pmin, std::min(tmin, tmax)), rows * P, static_cast<long long>(std::sqrt(rows * (V / 64.0)) + 0.5 * rows) + 1});
+  const long long slots = std::max({rows * pmin, rows * P, std::min(rows * std::min(tmin, tmax), kMixedParts),
+                                    static_cast<long long>(std::sqrt(rows * (V / 64.0)) + 0.5 * rows) + 1});
   const bool fits = !per_row || B * P <= kMixedParts;
   return {rows == B && P >= 2 && fits ? static_cast<int>(P) : 0, static_cast<size_t>(rows), static_cast<size_t>(slots)};
 }
@@ -297,12 +297,13 @@ SplitScratch split_scratch(const GenParts& gp, int words) {
 }
 
 // Slice shape: enough workgroups to fill the chip (>= 2048), slices of 256*EPT elements, and no
-// more slices than the small-k merge can hold (S * k <= kMergeCap).
-Plan plan(const vsmp_ctx* ctx, int B, int V, const vsmp_params* hostp) {
+// more slices than the small-k merge can hold (S * k <= kMergeCap). split: false plans without the split kernels
+// (a captured call that finds no scratch for them).
+Plan plan(const vsmp_ctx* ctx, int B, int V, const vsmp_params* hostp, bool split = true) {
   Plan pl{};
   const int fm = ctx->mode;
   const int cus = ctx->cus;
-  if (hostp && (fm == -1 || fm == 2)) {
+  if (split && hostp && (fm == -1 || fm == 2)) {
     const int path = path_host(*hostp, V, true);
     const int k = (hostp->top_k > 0 && hostp->top_k < V) ? hostp->top_k : V;
     const int P = path == kPathGreedy ? split_parts(B, V, cus, fm == 2, ctx->split_p)
@@ -347,7 +348,7 @@ Plan plan(const vsmp_ctx* ctx, int B, int V, const vsmp_params* hostp) {
     pl.side_general = !hostp;
     // k <= kGenCap or top-k off: the split takes the row (with per-row parameters it leaves a larger
     // k to one of their workgroups after the histogram)
-    if (pl.any_general && fm != 1) {
+    if (split && pl.any_general && fm != 1) {
       pl.gen = general_parts(B, V, !hostp, fm == 2, ctx->split_p);
       pl.gen_split = pl.gen.P > 0 && (!hostp || hostp->top_k <= kGenCap || hostp->top_k >= V);
       if (pl.gen_split) {  // one workgroup per part of every row, on the caller's stream
@@ -456,16 +457,18 @@ KArgs batch_args(const float* logits, int B, int V, long long ld, const vsmp_par
   return a;
 }
 
-// The split kernels' scratch. Which batches they take depends on k as well as on the shape, so every
-// call sizes it for whatever split the device can be given by default (about 1 MiB): a call at a shape,
-// with any parameters, then serves a graph capture at that shape or a smaller one. rows, slots: what a
-// call itself needs beyond that (pinned modes).
-bool split_rows_scratch(vsmp_ctx* ctx, size_t rows, size_t slots, hipStream_t st) {
-  const size_t most = 2 * static_cast<size_t>(ctx->cus);
-  // 256 rows more than needed: the tickets then lie 6 KiB behind the slots, on other memory channels
-  // (4 KiB apart, a greedy batch of 64 rows took 12.18 against 12.07 us)
-  return grow(ctx->g_rows, ctx->n_grows, 2 * (std::max(rows, most) + 256), true, "scratch", st) &&
-         grow(ctx->t_scr, ctx->n_tscr, std::max(slots, most) * (kKmax + 1), false, "scratch", st);
+// The split greedy and small-k kernels' scratch: at least (about 1 MiB) for whatever the device can be
+// given by default, so that one such call sizes it for all. rows, slots: what a call itself needs.
+// 256 rows more than needed: the tickets then lie 6 KiB behind the slots, on other memory channels
+// (4 KiB apart, a greedy batch of 64 rows took 12.18 against 12.07 us).
+size_t split_row_words(const vsmp_ctx* ctx, size_t rows) { return 2 * (std::max(rows, 2 * static_cast<size_t>(ctx->cus)) + 256); }
+size_t split_list_words(const vsmp_ctx* ctx, size_t slots) { return std::max(slots, 2 * static_cast<size_t>(ctx->cus)) * (kKmax + 1); }
+
+bool capturing(hipStream_t st) {
+  hipStreamCaptureStatus c = hipStreamCaptureStatusNone;
+  if (!st) return false;  // the null stream cannot be captured
+  if (hipStreamIsCapturing(st, &c) != hipSuccess) (void)hipGetLastError();
+  return c != hipStreamCaptureStatusNone;
 }
 
 int launch_batch(vsmp_ctx* ctx, const float* logits, int B, int V, long long ld, const vsmp_params* params,
@@ -475,12 +478,31 @@ int launch_batch(vsmp_ctx* ctx, const float* logits, int B, int V, long long ld,
   if (check_batch(logits, B, V, ld, params, hist, hist_off, u_mode, u, rng_state, out, dbg) != 0) return -1;
   KArgs a = batch_args(logits, B, V, ld, params, params_per_row, hist, hist_off, u_mode, u, rng_state, counter, out, dbg,
                        hist_len, slot);
-  const Plan pl = plan(ctx, B, V, params_per_row ? nullptr : params);
+  const vsmp_params* hostp = params_per_row ? nullptr : params;
+  const int words = a.words;
+  Plan pl = plan(ctx, B, V, hostp);
+  // The split kernels' scratch is sized by the calls that take them (a context of wide batches would hold
+  // some 20 MB for nothing, and its first call take 10 to 20 us longer). A capture cannot allocate: a
+  // captured call that finds too little takes the route without them, whose ids are the same.
+  SplitScratch ss{};
+  if (pl.gen_split) ss = split_scratch(pl.gen, words);
+  const size_t parts = static_cast<size_t>(B) * static_cast<size_t>(pl.S);
+  const bool sized = pl.split ? ctx->n_grows >= split_row_words(ctx, B) && (!pl.topk || ctx->n_tscr >= split_list_words(ctx, parts))
+                              : !pl.gen_split || ctx->n_pscr >= ss.bytes;
+  if (!sized) {
+    if (capturing(st))
+      pl = plan(ctx, B, V, hostp, false);
+    else if (pl.split) {
+      if (parts > static_cast<size_t>(INT32_MAX) / kKmax) return set_error("vsmp: batch too large");
+      if (!grow(ctx->g_rows, ctx->n_grows, split_row_words(ctx, B), true, "scratch", st) ||
+          (pl.topk && !grow(ctx->t_scr, ctx->n_tscr, split_list_words(ctx, parts), false, "scratch", st)))
+        return -1;
+    } else if (!grow(ctx->p_scr, ctx->n_pscr, ss.bytes, false, "scratch", st))
+      return -1;
+  }
   const size_t slots = static_cast<size_t>(B) * static_cast<size_t>(pl.S);
   if (slots > static_cast<size_t>(INT32_MAX) / kKmax) return set_error("vsmp: batch too large");
-  const int words = a.words;
   const bool slices = !pl.rows && !pl.split;
-  if (!slices && !split_rows_scratch(ctx, pl.split ? static_cast<size_t>(B) : 0, pl.split && pl.topk ? slots : 0, st)) return -1;
   if (slices && (!grow(ctx->s_cnt, ctx->n_cnt, slots, false, "scratch", st) ||
                  !grow(ctx->s_npen, ctx->n_npen, slots, false, "scratch", st) ||
                  !grow(ctx->s_max, ctx->n_max, slots, false, "scratch", st) ||
@@ -499,11 +521,6 @@ int launch_batch(vsmp_ctx* ctx, const float* logits, int B, int V, long long ld,
     return -1;
   if (pl.any_general && !pl.rows && !grow(ctx->s_bits, ctx->n_bits, static_cast<size_t>(B) * words, false, "scratch", st))
     return -1;
-  SplitScratch ss{};
-  if (pl.gen.rows > 0) {
-    ss = split_scratch(pl.gen, words);
-    if (!grow(ctx->p_scr, ctx->n_pscr, ss.bytes, false, "scratch", st)) return -1;
-  }
   if (a.pen_bits) {  // diagnostics: the kernels store or OR each row's penalised ids into zeroed bitmaps
     launch_zero_u32(a.pen_bits, static_cast<long long>(B) * words, st);
     if (!hip_ok(hipGetLastError(), "zero-fill launch")) return -1;
@@ -711,9 +728,13 @@ int head_pick(vsmp_ctx* ctx, const void* hidden, long long ldh, const void* head
   long long fld = ldl;
   if (!full && (whole || params_per_row)) {
     fld = (static_cast<long long>(V) + 3) & ~3LL;
-    if (!grow(ctx->h_full, ctx->n_full, static_cast<size_t>(B) * static_cast<size_t>(fld), false, "head scratch", st))
-      return -1;
-    full = ctx->h_full;
+    const size_t need = static_cast<size_t>(B) * static_cast<size_t>(fld);
+    if (whole && need > ctx->n_full && need <= 2 * ctx->n_rcand) {
+      full = reinterpret_cast<float*>(ctx->h_rcand);  // the fused route's lists, which this call leaves alone
+    } else {
+      if (!grow(ctx->h_full, ctx->n_full, need, false, "head scratch", st)) return -1;
+      full = ctx->h_full;
+    }
   }
   HeadArgs h = head_args(hidden, ldh, head, ldw, B, V, D);
   if (whole) {  // the head, then the batched pick (every row of a shared general batch samples whole)
@@ -728,13 +749,6 @@ int head_pick(vsmp_ctx* ctx, const void* hidden, long long ldh, const void* head
   }
   const int n0 = std::min(kHeadProbe, V);
   const int tile = head_tile(B, false);
-  // fewer rows of this head take the other route: its logits and the pick's scratch, sized here too
-  if (!params_per_row && ctx->head_route < 0) {
-    const size_t rows = static_cast<size_t>(kHeadFuseLogits / V);
-    if (!grow(ctx->h_full, ctx->n_full, rows * static_cast<size_t>((V + 3) & ~3), false, "head scratch", st) ||
-        !split_rows_scratch(ctx, 0, 0, st))
-      return -1;
-  }
   if (!grow(ctx->h_tk, ctx->n_tk, static_cast<size_t>(B), false, "head scratch", st) ||
       !grow(ctx->h_rmode, ctx->n_rmode, static_cast<size_t>(B), false, "head scratch", st) ||
       !grow(ctx->h_rcand, ctx->n_rcand, static_cast<size_t>(B) * static_cast<size_t>(V), false, "head scratch", st) ||
