@@ -19,9 +19,10 @@ KAT = np.array([0.1, 3.0, 2.9, -1.0, 0.0], np.float32)
 
 @pytest.fixture(params=["slices", "rows", "split"])
 def mode(request):
-    """Each decomposition on the same inputs: slices + merge, one workgroup per row, and (for
-    greedy and small-k batches with shared parameters; other batches take the default) rows cut
-    into parts finished by their last part. A context reads VSMP_MODE when it is created."""
+    """Each decomposition on the same inputs: slices + merge, one workgroup per row, and rows cut into
+    parts finished by their last part (vocabularies beyond the row kernel take slices, and per-row
+    batches of more than 2^18 logits and shared top-k above 1,024 one workgroup per general row). A
+    context reads VSMP_MODE when it is created."""
     return request.param
 
 
@@ -601,14 +602,17 @@ def test_vocabulary_beyond_the_row_kernel(ctx):
     Run(ctx, lg, p, h, off, cand_cap=64).report()
 
 
-def test_graph_capture_and_replay(ctx):
+@pytest.mark.parametrize("dmode", [None, "rows"])
+def test_graph_capture_and_replay(dmode):
     """vsmp_pick_batch captured into a HIP graph (after one eager call has sized the scratch) and
     replayed with new logits and draws copied into the captured buffers between replays: every
-    replay equals the eager call on the same inputs, for a greedy batch (split mode), a top-k batch
-    (row mode), a general batch (k_general alone) and a batch with per-row parameters mixing top-k
-    and general rows (k_rows, and k_general on a stream forked from and joined back to the
-    capturing one), all four in one graph."""
+    replay equals the eager call on the same inputs, for a greedy batch, a top-k batch, a general batch
+    and a batch with per-row parameters mixing top-k and general rows, all four in one graph. By default
+    each takes its split kernels; in row mode k_rows, k_general alone, and for the per-row batch k_rows
+    with k_general on a stream forked from and joined back to the capturing one."""
     import torch
+
+    ctx = mode_ctx(dmode)
 
     rng = np.random.default_rng(51)
     B, Vv = 8, 30000
@@ -817,14 +821,13 @@ def test_general_path_all_rows_marked(ctx):
     assert (run.info["keep"] == run.o_info["keep"]).all() and (run.ids == run.o_ids).all()
 
 
-@pytest.mark.parametrize("parts", [1, 3, 64])
-@pytest.mark.parametrize("Vv", [1030, 20003, 70001])
+@pytest.mark.parametrize("parts,Vv", [(1, 1030), (3, 20003), (16, 20003), (5, 70001), (16, 70001)])
 def test_general_split_parts(monkeypatch, parts, Vv):
-    """General rows cut into parts (per-row parameters, so every plan in one batch): parts of several
-    register chunks, a last part of a few elements, empty parts, top-k lists of 257 to 1,024 elements
-    and beyond, a bucket of 4,000 to 5,000 equal values (whose count the raw sums cannot give), min-p
-    prefixes, draws without a cut, rows that are flat, cold, tied in steps, all -inf but one, and
-    the reference's draw stream advanced once per row."""
+    """General rows cut into parts, per-row parameters, so every plan in one batch (at most 16 parts, each
+    held in registers): one part, parts of unequal size, top-k lists of 257 to 1,024 elements
+    and beyond, a bucket of 4,000 to 5,000 equal values (whose count the raw sums do not hold), min-p
+    prefixes, draws without a cut, rows that are flat, cold, tied in steps, all -inf but one, greedy and
+    small-k rows among them, and the reference's draw stream advanced once per row."""
     import torch
 
     monkeypatch.setenv("VSMP_MODE", "split")
@@ -833,7 +836,8 @@ def test_general_split_parts(monkeypatch, parts, Vv):
     rng = np.random.default_rng(parts * 100003 + Vv)
     kinds = ["normal", "flat", "steps", "equal", "cold", "neginf", "spiky"]
     opts = [dict(top_p=0.95), dict(top_p=1.0), dict(top_p=0.9, min_p=0.02), dict(top_p=1.0, min_p=1e-4), dict(top_k=257, top_p=0.9),
-            dict(top_k=1000, min_p=0.01), dict(top_k=1024, top_p=0.5), dict(top_k=Vv - 1, top_p=0.8), dict(top_p=0.01)]
+            dict(top_k=1000, min_p=0.01), dict(top_k=1024, top_p=0.5), dict(top_k=Vv - 1, top_p=0.8), dict(top_p=0.01),
+            dict(temp=0.0), dict(top_k=1), dict(top_k=40, top_p=0.9), dict(top_k=256, min_p=0.01)]
     B = len(kinds) * len(opts)
     lg = rng.normal(0, 1.0, (B, Vv)).astype(np.float32)
     p = np.zeros(B, V.SAMPLING_DTYPE)
@@ -852,7 +856,7 @@ def test_general_split_parts(monkeypatch, parts, Vv):
             n = min(Vv - 5, int(rng.integers(4000, 5000)))
             lg[r, rng.permutation(Vv)[:n]] = 0.25
         elif kind == "cold":
-            p[r]["temp"] = 0.01
+            p[r]["temp"] = min(p[r]["temp"], 0.01)
         elif kind == "neginf":
             lg[r] = -np.inf
             lg[r, rng.integers(0, Vv)] = 2.0
@@ -877,6 +881,62 @@ def test_general_split_parts(monkeypatch, parts, Vv):
         states.append(st.cpu())
         ids.append(torch.stack(out))
     assert torch.equal(states[0], states[1]) and torch.equal(ids[0], ids[1])
+
+
+@pytest.mark.parametrize("parts,Vv", [(2, 70001), (3, 70001), (17, 70001), (64, 70001), (64, 66529), (8, 500003)])
+def test_general_split_shared_parts(monkeypatch, parts, Vv):
+    """General rows of one set of parameters cut into 2 to 64 parts: parts of several register chunks (more
+    than 4,096 groups of four: 2 and 3 parts of 70,001 logits, 8 of 500,003), a last part of one
+    element (64 of 66,529), an empty one (64 of 70,001), with every plan of the last launch."""
+    monkeypatch.setenv("VSMP_MODE", "split")
+    monkeypatch.setenv("VSMP_SPLIT_P", str(parts))
+    groups = (Vv + 3) // 4
+    share = ((groups + parts - 1) // parts + 7) // 8 * 8  # the kernels' rule: whole words of the penalty bitmap
+    last = max(0, Vv - 4 * share * (parts - 1))
+    assert (share > 4096) == (parts < 17) and last == {(64, 66529): 1, (64, 70001): 0}.get((parts, Vv), last) and (last > 0 or Vv == 70001)
+    ctx = V.Context(0)
+    rng = np.random.default_rng(parts)
+    lg = rng.normal(0, 1.0, (6, Vv)).astype(np.float32)
+    lg[1] = np.round(lg[1] * 64) / 64
+    lg[2, rng.integers(0, Vv, 12)] += 7.0
+    lg[3] = -np.inf
+    lg[3, rng.permutation(Vv)[:50]] = rng.normal(0, 1.0, 50)
+    lg[4, -3:] = 9.0  # the row's end holds its maximum
+    lg[5, ::7] = 0.5
+    h, off = csr([rng.integers(-2, Vv + 2, int(rng.integers(0, 3000))) for _ in range(6)])
+    for f in (dict(top_p=0.95), dict(top_p=0.01), dict(), dict(top_p=0.9, min_p=0.02), dict(min_p=1e-4), dict(top_k=257, top_p=0.9),
+              dict(top_k=1024, min_p=0.01), dict(temp=0.02, top_p=0.99)):
+        log("general split, shared", parts, Vv, f)
+        p = V.params_array(n=1, **dict(dict(temp=0.9, top_k=0, top_p=1.0, repeat=1.2, repeat_last=0, seed=41), **f))
+        run = Run(ctx, lg, p, h, off)
+        assert (run.info["path"] == V.PATH_GENERAL).all() and run.report()[1] == 0
+
+
+@pytest.mark.parametrize("Vv", [49152, 151936, 262144])
+def test_one_row_picks_by_name(Vv):
+    """The default plan of one row: nucleus picks and top-k of 257 to 1,024 (28, 49 and 64 parts), top-k
+    2,000 (one workgroup), small k and greedy, from device memory and from host memory, whose kernels read
+    the row over PCIe."""
+    import torch
+
+    ctx = V.Context(0)
+    rng = np.random.default_rng(Vv)
+    lg = rng.normal(0, 2.0, (1, Vv)).astype(np.float32)
+    lg[0, rng.integers(0, Vv, 16)] += 6.0
+    hist = rng.integers(0, Vv, 300).astype(np.int32)
+    off = np.array([0, 300], np.int32)
+    for f in (dict(top_k=0, top_p=0.95), dict(top_k=0, top_p=1.0), dict(top_k=0, top_p=0.9, min_p=0.02), dict(top_k=300), dict(top_k=1000),
+              dict(top_k=2000), dict(top_k=40), dict(top_k=100), dict(top_k=256), dict(temp=0.0)):
+        fields = dict(dict(temp=0.8, top_k=40, top_p=0.95, min_p=0.0, repeat=1.1, repeat_last=0, seed=8), **f)
+        for u in (0.02, 0.37, 0.93):
+            log("one row", Vv, f, u)
+            run = Run(ctx, lg, V.params_array(n=1, **fields), hist, off, u=[u])
+            assert run.report()[1] == 0
+            ids = torch.empty(1, dtype=torch.int32, device="cuda")
+            d = [torch.from_numpy(np.ascontiguousarray(t)).cuda() for t in (lg, hist, off, np.array([u]))]
+            ctx.pick_batch(d[0], V.Params(**fields), d[1], d[2], V.U_SUPPLIED, d[3], out=ids)  # without diagnostics
+            assert int(ids.cpu()[0]) == run.ids[0]
+            assert ctx.pick_host(lg[0], V.Params(**fields), hist, u) == run.ids[0]
 
 
 @pytest.mark.parametrize("per_row", [False, True])
