@@ -2683,11 +2683,14 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
   const bool flat = comp_key(mxc) == static_cast<uint32_t>(mnk) && isfinite(g.mx);
   // top-k prefix when 256 < k < V: the k-th element's composite, once it is known
   g.ckk = flat && k < V ? comp(comp_key(mxc), static_cast<uint32_t>(k - 1)) : 0ull;
-  // SPLIT: alone = the rest of the row is taken by this workgroup by itself (part 0; the others have
-  // returned), pass by pass as without the split. Every part decides it from the same values.
+  // SPLIT: alone = the rest of the row is taken by this workgroup by itself (the row's chief; the others
+  // have returned), pass by pass as without the split. Every part decides it from the same values. The
+  // chiefs are different parts: workgroups go round the eight XCDs, and the first parts of rows in 16
+  // parts all meet on one (40 x 262,144, per-row top-k 2,000: 259 us).
   bool alone = !SPLIT || flat;
+  const bool chief = !SPLIT || part.part == row % a.P;
   if constexpr (SPLIT)
-    if (alone && part.part != 0) return;
+    if (alone && !chief) return;
   bool by_hist = false;  // ... with the parts' histogram, once the k-th element is found in its bucket
   constexpr int BP = kGenBuckets / kGenThreads;
   static_assert(BP % 4 == 0, "a thread's buckets are read as 16-byte vectors");
@@ -2791,7 +2794,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
       __syncthreads();
       if (sgpr_u32(total) != static_cast<uint32_t>(V)) {  // a bucket's count is still not known
         alone = true;
-        if (part.part != 0) return;
+        if (!chief) return;
         __syncthreads();
       }
     }
@@ -2802,7 +2805,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
         // and 158 in one workgroup of 1,024 threads that took every pass).
         qk = min(sgpr_i32(sh.ints[0]), kGenBuckets - 1);
         by_hist = k > kGenCap || (capped && qk == kGenBuckets - 1) || sgpr_u32(sh.cnt0[qk]) > kGenPartList;
-        if (by_hist && part.part != 0) return;
+        if (by_hist && !chief) return;
         __syncthreads();
       }
     }
@@ -3384,7 +3387,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
       if (!plan) {
         // the min-p prefix, which k_gen_hist listed, or a plan whose lists do not fit: one workgroup
         // ends the row
-        if (part.part != 0) return;
+        if (!chief) return;
         alone = true;
         __syncthreads();
         if (tid < 4) sh.fb[tid] = kGenBuckets;
