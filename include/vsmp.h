@@ -172,8 +172,9 @@ VSMP_API int vsmp_head_logits(vsmp_ctx* ctx, const void* hidden, long long ldh, 
 /* The LM head and the pick in one call: the ids vsmp_pick_batch would pick from the logits that
  * vsmp_head_logits writes. Replaces Session's head product (src/session.cpp:169) followed by
  * Sampler::pick (src/sampler.cpp:50-109) on its row; the reference has no such fused call.
- * Fused (31 to 64 rows of a head of 151,936 columns and in proportion, from 120,000 columns on, where
- * it measured faster; 16 to 64 rows with per-row parameters; any batch with VSMP_HEAD_ROUTE=fused set when the context is created): greedy and small-k rows (temp <= 0, or
+ * Fused (up to 64 rows, from 45 rows of a head of 151,936 columns on and in proportion, more where the
+ * probe's columns save the product a round of tiles, where it measured faster; 16 to 64 rows with per-row
+ * parameters; any batch with VSMP_HEAD_ROUTE=fused set when the context is created): greedy and small-k rows (temp <= 0, or
  * 0 < top_k <= 256) keep only the columns whose logit reaches a per-row bound (the k-th largest
  * penalised logit of the first 4096 columns) and never write their logits; other rows (top-k off
  * or above 256) are written whole and sampled by the general path. Other batches (or

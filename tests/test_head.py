@@ -301,3 +301,18 @@ def test_head_pick_routes_agree():
             assert np.array_equal(fi[f], wi[f]), (prm, f)
         assert np.allclose(fi["sum"], wi["sum"], rtol=1e-12, atol=0) and np.allclose(fi["tot"], wi["tot"], rtol=1e-12, atol=0)
         assert np.array_equal(fc, wc), prm
+
+@pytest.mark.parametrize("B,Vv,D", [(44, 151936, 64), (45, 151936, 64), (45, 33000, 4096), (46, 33000, 4096), (31, 133000, 64), (32, 133000, 64), (33, 67000, 2048)])
+def test_head_pick_on_both_sides_of_the_route(B, Vv, D):
+    """Shapes on either side of the lines between the fused and the whole route (with and without a round
+    of tiles that the probe's columns save), each at its own route and at both pinned ones: the same ids."""
+    import torch
+
+    g = torch.Generator(device="cuda").manual_seed(B)
+    hidden = torch.randn(B, D, generator=g, device="cuda").bfloat16()
+    head = (torch.randn(Vv, D, generator=g, device="cuda") * (2.5 / D ** 0.5)).bfloat16()
+    for k in (40, 256):
+        p = V.Params(temp=0.9, top_k=k, top_p=0.95, min_p=0.01, repeat=1.0, repeat_last=0, seed=6)
+        log("head routes", B, Vv, D, k)
+        ids = [mode_ctx(None, r).head_pick(hidden, head, p).cpu() for r in (None, "fused", "whole")]
+        assert torch.equal(ids[0], ids[1]) and torch.equal(ids[0], ids[2])

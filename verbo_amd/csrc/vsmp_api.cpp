@@ -710,17 +710,26 @@ int head_pick(vsmp_ctx* ctx, const void* hidden, long long ldh, const void* head
   // The route. Fused, the call pays fixed stages (the probe's product, the bound, the finish: about 25
   // us) against the logits it does not write and the sampler's read of them it saves; whole, the
   // head's logits are written and the batched pick runs on them: the same ids and diagnostics, as the
-  // fused route is built to give. Measured (fused / whole, us, D = 896, top-k 20, 64 and 100, shared
-  // parameters): 151,936 columns 24 rows 74.2 / 69.9, 76.1 / 75.4, 81.0 / 79.3; 32 rows 75.0 / 73.6, 77.0
-  // / 78.5, 81.7 / 83.2; 64 rows 81.0 / 85.6, 83.0 / 89.0, 88.7 / 93.1; 96 rows at top-k 50 106.4 / 102.9;
-  // 110,000 columns 16 to 64 rows 62.6 to 74.5 / 52.3 to 73.5, and whole further ahead on fewer (50,257:
-  // 42.5 to 51.6 / 32.0 to 43.7). So fused for 31 to 64 rows of 151,936 columns and in proportion, not
-  // below 120,000. It does not depend on k, so that a call at a shape sizes its scratch. With per-row
-  // parameters (some rows general or not) it is taken for 16 to 64 rows.
-  constexpr int kHeadFuseMin = 16, kHeadFuseMax = 64, kHeadFuseV = 120000;
-  constexpr long long kHeadFuseLogits = 4600000;
-  const bool fuse_shape = B >= kHeadFuseMin && B <= kHeadFuseMax &&
-                          (params_per_row || (V >= kHeadFuseV && static_cast<long long>(B) * V >= kHeadFuseLogits));
+  // fused route is built to give. Measured (fused / whole, us, top-k 50, shared parameters; D = 896, 2,048,
+  // 4,096): 151,936 columns 24 rows 71.9 / 67.6, 143.8 / 137.9, 267.4 / 259.2; 40 rows 74.9 / 74.7, 147.8 /
+  // 147.6, 275.3 / 270.6; 48 rows 76.1 / 77.8, 146.4 / 152.2, 273.7 / 277.4; 64 rows 78.9 / 86.5, 146.6 /
+  // 162.7, 268.3 / 292.2; 80 rows 102.5 / 99.7, 180.0 / 186.2, 291.9 / 306.0. 110,000 columns 48 rows 64.7 /
+  // 61.8, 118.4 / 116.4, 213.5 / 210.9; 64 rows 67.2 / 68.5, 119.8 / 124.2, 214.3 / 222.3. 90,000 columns 64
+  // rows 58.8 / 55.8, 100.3 / 100.7, 178.9 / 181.4. So from 6.8 million logits on, to 64 rows.
+  // The main product leaves out the probe's columns. Where that saves it a round of tiles over the CUs,
+  // whole pays the round, D's time: 133,000 columns 24 rows 64.4 / 64.8, 123.6 / 128.8, 228.3 / 243.3; 32 rows
+  // 65.5 / 69.1; 100,000 columns 32 rows 55.3 / 52.5, 104.0 / 110.5, 182.7 / 194.5; 67,000 columns 32 rows 45.7
+  // / 40.4, 79.0 / 80.2, 134.7 / 142.0; 34,000 columns 48 rows 38.2 / 31.6, 57.9 / 55.9, 89.2 / 93.6.
+  // It does not depend on k, so that a call at a shape sizes its scratch. With per-row parameters it is
+  // fused for 16 to 64 rows: ahead where no row is general (64 rows of 151,936 x 896, all top-k 50, 84.0 /
+  // 97.5; level at 24 rows, behind below 110,000 columns: 64 rows of 50,257 50.5 / 48.0), and behind where
+  // some are, whose rows it leaves to one workgroup each (a quarter general: 152.1 / 112.6 and 86.5 / 85.3).
+  constexpr int kHeadFuseMin = 16, kHeadFuseMax = 64;
+  const int tile_cols = head_tile_cols(head_tile(B, false));
+  auto rounds = [&](int cols) { return ((cols + tile_cols - 1) / tile_cols + ctx->cus - 1) / ctx->cus; };
+  const bool round_more = rounds(V) > rounds(std::max(0, V - kHeadProbe));
+  const long long least = !round_more ? 6800000 : (D < 1536 ? 4200000 : (D < 3072 ? 2200000 : 1500000));
+  const bool fuse_shape = B >= kHeadFuseMin && B <= kHeadFuseMax && (params_per_row || static_cast<long long>(B) * V >= least);
   const bool fused = ctx->head_route == 1 || (ctx->head_route < 0 && fuse_shape);
   const bool whole = shared_general || !fused;
   // logits written whole: the caller's, or (general rows possible, none kept by the caller) scratch
