@@ -217,15 +217,15 @@ int topk_parts(int B, int V, int cus, int k, bool forced, long long forced_p) {
   const long long pmax = std::min<long long>({std::max(pmin, V4 / 512), kMaxMergeSlices, kMergeCap / kKmax});
   if (pmin > pmax) return 0;
   const long long P = forced_p > 0 ? std::min(std::max(forced_p, pmin), pmax) : pmin;
-  // Measured against row mode (top-k 40, back to back): 151,936 logits in 10 parts 13.4 against 20.4 us
-  // at 1 row, 16.4 / 21.6 at 24, 19.3 / 21.6 at 48, 24.4 / 22.0 at 64; 49,152 in 3 parts 11.6 / 12.9 at
-  // 1 row, 13.4 / 13.9 at 64, 15.5 / 14.1 at 96; 262,144 in 16 parts 15.0 / 27.1 at 1 row, 26.4 / 29.1
-  // at 32, 33.9 / 29.7 at 48: ahead while the parts fit the chip at once (two per CU) and, on short
-  // rows, up to about V / 250 parts. Longer lists cost the split more than row mode: k = 100 at 1 and
-  // 24 rows 18.4-21.0 / 24.6 and 23.0 / 26.4 us at 151,936, but 15.9 / 14.4 at 1 row of 49,152 and 50.1
-  // / 36.4 at 24 rows of 262,144; and from k of about 190 a part's first bound lets more keys through
-  // than a list holds (256), whose select passes take 56.3 / 33.9 us at 1 row of 151,936, k = 256.
-  const long long parts = k <= 64 ? std::min<long long>(2LL * cus, V / 250) : (k <= 100 && P >= 8 ? cus : 0);
+  // Measured against row mode (k = 40, back to back): 151,936 logits in 10 parts 11.1 against 19.0 us at 1
+  // row, 13.1 / 21.5 at 24, 15.9 / 21.7 at 51, 20.3 / 22.1 at 64; 49,152 in 3 parts 10.1 / 12.2 at 1 row,
+  // 11.6 / 13.6 at 64, 13.2 / 14.0 at 96; 262,144 in 16 parts 12.2 / 27.6 at 1 row, 18.2 / 29.0 at 32, 23.0
+  // / 29.4 at 40; 20,000 in 2 parts 9.7 / 10.3 at 1 row, 10.8 / 11.7 at 64. Ahead while the parts fit the
+  // chip at once (two per CU) and, on short rows, up to about V / 170 parts; taken to V / 250. Longer lists
+  // leave the ratio as it is (k = 256: 19.0 / 32.6 and 21.3 / 35.4 at 1 and 24 rows of 151,936, 17.6 / 20.9 at 1
+  // of 49,152) except in 2 parts, whose lists the merge of 2 hardly shortens (1 row of 20,000, k = 200: 15.0 /
+  // 14.5).
+  const long long parts = k <= 64 || P > 2 ? std::min<long long>(2LL * cus, V / 250) : 0;
   if (!forced && (P < 2 || B * P > parts)) return 0;
   if (static_cast<long long>(B) * P > INT32_MAX) return 0;
   return static_cast<int>(std::max<long long>(P, 1));
@@ -240,11 +240,13 @@ int topk_parts(int B, int V, int cus, int k, bool forced, long long forced_p) {
 // 82.8; 49,152 logits 1 row 26.3 / 37.6, 32 rows 34.0 / 39.1, 64 rows 40.2 / 39.2. The line between
 // lies near B = V / 1200; the split is taken to V / kGenSplitLogits.
 constexpr int kGenSplitLogits = 1500;
-// Per-row parameters (against k_rows beside k_general, us; rows all top-k 40 / all top-p / half of each):
-// 24 rows of 50,257 18.8 / 38.6, 32.8 / 62.7, 31.4 / 62.3; 64 of 151,936 (640 parts) 30.2 / 39.0, 73.7 / 94.5,
-// 56.1 / 94.2; 100 of 151,936 38.9 / 38.6, 95.1 / 95.3, 75.6 / 94.7; 100 of 262,144 (1,600 parts) 65.0 /
-// 41.3, 147.2 / 128.8, 120.7 / 128.1. Rows with k of 200 (lists overflow) or above 1,024 (one workgroup)
-// are the split's worst: 46-59 / 39-41 and 100-203 / 105-174 up to 33 rows.
+// Per-row parameters (against k_rows beside k_general, us; rows all of one kind, or mixed: a quarter greedy,
+// the others top-k off, 20, 40 and 100): 24 rows of 50,257 (144 parts) top-k 40 17.6 / 36.7, 256 25.4 / 36.7,
+// top-k off 32.8 / 60.4, 2,000 54.1 / 71.9, greedy 13.8 / 36.7, mixed 30.5 / 60.8; 64 of 151,936 (640 parts) 27.4 /
+// 37.0, 41.9 / 45.0, 72.3 / 91.5, 126.1 / 114.7, 20.3 / 35.8, 46.4 / 90.2; 80 of 151,936 (800) 31.3 / 36.6, 49.0 /
+// 45.5, 82.4 / 93.4, 133.3 / 115.9, 23.7 / 36.5, 50.6 / 90.8; 100 of 151,936 (1,000) 34.9 / 36.9, 56.3 / 45.9, 90.8
+// / 93.7, 141.6 / 116.2, 25.5 / 35.5, 57.5 / 91.5. The line lies where long lists (k = 256) are still ahead;
+// only rows of k above 1,024 are behind below it, when most are such (one workgroup ends each).
 constexpr long long kMixedParts = 640;
 // per_row: the greedy and small-k rows among them are cut into the same parts (k_topk_split's, so
 // register-held ones, at most 16), and a batch that cannot be takes no split.
