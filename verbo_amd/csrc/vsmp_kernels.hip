@@ -1653,7 +1653,9 @@ __device__ __forceinline__ Sel refine_select(const GenCtx& g, GenShared<NT>& sh,
   constexpr int kGenThreads = NT;
   const int tid = threadIdx.x;
   for (int level = 0; level < 8 && n > kGenCap && clo < chi; ++level) {
-    const uint64_t span = chi - clo;
+    // ranges of whole values from a value's first composite on, so that no bucket holds parts of two
+    const uint64_t base = comp_key(clo) == comp_key(chi) ? clo : clo >> 32 << 32;
+    const uint64_t span = chi - base;
     int shift = 0;
     while ((span >> shift) >= static_cast<uint64_t>(kRefBuckets)) ++shift;
     for (int i = tid; i < kRefBuckets; i += kGenThreads) {
@@ -1668,13 +1670,15 @@ __device__ __forceinline__ Sel refine_select(const GenCtx& g, GenShared<NT>& sh,
       if (kv < klo || kv > khi || !pred_v(v)) return -1;
       const uint64_t ck = comp(kv, static_cast<uint32_t>(e));
       if (ck < clo || ck > chi || !pred_c(ck)) return -1;
-      return static_cast<int>((ck - clo) >> shift);
+      return static_cast<int>((ck - base) >> shift);
     };
-    // A thread's successive elements of one bucket add with one atomic pair: where thousands of equal
-    // values share a bucket, the atomics on its address are what the pass waits for.
+    // A thread's successive elements of one bucket add with one atomic pair, and equal values take their
+    // numerator once: where thousands of them share a bucket, the atomics on its address and the
+    // numerators, computed by the few lanes that hold one, are what the pass waits for.
     int run_d = -1;
     uint32_t run_n = 0u;
-    double run_m = 0.0;
+    double run_m = 0.0, last_p = 0.0;
+    float last_v = INFINITY;  // no element's value: d = v - mx is finite or -inf
     auto flush = [&]() {
       if (run_d < 0) return;
       atomicAdd(&sh.rcnt[run_d], run_n);
@@ -1690,7 +1694,13 @@ __device__ __forceinline__ Sel refine_select(const GenCtx& g, GenShared<NT>& sh,
         run_m = 0.0;
       }
       ++run_n;
-      if (MASS) run_m += numer_g(g, v);
+      if (MASS) {
+        if (v != last_v) {
+          last_v = v;
+          last_p = numer_g(g, v);
+        }
+        run_m += last_p;
+      }
     });
     flush();
     __syncthreads();
@@ -1760,11 +1770,15 @@ __device__ __forceinline__ Sel refine_select(const GenCtx& g, GenShared<NT>& sh,
     rank_above = sgpr_i32(sh.ints[2]);
     n = sgpr_i32(sh.ints[3]);
     const int d = kRefBuckets - 1 - pos;
-    const uint64_t nlo = clo + (static_cast<uint64_t>(d) << shift);
+    const uint64_t nlo = base + (static_cast<uint64_t>(d) << shift);
     uint64_t nhi = nlo + ((1ull << shift) - 1ull);
     if (nhi < nlo) nhi = ~0ull;  // wrapped past the top of the key space
-    clo = nlo;
+    clo = max64(nlo, clo);
     chi = nhi < chi ? nhi : chi;
+    if (comp_key(clo) == comp_key(chi)) {  // one value left: its indices
+      clo = max64(clo, comp(comp_key(clo), static_cast<uint32_t>(g.R.V - 1)));
+      chi = min64(chi, comp(comp_key(chi), 0u));
+    }
     __syncthreads();
   }
   // collect, sort, scan
