@@ -1056,6 +1056,22 @@ def test_graph_capture_after_a_larger_warm_up(warm):
             assert torch.equal(out, mode_ctx("rows").pick_batch(x, pr)), (B, f, step)
 
 
+@pytest.mark.parametrize("Vv", [262144, 400000])
+def test_general_split_long_lists(Vv):
+    """Nearly flat rows whose buckets hold 240 to 370 elements, plain and rounded to bf16 (equal values by
+    the hundred): the draw's buckets fill list B between 256 and 1,024 entries, or beyond it, where one
+    workgroup ends the row; the default plan, with and without a cut."""
+    rng = np.random.default_rng(Vv)
+    ctx = V.Context(0)
+    lg = rng.normal(0, 0.5, (16, Vv)).astype(np.float32)
+    lg[8:] = (lg[8:].view(np.uint32) & 0xFFFF0000).view(np.float32)
+    for f in (dict(top_p=0.95), dict(top_p=0.6, temp=1.5), dict(), dict(top_p=0.8, repeat=1.3)):
+        h, off = csr([rng.integers(0, Vv, 2000) if "repeat" in f else [] for _ in range(16)])
+        log("general split, long lists", Vv, f)
+        p = V.params_array(n=1, **dict(dict(temp=1.0, top_k=0, top_p=1.0, repeat=1.0, repeat_last=0, seed=17), **f))
+        assert Run(ctx, lg, p, h, off).report()[1] == 0
+
+
 def test_scratch_on_demand():
     """A context holds the split kernels' scratch only once a call has taken them: the first call of a
     batch too wide for a split allocates the exact redo's sort slots (256 of 1 MiB here) and nothing

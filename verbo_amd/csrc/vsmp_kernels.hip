@@ -2702,9 +2702,9 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
   // chiefs are different parts: workgroups go round the eight XCDs, and the first parts of rows in 16
   // parts all meet on one (40 x 262,144, per-row top-k 2,000: 259 us).
   bool alone = !SPLIT || flat;
-  const bool chief = !SPLIT || part.part == row % a.P;
+  auto chief = [&]() { return !SPLIT || part.part == row % a.P; };
   if constexpr (SPLIT)
-    if (alone && !chief) return;
+    if (__builtin_expect(alone, 0) && !chief()) return;
   bool by_hist = false;  // ... with the parts' histogram, once the k-th element is found in its bucket
   constexpr int BP = kGenBuckets / kGenThreads;
   static_assert(BP % 4 == 0, "a thread's buckets are read as 16-byte vectors");
@@ -2808,7 +2808,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
       __syncthreads();
       if (sgpr_u32(total) != static_cast<uint32_t>(V)) {  // a bucket's count is still not known
         alone = true;
-        if (!chief) return;
+        if (!chief()) return;
         __syncthreads();
       }
     }
@@ -2819,13 +2819,13 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
         // and 158 in one workgroup of 1,024 threads that took every pass).
         qk = min(sgpr_i32(sh.ints[0]), kGenBuckets - 1);
         by_hist = k > kGenCap || (capped && qk == kGenBuckets - 1) || sgpr_u32(sh.cnt0[qk]) > kGenPartList;
-        if (by_hist && !chief) return;
+        if (by_hist && !chief()) return;
         __syncthreads();
       }
     }
   }
   // Stores this part's elements of the buckets that inA and inB take in its lists A (at most capA) and
-  // B (at most kGenCap / 2, from that place on), counted in ints[4] and ints[7]. pv, pnibs: the part's
+  // B (at most kGenCap, from place kGenCap / 2 on), counted in ints[4] and ints[7]. pv, pnibs: the part's
   // first chunk. A lane marks its elements in two masks; a wave's take their places by one scan of the
   // packed counts and one LDS atomic per list, not one per element.
   unsigned long long* plist = nullptr;
@@ -2874,7 +2874,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
               ++pA;
             }
             if ((hB >> (4 * u + i)) & 1u) {
-              if (pB < kGenCap / 2) __hip_atomic_store(&plist[kGenCap / 2 + pB], ck, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+              if (pB < kGenCap) __hip_atomic_store(&plist[kGenCap / 2 + pB], ck, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
               ++pB;
             }
           }
@@ -2897,7 +2897,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
   // relative to the table points, numer_fix, in the mass array's 8-byte slots until the prefix
   // below turns them into fp64 masses)
   uint64_t* fix0 = reinterpret_cast<uint64_t*>(sh.mass0);
-  if (alone) {
+  if (__builtin_expect(alone, !SPLIT)) {
     for (int i = tid; i < kGenBuckets; i += kGenThreads) {
       sh.cnt0[i] = 0u;
       fix0[i] = 0ull;
@@ -2907,13 +2907,13 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
   // prefix below has used it
   double* etab = sh.rmass;
   const double wq = table_width(g.qs, P.temp);
-  if (alone) {
+  if (__builtin_expect(alone, !SPLIT)) {
     for (int j = tid; j < kGenBuckets / 2; j += kGenThreads) etab[j] = exp_tab(-static_cast<double>(2 * j + 1) * wq);
   }
   const FixCoef fc = fix_coef(wq, P.temp, g.inv_temp);
   // The main pass also collects the min-p prefix (its elements' exact numerators are taken there)
   // into the list, which aliases the refinement counts, idle until the pass ends.
-  if (alone) {
+  if (__builtin_expect(alone, !SPLIT)) {
     if (tid == 0) sh.ints[4] = 0;
     __syncthreads();
   }
@@ -2988,7 +2988,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
   // normal values).
   // With a top-k cut the kept elements are the first k by index (equal values rank by index).
   // one instance per combination: no per-element branches beyond the ones asked for
-  if (!alone) {  // SPLIT: k_gen_hist took the pass
+  if (__builtin_expect(!alone, SPLIT)) {  // k_gen_hist took the pass
   } else if (flat) {
     const int n_in = k;  // V with top-k off
     if (tid == 0) {
@@ -3012,7 +3012,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
     main_pass(std::false_type{}, std::true_type{});
   else
     main_pass(std::false_type{}, std::false_type{});
-  if (alone) {
+  if (__builtin_expect(alone, !SPLIT)) {
     const uint32_t oc = block_sum_u32<kGenThreads>(t_ocnt, sh.r32);
     const double om = block_sum_f64<kGenThreads>(t_omass, sh.rd);
     for (int o = 32; o > 0; o >>= 1) t_ofix += __shfl_xor(t_ofix, o);
@@ -3069,7 +3069,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
     chi = block_max64<kGenThreads>(hi_, sh.r64);
   };
   // level-0 inclusive prefixes (BP consecutive buckets per thread, bucket 0 = closest to the maximum)
-  if (alone) {
+  if (__builtin_expect(alone, !SPLIT)) {
     double m[BP];
     uint32_t c[BP];
     double ms = 0.0;
@@ -3098,11 +3098,11 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
     if (tid < 4) sh.fb[tid] = kGenBuckets;
     __syncthreads();
   }
-  if (k < V && !flat && (alone || by_hist)) {
+  if (__builtin_expect(k < V && !flat && (alone || by_hist), 0)) {
     // The k-th element, in the bucket where the counts reach k; the prefixes then end with it, as if the
     // pass had taken no other. From the whole row instead of its bucket the k-th took two histogram
     // passes more, and the main pass a compare per element.
-    if (alone) {
+    if (__builtin_expect(alone, !SPLIT)) {
       if (tid == 0) sh.ints[0] = kGenBuckets - 1;
       __syncthreads();
       int f = kGenBuckets;
@@ -3346,11 +3346,14 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
     }
   }
   if constexpr (SPLIT) {
-    if (!alone) {
+    if (__builtin_expect(!alone, 1)) {
       // Top-k off: the shared pass below over the parts, or (no cut to find) the draw's bucket alone.
       // List A: the cut's bucket; list B: the buckets the draw may fall in.
-      constexpr int LC = kGenCap / 2;
-      static_assert(LC == NT, "one entry of each list per thread");
+      // (Nearly flat rows of 262,144 have 240 elements a bucket: with 512 entries in B their draws' two or
+      // three buckets did not fit, and 16 rows took 169 us where one workgroup per row had taken 161.)
+      constexpr int LC = kGenCap / 2, LB = kGenCap;
+      static_assert(LC == NT && LB == 2 * NT, "one entry of list A per thread, two of list B");
+      static_assert(LC + LB <= kGenPartList && 2 * (LC + LB) * 8 <= sizeof(sh.rcnt) + sizeof(sh.rmass), "the lists and their sums");
       const int lane = tid & 63, w = tid >> 6;
       float4 pv[LU];
       gen_part_load(g.R.rp, V, part, part.g0, pv);
@@ -3397,11 +3400,11 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
         plan = true;
       }
       const int base_d = d_lo > 0 && d_lo < kGenBuckets ? sgpr_i32(static_cast<int>(sh.cnt0[d_lo - 1])) : 0;
-      plan = plan && d_hi < kGenBuckets && sgpr_i32(static_cast<int>(sh.cnt0[min(d_hi, kGenBuckets - 1)])) - base_d <= LC;
-      if (!plan) {
+      plan = plan && d_hi < kGenBuckets && sgpr_i32(static_cast<int>(sh.cnt0[min(d_hi, kGenBuckets - 1)])) - base_d <= LB;
+      if (__builtin_expect(!plan, 0)) {
         // the min-p prefix, which k_gen_hist listed, or a plan whose lists do not fit: one workgroup
         // ends the row
-        if (!chief) return;
+        if (!chief()) return;
         alone = true;
         __syncthreads();
         if (tid < 4) sh.fb[tid] = kGenBuckets;
@@ -3414,15 +3417,15 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
         part_lists(pv, pnibs, LC, [qp](int q) { return q == qp; }, [d_lo, d_hi](int q) { return q >= d_lo && q <= d_hi; });
         if (!hand_over()) return;
         alone = true;
-        uint64_t* listA = sh.list;
-        uint64_t* listB = sh.list + LC;
-        double* lprA = sh.lpr;
-        double* lprB = sh.lpr + LC;
+        uint64_t* listA = reinterpret_cast<uint64_t*>(sh.rcnt);  // the refinement's area, which is one array's worth
+        uint64_t* listB = listA + LC;
+        double* lprA = reinterpret_cast<double*>(listB + LB);
+        double* lprB = lprA + LC;
         if (w < 2) gen_offsets(a, row, kGenPartListA + w, part_off[w]);
         if (tid < 4) sh.fb[tid] = kGenBuckets;
-        if (tid < 2) sh.ints[tid] = LC;
+        if (tid < 2) sh.ints[tid] = LB;
         __syncthreads();
-        const int mA = min(sgpr_i32(part_off[0][64]), LC), mB = min(sgpr_i32(part_off[1][64]), LC);
+        const int mA = min(sgpr_i32(part_off[0][64]), LC), mB = min(sgpr_i32(part_off[1][64]), LB);
         // Lists that half the threads hold are ranked side by side, longer ones one after the other
         // (counting all 512 is still faster than a bitonic sort's 45 barriers).
         const double above_d = d_lo > 0 ? sgpr_f64(sh.mass0[d_lo - 1]) : 0.0;
@@ -3444,28 +3447,36 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
           }
         } else {
           const uint64_t xA = tid < mA ? gen_entry(a, row, 0, part_off[0], tid) : 0ull;
-          const uint64_t xB = tid < mB ? gen_entry(a, row, LC, part_off[1], tid) : 0ull;
+          uint64_t xB[2];
+#pragma unroll
+          for (int c = 0; c < 2; ++c) xB[c] = tid + c * NT < mB ? gen_entry(a, row, LC, part_off[1], tid + c * NT) : 0ull;
           listA[tid] = xA;
-          listB[tid] = xB;
+#pragma unroll
+          for (int c = 0; c < 2; ++c) listB[tid + c * NT] = xB[c];
           __syncthreads();
-          int rA = 0, rB = 0;
+          int rA = 0, rB[2] = {0, 0};
           if (tid < mA) rA = rank_count(listA, mA, xA);
-          if (tid < mB) rB = rank_count(listB, mB, xB);
-          const double wA = numer_g(g, comp_val(xA)), wB = numer_g(g, comp_val(xB));
+#pragma unroll
+          for (int c = 0; c < 2; ++c)
+            if (tid + c * NT < mB) rB[c] = rank_count(listB, mB, xB[c]);
           __syncthreads();
           if (tid < mA) {
             listA[rA] = xA;
-            lprA[rA] = wA;
+            lprA[rA] = numer_g(g, comp_val(xA));
           }
-          if (tid < mB) {
-            listB[rB] = xB;
-            lprB[rB] = wB;
+#pragma unroll
+          for (int c = 0; c < 2; ++c) {
+            if (tid + c * NT >= mB) continue;
+            listB[rB[c]] = xB[c];
+            lprB[rB[c]] = numer_g(g, comp_val(xB[c]));
           }
         }
         __syncthreads();
-        // running sums through both lists, and the first entry of each that reaches its target
+        // running sums through both lists (two entries of B per thread), and the first entry of each that
+        // reaches its target
+        const double wB0 = 2 * tid < mB ? lprB[2 * tid] : 0.0, wB1 = 2 * tid + 1 < mB ? lprB[2 * tid + 1] : 0.0;
         double iA = wave_incl_scan_f64(tid < mA ? lprA[tid] : 0.0);
-        double iB = wave_incl_scan_f64(tid < mB ? lprB[tid] : 0.0);
+        double iB = wave_incl_scan_f64(wB0 + wB1);
         if (lane == 63) {
           sh.wm[w] = iA;
           sh.rd[w] = iB;
@@ -3477,9 +3488,11 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
           pB += sh.rd[i];
         }
         iA += pA;
+        const double eB = (iB - wB1) + pB;  // through the first of this thread's two
         iB += pB;
         lprA[tid] = iA;
-        lprB[tid] = iB;
+        lprB[2 * tid] = eB;
+        lprB[2 * tid + 1] = iB;
         if (cut) {
           wave_claim_min(&sh.ints[0], tid < mA && iA >= tgt, tid);
           __syncthreads();
@@ -3495,7 +3508,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
           target = u * tot;
           flags |= VSMP_FLAG_ONE_PASS;
         }
-        wave_claim_min(&sh.ints[1], tid < mB && iB >= target, tid);
+        const bool b0_in = 2 * tid < mB && eB >= target, b1_in = 2 * tid + 1 < mB && iB >= target;
+        wave_claim_min(&sh.ints[1], b0_in || b1_in, b0_in ? 2 * tid : 2 * tid + 1);
         __syncthreads();
         const int j = sgpr_i32(sh.ints[1]);
         if (j < mB) {  // (not so: rounding at the list's end; a select of its own below)
