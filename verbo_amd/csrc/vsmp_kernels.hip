@@ -2706,6 +2706,9 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
   if constexpr (SPLIT)
     if (__builtin_expect(alone, 0) && !chief()) return;
   bool by_hist = false;  // ... with the parts' histogram, once the k-th element is found in its bucket
+  // a top-k of at most kGenCap elements, all of them listed: the buckets through the k-th's fit the list
+  bool topk_list = false;
+  auto lists_fit = [&](int q) { return k <= kGenCap && !(capped && q == kGenBuckets - 1) && sgpr_u32(sh.cnt0[q]) <= kGenPartList; };
   constexpr int BP = kGenBuckets / kGenThreads;
   static_assert(BP % 4 == 0, "a thread's buckets are read as 16-byte vectors");
   const int b0 = BP * tid;
@@ -2818,7 +2821,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
         // parts' histogram (24 x 128,256, per-row top-k 2,000: 85 us, against 180 when it took every pass
         // and 158 in one workgroup of 1,024 threads that took every pass).
         qk = min(sgpr_i32(sh.ints[0]), kGenBuckets - 1);
-        by_hist = k > kGenCap || (capped && qk == kGenBuckets - 1) || sgpr_u32(sh.cnt0[qk]) > kGenPartList;
+        topk_list = lists_fit(qk);
+        by_hist = !topk_list;
         if (by_hist && !chief()) return;
         __syncthreads();
       }
@@ -3098,21 +3102,22 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
     if (tid < 4) sh.fb[tid] = kGenBuckets;
     __syncthreads();
   }
-  if (__builtin_expect(k < V && !flat && (alone || by_hist), 0)) {
-    // The k-th element, in the bucket where the counts reach k; the prefixes then end with it, as if the
+  if (k < V && !flat && alone) {  // the bucket where the counts reach k
+    if (tid == 0) sh.ints[0] = kGenBuckets - 1;
+    __syncthreads();
+    int f = kGenBuckets;
+#pragma unroll
+    for (int i = BP - 1; i >= 0; --i)
+      if (sh.cnt0[b0 + i] >= static_cast<uint32_t>(k)) f = b0 + i;
+    wave_claim_min(&sh.ints[0], f < kGenBuckets, f);
+    __syncthreads();
+    qk = sgpr_i32(sh.ints[0]);
+    topk_list = lists_fit(qk);
+  }
+  if (__builtin_expect(k < V && !flat && !topk_list, 0)) {
+    // The k-th element, in its bucket; the prefixes then end with it, as if the
     // pass had taken no other. From the whole row instead of its bucket the k-th took two histogram
     // passes more, and the main pass a compare per element.
-    if (__builtin_expect(alone, !SPLIT)) {
-      if (tid == 0) sh.ints[0] = kGenBuckets - 1;
-      __syncthreads();
-      int f = kGenBuckets;
-#pragma unroll
-      for (int i = BP - 1; i >= 0; --i)
-        if (sh.cnt0[b0 + i] >= static_cast<uint32_t>(k)) f = b0 + i;
-      wave_claim_min(&sh.ints[0], f < kGenBuckets, f);
-      __syncthreads();
-      qk = sgpr_i32(sh.ints[0]);
-    }
     const int ra = qk > 0 ? sgpr_i32(static_cast<int>(sh.cnt0[qk - 1])) : 0;
     const int n = sgpr_i32(static_cast<int>(sh.cnt0[qk])) - ra;
     const double above = qk > 0 ? sgpr_f64(sh.mass0[qk - 1]) : 0.0;
@@ -3291,26 +3296,42 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
   // Small min-p prefix: its elements (numerator >= thr, all of them close to the maximum) are
   // collected whole, by the main pass as a rule; the top-p cut and the draw are then taken on the
   // sorted prefix sums.
-  if constexpr (SPLIT) {
-    if (!alone && k < V) {
-      // A top-k of at most kGenCap elements: every element through the k-th's bucket, listed by the
-      // parts and put in order by the last one (each bucket's entries at its count prefix, then
-      // ranked within the bucket), in the histogram's mass array, read no more. The sum, the cuts and
-      // the draw are taken on the sorted list.
-      float4 pv[LU];
-      gen_part_load(g.R.rp, V, part, part.g0, pv);
-      part_lists(pv, g.R.pen && part.hi > part.lo ? gen_part_nibs<LU>(g.R.bits, part, part.g0) : 0u, kGenPartList,
-                 [qk](int q) { return q <= qk; }, [](int) { return false; });
-      if (!hand_over()) return;
+  {
+    if (topk_list) {
+      // A top-k of at most kGenCap elements: every element through the k-th's bucket, listed by a pass
+      // (SPLIT: by the parts, of which the last goes on) and put in order (each bucket's entries at its
+      // count prefix, then ranked within the bucket), in the histogram's mass array, read no more. The
+      // sum, the cuts and the draw are taken on the sorted list.
+      static_assert(sizeof(sh.list) + sizeof(sh.lpr) >= kGenPartList * 8, "the gathered list");
+      int m = 0;
+      if constexpr (SPLIT) {
+        if (__builtin_expect(!alone, 1)) {
+          float4 pv[LU];
+          gen_part_load(g.R.rp, V, part, part.g0, pv);
+          part_lists(pv, g.R.pen && part.hi > part.lo ? gen_part_nibs<LU>(g.R.bits, part, part.g0) : 0u, kGenPartList,
+                     [qk](int q) { return q <= qk; }, [](int) { return false; });
+          if (!hand_over()) return;
+          // gathered through the refinement area (the lists' own place)
+          m = gen_gather<NT>(a, row, kGenPartListA, 0, sh.list, 2 * kGenCap, part_off[0]);
+        }
+      }
+      if (alone) {
+        if (tid == 0) sh.ints[4] = 0;
+        __syncthreads();
+        gen_pass<NT>(g.R, [&](int e, float v) {
+          if (q_of(g, v) > qk) return;
+          const int p = atomicAdd(&sh.ints[4], 1);
+          if (p < kGenPartList) sh.list[p] = comp(ord_key(v), static_cast<uint32_t>(e));
+        });
+        __syncthreads();
+        m = min(sgpr_i32(sh.ints[4]), kGenPartList);
+      }
       alone = true;
       uint64_t* big = reinterpret_cast<uint64_t*>(sh.mass0);            // kGenPartList entries
       uint32_t* fill = reinterpret_cast<uint32_t*>(big + kGenPartList);  // per bucket
       static_assert(kGenPartList * 8 + kGenBuckets * 4 <= kGenBuckets * 8, "both fit the mass array");
       for (int i = tid; i < kGenBuckets; i += kGenThreads) fill[i] = 0u;
-      // gathered through the refinement area (the lists' own place), half a list at a time at most
-      int* off = part_off[0];
-      const int m = gen_gather<NT>(a, row, kGenPartListA, 0, sh.list, 2 * kGenCap, off);
-      static_assert(sizeof(sh.list) + sizeof(sh.lpr) >= kGenPartList * 8, "the gathered list");
+      __syncthreads();
       for (int i = tid; i < m; i += kGenThreads) {
         const uint64_t x = sh.list[i];
         const int q = q_of(g, comp_val(x));
