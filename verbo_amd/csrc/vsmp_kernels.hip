@@ -3950,7 +3950,7 @@ __global__ __launch_bounds__(kGenThreads) void k_general_exact(KArgs a) {
   __shared__ uint32_t xk[2];  // the row's smallest and largest penalised order key
   __shared__ __align__(16) uint64_t blk[kXBlock];  // sort blocks; staged chunks of the chains
   // A workgroup with one row leaves on that row's mark: most calls mark none, and their launch should
-  // cost no more than it must.
+  // cost no more than it must. (The launch has at most a.B workgroups.)
   if (gridDim.x >= static_cast<unsigned>(a.B) && a.x_flag[blockIdx.x] == 0) return;
   double* stage = reinterpret_cast<double*>(blk);
   const int tid = threadIdx.x;
