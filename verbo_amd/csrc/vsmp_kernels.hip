@@ -2150,7 +2150,7 @@ __device__ __forceinline__ void topk_part(const KArgs& a, TkShared& sh, const vs
     np = block_sum_u32<kTkNT>(np, sh.red32);
   }
   if (tid == 0) {
-    __hip_atomic_store(&a.s_cnt[slot], ks, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(&a.s_cnt[slot], min(nt, ks), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __hip_atomic_store(&a.s_npen[slot], static_cast<int>(np), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
   if (!topk_last_part(a, row, &sh.ints[9])) return;
@@ -2210,7 +2210,7 @@ __device__ __forceinline__ uint32_t gen_raw_count_any(uint64_t raw, double w, ui
   const uint32_t most = missing + gen_raw_count(raw);
   uint32_t n = 0u;
   int found = 0;
-  for (uint32_t F = 0u; F <= (most >> 12) + 1u; ++F) {  // f 2^-40 below 1.017 n, n below 2^18
+  for (uint32_t F = 0u; F <= (most >> 12) + (most >> 17) + 1u; ++F) {  // f 2^-40 is below 1.02 n
     const double f = low + 4096.0 * F;
     const uint32_t from = static_cast<uint32_t>(fmax(f * lo - 1.0, 1.0)), to = min(static_cast<uint32_t>(f * hi + 1.0), most);
     const uint32_t c = from + (((top - F) * kRawInv - from) & 4095u);
