@@ -217,7 +217,7 @@ def settle(graph, stream, ms=20.0):
 
 
 def bench_head(args):
-    """The LM head and the pick in one call (vsmp_head_pick, its route by batch size), the fused
+    """The LM head and the pick in one call (vsmp_head_pick, its route by shape), the fused
     route pinned, the same work unfused (the head's logits written by vsmp_head_logits, then
     vsmp_pick_batch over them), and the head's product alone. Each variant: K steps captured into a
     HIP graph and replayed, timed by two events on the launch stream; the head rotates over three

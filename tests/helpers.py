@@ -36,7 +36,7 @@ _CTX = {}
 
 def mode_ctx(mode=None, head_route=None):
     """A context created under VSMP_MODE=mode (None: the planner's choice) and
-    VSMP_HEAD_ROUTE=head_route (None: vsmp_head_pick's route by batch size), cached per pair: the
+    VSMP_HEAD_ROUTE=head_route (None: vsmp_head_pick's route by shape), cached per pair: the
     library reads its tuning switches once, when a context is created."""
     key = (mode, head_route)
     if key not in _CTX:

@@ -2,7 +2,7 @@
 
 The head's product (reference src/session.cpp:169, matmul(m->head, ...)) is checked against a
 plain fp32 product of the same bf16 operands on the CPU. vsmp_head_pick is checked, on its route
-by batch size and with the fused route pinned for every batch, against the oracle (the reference's
+by shape and with the fused route pinned for every batch, against the oracle (the reference's
 Sampler::pick, src/sampler.cpp:50-109) on the logits the head itself produces, with every
 comparison rule of the batched path (penalised ids, keep counts, candidate ids, sums, ids), and
 against vsmp_pick_batch on those logits, field for field.
@@ -272,7 +272,7 @@ def test_head_pick_row_tiles_padding_and_draw_modes(ctx):
 
 
 def test_head_pick_routes_agree():
-    """VSMP_HEAD_ROUTE pins vsmp_head_pick's route. At 32 rows (fused by batch size) the whole route
+    """VSMP_HEAD_ROUTE pins vsmp_head_pick's route. At 32 rows the whole route
     (the head's logits written, then the batched pick) and the fused one give the same ids, the
     same row diagnostics and the same candidate ids, for greedy, small-k and general parameters
     with penalised histories and counter draws."""

@@ -86,7 +86,7 @@ struct vsmp_ctx {
   int cus = 256;                 // compute units of the device
   // tuning and testing switches, read from the environment when the context is created:
   // VSMP_MODE=rows|slices|split (-1: the planner's choice), VSMP_SPLIT_P, VSMP_EPT,
-  // VSMP_HEAD_ROUTE=fused|whole (-1: vsmp_head_pick's route by batch size)
+  // VSMP_HEAD_ROUTE=fused|whole (-1: vsmp_head_pick's route by shape)
   int mode = -1;
   int head_route = -1;  // 1: fused, 0: whole
   long long split_p = 0;
